@@ -525,6 +525,8 @@ FillWork fill_work_of(const vx_chunk *c, int terrain) {
     w.cz = c->coord.z;
     w.edge = c->edge;
     w.terrain = terrain;
+    if (terrain >= 0)
+        w.variant = fill_variant(c->ctx->terrains[terrain], w.cx, w.cy, w.cz, w.edge);
     w.ids = c->ids;
     w.occ = c->occ;
     w.planes = c->planes;
@@ -597,7 +599,7 @@ extern "C" int vx_chunk_from_ids(vx_ctx *ctx, vx_coord coord, int32_t edge, cons
     bind_chunk_ptrs(c, (char *)c->block);
     hipError_t e = hipMemcpyAsync(c->ids, ids, nv, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);  // caller's buffer is pageable
-    if (e == hipSuccess) e = launch_pack_one(fill_work_of(c, 0), ctx->stream);
+    if (e == hipSuccess) e = launch_pack_one(fill_work_of(c, -1), ctx->stream);
     uint32_t meta0 = kBlockMixed;
     if (e == hipSuccess)
         e = hipMemcpyAsync(ctx->pinned, c->meta, 4, hipMemcpyDeviceToHost, ctx->stream);

@@ -164,7 +164,7 @@ int32_t emit_split_of(const vx_batch *b) {
 hipError_t enqueue_fill(vx_batch *b) {
     vx_ctx *ctx = b->ctx;
     return launch_fill(b->fill_dev, b->order_dev, b->n, b->max_edge, ctx->terrains_dev,
-                       ctx->lut_dev, b->overflow + 1, fill_split_of(b), ctx->stream);
+                       ctx->lut_dev, b->overflow + 1, fill_split_of(b), b->fill_kinds, ctx->stream);
 }
 hipError_t enqueue_count(vx_batch *b) {
     return launch_count(b->mesh_dev, b->n, b->max_edge, b->counts, b->slabs, b->ctx->stream);
@@ -241,7 +241,7 @@ hipError_t enqueue_split(vx_batch *b) {
     e = launch_cull(b->cull, s0);
     if (e == hipSuccess)
         e = launch_fill(b->fill_dev, nullptr, m2, b->max_edge, ctx->terrains_dev, ctx->lut_dev,
-                        b->overflow + 1, fs, s0);
+                        b->overflow + 1, fs, b->fill_kinds, s0);
     if (e == hipSuccess) e = hipEventRecord(b->split_ev[0], s0);
     // first half on the second stream
     if (e == hipSuccess) e = hipStreamWaitEvent(s1, b->split_ev[0], 0);
@@ -258,7 +258,7 @@ hipError_t enqueue_split(vx_batch *b) {
     // second half on the context stream
     if (e == hipSuccess)
         e = launch_fill(b->fill_dev + m2, nullptr, n - m2, b->max_edge, ctx->terrains_dev,
-                        ctx->lut_dev, b->overflow + 1, fs, s0);
+                        ctx->lut_dev, b->overflow + 1, fs, b->fill_kinds, s0);
     if (e == hipSuccess && !b->fill_counts)
         e = launch_count(b->mesh_dev + m, n - m, b->max_edge, b->counts + m, nullptr, s0);
     if (e == hipSuccess) e = hipStreamWaitEvent(s0, b->split_ev[1], 0);
@@ -505,6 +505,8 @@ extern "C" int vx_batch_create_ext(vx_ctx *ctx, const vx_batch_req *reqs, int32_
         f.cz = r.coord.z;
         f.edge = r.edge;
         f.terrain = r.terrain_id;
+        f.variant = fill_variant(ctx->terrains[r.terrain_id], f.cx, f.cy, f.cz, f.edge);
+        b->fill_kinds |= f.variant ? kFillFast : kFillGeneral;
         f.ids = (uint8_t *)base;
         f.occ = (uint32_t *)(base + L.occ);
         f.planes = (uint32_t *)(base + L.planes);
@@ -535,7 +537,7 @@ extern "C" int vx_batch_create_ext(vx_ctx *ctx, const vx_batch_req *reqs, int32_
     // workgroup and no neighbour inside the batch (each neighbour plane is
     // absent or resident before the run): the staged form then has no
     // count kernel.
-    b->fill_counts = fill_whole_chunks(n);
+    b->fill_counts = b->max_edge <= 32 && fill_whole_chunks(n);
     for (int i = 0; i < n && b->fill_counts; i++)
         for (int k = 0; k < 4; k++)
             if (reqs[i].nb[k] >= 0) b->fill_counts = false;
@@ -752,7 +754,7 @@ extern "C" int vx_batch_run_per_chunk(vx_ctx *ctx, vx_batch *b) {
     const int n = b->n;
     for (int i = 0; i < n; i++)
         VX_HIP(ctx, launch_fill(b->fill_dev + i, nullptr, 1, b->reqs[i].edge, ctx->terrains_dev,
-                                ctx->lut_dev, b->overflow + 1, 0, ctx->stream));
+                                ctx->lut_dev, b->overflow + 1, 0, b->fill_kinds, ctx->stream));
     auto slabs_of = [&](int i) { return b->slabs ? b->slabs + (size_t)kSlabs * i : nullptr; };
     for (int i = 0; i < n; i++)
         VX_HIP(ctx, launch_count(b->mesh_dev + i, 1, b->reqs[i].edge, b->counts + i, slabs_of(i),

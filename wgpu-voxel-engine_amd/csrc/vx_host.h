@@ -139,6 +139,7 @@ struct vx_batch {
     hipEvent_t planes_ev = nullptr; // the staging copy has been consumed
     vx::FillWork *fill_dev = nullptr;
     vx::MeshWork *mesh_dev = nullptr;
+    uint32_t fill_kinds = 0;        // kFillFast / kFillGeneral: the chunks' fill kernels
     int32_t *order_dev = nullptr;   // longest-first schedule (null when uniform)
     int32_t *coords_dev = nullptr;  // chunk coordinates (draw lists), made on first use
     void *ctl = nullptr;            // counts[n] | bases[n] | total | overflow | emit_order[n_items]

@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "vx_fill_rule.h"
+
 namespace vx {
 
 constexpr int kBlock = 256;        // threads per workgroup (4 wave64)
@@ -68,7 +70,7 @@ struct MeshTables {
 struct FillWork {
     int32_t cx, cy, cz, edge;
     int32_t terrain;       // index into the terrain table
-    int32_t pad0;
+    int32_t variant;       // fill_variant: 0 = the general kernels, else the fast one's
     uint8_t *ids;          // edge^3
     uint32_t *occ;         // edge^2 rows * W words (W = 1 for edge <= 32, 2 for 64)
     uint32_t *planes;      // 4 planes * edge * W words: x=0, x=N-1, z=0, z=N-1
@@ -160,6 +162,13 @@ struct DrawArgs {
 };
 enum : uint32_t { kDrawInstanced = 1u, kDrawExpanded = 2u };
 
+// Variant of the fast fill for a chunk of terrain T (vx_fill_rule.h), 0 for
+// the general kernels; chunks without 3-D noise always take the fast one.
+inline int32_t fill_variant(const TerrainDev &T, int32_t cx, int32_t cy, int32_t cz, int32_t edge) {
+    if (T.kind != kDensity && T.kind != kReference) return 1;
+    return fast_variant(T.octaves, T.frequency, T.lacunarity, T.gain, cx, cy, cz, edge);
+}
+
 inline int words_per_row(int edge) { return (edge + 31) / 32; }
 
 // ---- kernel launchers (vx_kernels.hip) --------------------------------
@@ -186,10 +195,12 @@ inline int emit_parts_for(int32_t items, int32_t hint = 0) {
     const int p = (kEmitGrid + items - 1) / items;
     return p < 4 ? p : 4;
 }
-// parts_hint: fill_parts_for's hint.
+// parts_hint: fill_parts_for's hint.  kinds: which chunks the work holds
+// (kFillFast: a FillWork.variant set, kFillGeneral: 0): a kernel for each.
+enum : uint32_t { kFillFast = 1u, kFillGeneral = 2u };
 hipError_t launch_fill(const FillWork *work, const int32_t *order, int32_t n, int32_t max_edge,
                        const TerrainDev *terrains, const GradLut *lut, uint32_t *error,
-                       int32_t parts_hint, hipStream_t s);
+                       int32_t parts_hint, uint32_t kinds, hipStream_t s);
 // True iff launch_fill gives each chunk one workgroup (fill_kernel), so that
 // FillWork.count_out is honoured for every chunk of the batch (whatever the
 // hint).

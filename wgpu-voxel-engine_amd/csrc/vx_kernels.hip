@@ -35,6 +35,14 @@ __device__ __forceinline__ int popc(uint64_t v) { return __popcll(v); }
 __device__ __forceinline__ int ctz(uint32_t v) { return __ffs(v) - 1; }
 __device__ __forceinline__ int ctz(uint64_t v) { return __ffsll((unsigned long long)v) - 1; }
 
+// A device pointer read from memory (a work descriptor's) is a generic
+// pointer to the compiler, and its accesses flat instructions, which also
+// occupy the LDS unit and its wait counter; these all point to HBM.
+template <class T> using GlobalPtr = __attribute__((address_space(1))) T *;
+template <class T> __device__ __forceinline__ GlobalPtr<T> as_global(T *p) {
+    return (GlobalPtr<T>)p;
+}
+
 // Exclusive scan of one u32 per thread over a BLOCK-thread workgroup.
 template <int BLOCK = kBlock>
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t *s_wave,
@@ -64,6 +72,20 @@ __device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t *s_wave) {
     uint32_t total;
     block_exclusive_scan(v, s_wave, &total);
     return total;
+}
+
+// Orders the LDS accesses of one wave: staging written by some lanes is read
+// by others of the same wave (LDS executes one wave's operations in order).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// v with lane `lane` replaced by the uniform value x (v_writelane_b32, which
+// this compiler exposes as an intrinsic only).
+extern "C" __device__ int vx_llvm_writelane(int x, int lane, int v) __asm("llvm.amdgcn.writelane.i32");
+__device__ __forceinline__ uint32_t write_lane(uint32_t x, uint32_t lane, uint32_t v) {
+    return (uint32_t)vx_llvm_writelane((int)x, (int)lane, (int)v);
 }
 
 // 2-D improved-noise gradient: x+y, -x+y, x-y, -x-y, x, -x, y, -y.
@@ -579,7 +601,7 @@ __device__ void generate_rows(const TerrainDev &T, int ox, int oy, int oz, const
 }
 
 // Writes the layers y_lo <= y < y_hi of a chunk whose occupancy rows for
-// them are in S.occ: occupancy and boundary planes always, u8 ids (all solid
+// them are in S.occ (which starts at layer y_base): occupancy and boundary planes always, u8 ids (all solid
 // voxels = kBlockGrass) when write_ids; meta[0] = solid block id from the
 // workgroup that writes layer 0.  COHERENT: the occupancy rows and boundary
 // planes, which other workgroups of the same launch read, are written with
@@ -587,46 +609,49 @@ __device__ void generate_rows(const TerrainDev &T, int ox, int oy, int oz, const
 // write-back; a plain store may stay in the writing XCD's L2).
 template <int N, int MAXN, bool COHERENT = false, class SH>
 __device__ void write_chunk_outputs(const FillWork &w, SH &S, bool write_ids, uint32_t solid_type,
-                                    int y_lo = 0, int y_hi = N) {
+                                    int y_lo = 0, int y_hi = N, int y_base = 0) {
     constexpr int W = N == 64 ? 2 : 1;
     constexpr int RS = RowStride<MAXN>::v;
-    const uint32_t *occ = reinterpret_cast<const uint32_t *>(S.occ);
+    const uint32_t *occ = reinterpret_cast<const uint32_t *>(S.occ) - y_base * N * RS;
     const int tid = threadIdx.x;
     const int span = y_hi - y_lo;
+    auto put = [](uint32_t *p, uint32_t v) {
+        if (COHERENT) __hip_atomic_store(as_global(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else *as_global(p) = v;
+    };
     for (int i = y_lo * N * W + tid; i < y_hi * N * W; i += kBlock) {
         const int r = i / W, j = i - r * W;
-        if (COHERENT)
-            __hip_atomic_store(w.occ + i, occ[r * RS + j], __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        else
-            w.occ[i] = occ[r * RS + j];
+        put(w.occ + i, occ[r * RS + j]);
     }
-    // boundary planes: [0] x=0, [1] x=N-1 (bit z per y); [2] z=0, [3] z=N-1 (row bits)
-    for (int k = tid; k < 4 * span * W; k += kBlock) {
-        const int pl = k / (span * W), rem = k - pl * span * W, y = y_lo + rem / W;
-        const int j = rem - (y - y_lo) * W, i = pl * N * W + y * W + j;
-        uint32_t v = 0;
-        if (pl < 2) {
-            const int xb = pl == 0 ? 0 : N - 1;
-            const int zlim = N < 32 ? N : 32;
-            for (int zz = 0; zz < zlim; zz++) {
-                const int z = j * 32 + zz;
-                const uint32_t word = occ[(y * N + z) * RS + (xb >> 5)];
-                v |= ((word >> (xb & 31)) & 1u) << zz;
-            }
-        } else {
-            const int z = pl == 2 ? 0 : N - 1;
-            v = occ[(y * N + z) * RS + j];
+    // boundary planes: [0] x=0, [1] x=N-1 (bit z per y): one ballot of the
+    // z rows each, 64 / N layers per wave pass
+    {
+        constexpr int L = 64 / N, BITS = N < 32 ? N : 32;
+        constexpr uint32_t MASK = N >= 32 ? 0xFFFFFFFFu : ((1u << (N & 31)) - 1u);
+        const int lane = tid & 63, wave = tid >> 6;
+        for (int y0 = y_lo + wave * L; y0 < y_hi; y0 += kBlock / 64 * L) {
+            const int y = min(y0 + lane / N, y_hi - 1);
+            const uint32_t *row = occ + (y * N + lane % N) * RS;
+            const uint64_t first = __ballot(row[0] & 1u);
+            const uint64_t last = __ballot((row[W - 1] >> (BITS - 1)) & 1u);
+            const int pl = lane / (L * W), q = lane - pl * (L * W);
+            const int yq = y0 + q / W;
+            if (pl < 2 && yq < y_hi)
+                put(w.planes + pl * N * W + yq * W + q % W,
+                    (uint32_t)((pl ? last : first) >> (q * BITS)) & MASK);
         }
-        if (COHERENT)
-            __hip_atomic_store(w.planes + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        else
-            w.planes[i] = v;
+    }
+    // [2] z=0, [3] z=N-1: rows
+    for (int k = tid; k < 2 * span * W; k += kBlock) {
+        const int pl = k / (span * W), rem = k - pl * span * W, y = y_lo + rem / W;
+        const int j = rem % W;
+        put(w.planes + (2 + pl) * N * W + y * W + j, occ[(y * N + (pl ? N - 1 : 0)) * RS + j]);
     }
     if (write_ids) {
         // u8 block ids, 16 voxels per 16-byte store
         constexpr int PER_ROW = N / 16;
-        uint4 *ids4 = reinterpret_cast<uint4 *>(w.ids);
+        typedef uint32_t Ids16 __attribute__((ext_vector_type(4)));
+        const GlobalPtr<Ids16> ids4 = as_global(reinterpret_cast<Ids16 *>(w.ids));
         for (int q = y_lo * N * PER_ROW + tid; q < y_hi * N * PER_ROW; q += kBlock) {
             const int r = q / PER_ROW, part = q - r * PER_ROW;
             const uint32_t word = occ[r * RS + (part >> 1)];
@@ -635,12 +660,12 @@ __device__ void write_chunk_outputs(const FillWork &w, SH &S, bool write_ids, ui
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 const uint32_t nib = (bits >> (4 * k)) & 0xFu;
-                o[k] = ((nib * 0x00204081u) & 0x01010101u) * kBlockGrass;
+                o[k] = (__umul24(nib, 0x00204081u) & 0x01010101u) * kBlockGrass;
             }
-            ids4[q] = make_uint4(o[0], o[1], o[2], o[3]);
+            ids4[q] = Ids16{o[0], o[1], o[2], o[3]};
         }
     }
-    if (tid == 0 && y_lo == 0) w.meta[0] = solid_type;
+    if (tid == 0 && y_lo == 0) *as_global(w.meta) = solid_type;
 }
 
 // Rows [part * N / parts, +N / parts) of chunk `w` through the octave-inner
@@ -660,6 +685,17 @@ __device__ void fill_part(const FillWork &w, const TerrainDev &T, FillShared<MAX
 template <int N, int MAXN, class SH>
 __device__ void count_loaded(SH &S, uint32_t *count_out, uint32_t *slabs);
 
+// The four planes facing a chunk (null = absent neighbour) into S.nb.
+template <int N, int MAXN, int BLOCK = kBlock, class SH>
+__device__ __forceinline__ void load_neighbours(const uint32_t *const (&planes)[4], SH &S) {
+    using R = typename RowType<MAXN>::T;
+    for (int i = threadIdx.x; i < 4 * N; i += BLOCK) {
+        const int k = i / N, y = i - k * N;
+        const uint32_t *p = planes[k];
+        S.nb[k][y] = p ? (R)as_global(reinterpret_cast<const typename RowType<N>::T *>(p))[y] : (R)0;
+    }
+}
+
 // With w.count_out the fill also counts the chunk's faces from the rows it
 // holds in LDS and the neighbour planes w.cnb (all written before the
 // launch), which spares the batch its count kernel.
@@ -671,18 +707,7 @@ __device__ __forceinline__ void fill_chunk(const FillWork &w, const TerrainDev &
     __syncthreads();
     write_chunk_outputs<N, MAXN>(w, S, true, kBlockGrass);
     if (w.count_out) {
-        using R = typename RowType<MAXN>::T;
-        constexpr int W = N == 64 ? 2 : 1;
-        for (int i = threadIdx.x; i < 4 * N; i += kBlock) {  // S.nb: no halo lines here
-            const int k = i / N, y = i - k * N;
-            const uint32_t *p = w.cnb[k];
-            R v = 0;
-            if (p) {
-                if (W == 2) v = (R)p[2 * y] | ((R)p[2 * y + 1] << (W == 2 ? 32 : 0));
-                else v = (R)p[y];
-            }
-            S.nb[k][y] = v;
-        }
+        load_neighbours<N, MAXN>(w.cnb, S);  // S.nb: no halo lines here
         __syncthreads();
         count_loaded<N, MAXN>(S, w.count_out, w.slab_out);
     }
@@ -748,7 +773,7 @@ __device__ void pack_chunk(const FillWork &w, FillShared<MAXN> &S) {
     for (int i = threadIdx.x; i < N * N * W; i += kBlock) {
         const int r = i / W, j = i - r * W;
         const int xs = j * 32, xe = min(N, xs + 32);
-        const uint8_t *row = w.ids + (size_t)r * N;  // row r = y*N + z -> ids[x + N*z + N*N*y]
+        const GlobalPtr<const uint8_t> row = as_global<const uint8_t>(w.ids + (size_t)r * N);  // row r = y*N + z -> ids[x + N*z + N*N*y]
         uint32_t bits = 0;
         for (int x = xs; x < xe; x++) {
             const uint32_t b = row[x];
@@ -827,6 +852,7 @@ fill_kernel(const FillWork *__restrict__ work, const int32_t *__restrict__ order
     __shared__ FillShared<MAXN> S;
     const int item = order ? order[blockIdx.x] : (int)blockIdx.x;
     if (!order_entry_ok(item, n, error)) return;
+    if (work[item].variant) return;  // fill_fast_kernel's
     fill_item<MAXN>(work[item], terrains, lut, S);
 }
 
@@ -841,7 +867,604 @@ fill_split_kernel(const FillWork *__restrict__ work, const int32_t *__restrict__
     const int k = (int)blockIdx.x / parts, part = (int)blockIdx.x - k * parts;
     const int item = order ? order[k] : k;
     if (!order_entry_ok(item, n, error)) return;
+    if (work[item].variant) return;  // fill_fast_kernel's
     fill_item<MAXN, true>(work[item], terrains, lut, S, part, parts);
+}
+
+// ---- density with a decided sign
+//
+// A density voxel needs only the sign of fbm - threshold, and near the
+// threshold that sign needs the oracle's roundings; elsewhere any evaluation
+// with a known error decides it.  At a fixed column an octave is, within one
+// y cell, A0 + A1 fy + fade(fy) (D0 + D1 fy): three FMAs per voxel and octave
+// instead of the 29 operations of the oracle's blend.  A voxel whose sum lies
+// within `eps` of its threshold (about one in 10^5) has its row evaluated
+// again in the oracle's order (exact_fbm), so every bit is the oracle's.
+//
+// Error bound, in units of e = 2^-24 times the sum of |amplitude| (S), O
+// octaves.  Both evaluations take the same rounded fractions and fades and
+// approximate the same polynomial in them.  The oracle: 1 for a gradient, 5
+// per lerp level, 1 for the amplitude, O for the sums: 17 + O.  Here: 1 and 2
+// for a table entry's slopes and offset, 7 for a plane's value, 2.5 for its
+// slope, so 9.5 for a blend of two planes; 12 for the differences D0, D1 and
+// D; 2 per FMA into the running sum, which stays below 4 S, so 4 O, and 2 O
+// for the sum of the A0; 1 for fy - 1, which the oracle rounds.  Together
+// below 40 + 7 O; eps is (48 + 8 O) e S.  The threshold's own rounding is added to it.  NaN and
+// infinities satisfy neither comparison and so take the exact row.
+//
+// Bound by VALU issue at four waves per SIMD: per 64 voxels of four octaves 12
+// FMAs, two comparisons and two lane writes (a comparison, a lane write, a
+// shift or an SGPR operand issues in 4 cycles, an FMA, add or right shift in
+// 2), about 10 more for the columns' coefficients and the tables.  4096 chunks
+// of 32^3, four octaves: 128 us, against 376 us for the octave-inner loop of
+// the general kernels (152 VALU per 64 voxels); 1640 chunks under the
+// reference rule 49 against 146 us, 323 chunks of 64^3 136 against 381 us, 1023
+// chunks of six octaves 127 against 400 us.  Two columns per lane at five or
+// six waves per SIMD, or reading the next row's terms early, changed nothing
+// (143, 142, 139 against 136 us at that stage).
+template <int MAXN> struct FastShared {
+    // perm as byte offsets into itself (4 * perm[i & 255]) and perm's
+    // gradients as byte offsets (16 * (perm[i & 255] & 15)); three periods,
+    // so that a cell index plus a position in the chunk needs no wrap.  A
+    // heightmap keeps the plain permutation in perm.
+    int perm[768];
+    union {
+        int plut[768];
+        typename RowType<MAXN>::T nb[4][MAXN];  // counting, after the rows
+    };
+    float4 grad[kMaxOctaves][16];  // amplitude * gradient (x, col, row) by hash
+    union {
+        float4 tab[kBlock / 64][fast_tab(MAXN)];
+        alignas(16) uint8_t height[fast_slab(MAXN) * MAXN];  // heightmaps: solid layers per column
+    };
+    float2 yrow[MAXN * (kMaxOctaves + 1)];
+    float2 xcol[kMaxOctaves * MAXN];  // (fx, fade(fx)) per octave and x
+    uint8_t ycell[kMaxOctaves * MAXN], xcell[kMaxOctaves * MAXN];
+    uint32_t ychg[MAXN];
+    typename RowType<MAXN>::T occ[fast_slab(MAXN) * MAXN];
+    uint32_t red[kBlock / 64];
+};
+
+__device__ __forceinline__ float grad3(int hash, float x, float y, float z) {
+    const int h = hash & 15;
+    const float u = h < 8 ? x : y;
+    const float v = h < 4 ? y : (h == 12 || h == 14 ? x : z);
+    return ((h & 1) ? -u : u) + ((h & 2) ? -v : v);
+}
+
+// The oracle's fBm at (x, y, z), operation for operation; p4 = 4 * perm.
+__device__ float exact_fbm(const TerrainDev &T, const int *p4, float x, float y, float z) {
+    auto p = [p4](int i) { return p4[i] >> 2; };
+    float sum = 0.0f, f = T.frequency, amp = 1.0f;
+#pragma unroll 1
+    for (int o = 0; o < T.octaves; o++) {
+        const float xs = x * f, ys = y * f, zs = z * f;
+        const float fx = floorf(xs), fy = floorf(ys), fz = floorf(zs);
+        const int X = cell8(fx), Y = cell8(fy), Z = cell8(fz);
+        const float xr = xs - fx, yr = ys - fy, zr = zs - fz;
+        const float u = fade(xr), v = fade(yr), w = fade(zr);
+        const float x1 = xr - 1.0f, y1 = yr - 1.0f, z1 = zr - 1.0f;
+        const int A = p(X) + Y, AA = p(A) + Z, AB = p(A + 1) + Z;
+        const int B = p(X + 1) + Y, BA = p(B) + Z, BB = p(B + 1) + Z;
+        const float n = lerp(
+            w,
+            lerp(v, lerp(u, grad3(p(AA), xr, yr, zr), grad3(p(BA), x1, yr, zr)),
+                 lerp(u, grad3(p(AB), xr, y1, zr), grad3(p(BB), x1, y1, zr))),
+            lerp(v, lerp(u, grad3(p(AA + 1), xr, yr, z1), grad3(p(BA + 1), x1, yr, z1)),
+                 lerp(u, grad3(p(AB + 1), xr, y1, z1), grad3(p(BB + 1), x1, y1, z1))));
+        sum = sum + amp * n;
+        f = f * T.lacunarity;
+        amp = amp * T.gain;
+    }
+    return sum;
+}
+
+// Per-row terms of rows [0, N): S.yrow[y * (OCT + 1) + o] = (fy, fade(fy)) of
+// octave o, entry OCT = (threshold + eps, threshold - eps); S.ycell[o * N + y]
+// = y cell counted from row 0's; S.ychg[y] bit o = octave o enters a new cell.
+// Likewise S.xcol and S.xcell [o * N + x] for the columns.
+// S.grad = the gradients times the octave's amplitude (G: the axes' gradients).
+template <int N, int OCT, class SH>
+__device__ __forceinline__ void build_terms(const TerrainDev &T, const float4 *G, int ox, int oy,
+                                            SH &S) {
+    for (int i = threadIdx.x; i < OCT * 16; i += kBlock) {
+        const int o = i / 16;
+        float a = o < T.octaves ? 1.0f : 0.0f;
+        for (int k = 0; k < o; k++) a = a * T.gain;
+        const float4 g = G[i & 15];
+        S.grad[o][i & 15] = make_float4(a * g.x, a * g.y, a * g.z, 0.0f);
+    }
+    for (int i = kBlock - 1 - (int)threadIdx.x; i < OCT * N; i += kBlock) {
+        const int o = i / N, x = i - o * N;
+        float f = T.frequency;
+        for (int k = 0; k < o; k++) f = f * T.lacunarity;
+        if (o >= T.octaves) f = 0.0f;
+        const float X = (float)(ox + x) * f, fl = floorf(X), fx = X - fl;
+        S.xcol[i] = make_float2(fx, fade(fx));
+        S.xcell[i] = (uint8_t)((int)fl - (int)floorf((float)ox * f));
+    }
+    for (int y = threadIdx.x; y < N; y += kBlock) {
+        float f = T.frequency, amp = 1.0f, mag = 0.0f;
+        uint32_t chg = 0;
+#pragma unroll
+        for (int o = 0; o < OCT; o++) {
+            float fy = 0.0f, v = 0.0f;
+            int cell = 0;
+            if (o < T.octaves) {
+                const float Y = (float)(oy + y) * f;
+                const float fl = floorf(Y);
+                fy = Y - fl;
+                v = fade(fy);
+                cell = (int)fl - (int)floorf((float)oy * f);
+                if (floorf((float)(oy + y - 1) * f) != fl) chg |= 1u << o;
+                mag += fabsf(amp);
+                f = f * T.lacunarity;
+                amp = amp * T.gain;
+            }
+            S.yrow[y * (OCT + 1) + o] = make_float2(fy, v);
+            S.ycell[o * N + y] = (uint8_t)cell;
+        }
+        const float thr = T.kind == kReference ? 0.0f : (float)(oy + y) * T.y_scale;
+        const float eps = (float)(48 + 8 * OCT) * 5.9604645e-08f * mag + fabsf(thr) * 2.3841858e-07f;
+        S.yrow[y * (OCT + 1) + OCT] = make_float2(thr + eps, thr - eps);
+        S.ychg[y] = chg;
+    }
+}
+
+// Stores the rows of C * 64 / N lines from line z0: lane r < rows holds the
+// ballots of row y0 + r (klo, khi: C halves of 64 / N lines each).
+template <int N, int MAXN, int C, class SH>
+__device__ __forceinline__ void put_lines(SH &S, const uint32_t (&klo)[C], const uint32_t (&khi)[C],
+                                          int z0, int y0, int rows, int lane) {
+    constexpr int RS = RowStride<MAXN>::v;
+    if (lane >= rows) return;
+    uint32_t *dst = reinterpret_cast<uint32_t *>(S.occ) + ((y0 + lane) * N + z0) * RS;
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        if constexpr (N == 64) {
+            dst[2 * c] = klo[c];
+            dst[2 * c + 1] = khi[c];
+        } else if constexpr (N == 32) {
+            dst[2 * c * RS] = klo[c];
+            dst[(2 * c + 1) * RS] = khi[c];
+            if (RS == 2) dst[2 * c * RS + 1] = dst[(2 * c + 1) * RS + 1] = 0u;
+        } else {
+            const uint32_t v[4] = {klo[c] & 0xFFFFu, klo[c] >> 16, khi[c] & 0xFFFFu, khi[c] >> 16};
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                dst[(4 * c + k) * RS] = v[k];
+                if (RS == 2) dst[(4 * c + k) * RS + 1] = 0u;
+            }
+        }
+    }
+}
+
+// Rows [y_lo, y_hi) of a density (or reference-rule) chunk into S.occ (from
+// its start).  A wave
+// takes C * 64 / N lines along x, so a lane holds C columns (same x, lines
+// 64 / N apart) and reads each row's terms once for the C of them.  Per
+// octave the lines' lattice gradients are blended along z once into a table
+// of the wave (one entry per line, y plane and lattice x: value slope qx,
+// offset q0 and row slope qy); a column that enters a y cell blends four
+// entries along x into its A0, A1, D0, D1.
+template <int N, int MAXN, int OCT, int C, class SH>
+__device__ void density_rows_fast(const TerrainDev &T, int ox, int oy, int oz, SH &S, int y_lo,
+                                  int y_hi) {
+    constexpr int L = 64 / N, LINES = L * C, RS = RowStride<MAXN>::v;
+    constexpr int SLOTS = 64 / LINES;
+    const bool ref = T.kind == kReference;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int sub = lane / N, xl = lane % N;
+    float4 *tab = S.tab[wave];
+    float fo[OCT];
+    int lx[OCT];
+    {
+        float f = T.frequency;
+#pragma unroll
+        for (int o = 0; o < OCT; o++) {
+            const bool on = o < T.octaves;
+            fo[o] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(on ? f : 0.0f)));
+            lx[o] = __builtin_amdgcn_readfirstlane((int)S.xcell[o * N + N - 1]) + 2;
+            f = f * T.lacunarity;
+        }
+    }
+    for (int g = wave; g < N / LINES; g += kBlock / 64) {
+        int r0 = y_lo;
+#pragma unroll 1
+        while (r0 < y_hi) {
+            // as many rows as the wave's table holds the planes of
+            int rows = y_hi - r0;
+            int np[OCT], at[OCT];
+            for (;;) {
+                int e = 0;
+#pragma unroll
+                for (int o = 0; o < OCT; o++) {
+                    np[o] = __builtin_amdgcn_readfirstlane(
+                        (int)S.ycell[o * N + r0 + rows - 1] - (int)S.ycell[o * N + r0] + 2);
+                    at[o] = e;
+                    e += LINES * np[o] * lx[o];
+                }
+                if (e <= fast_tab(MAXN) || rows == 1) break;  // one row fits: fast_variant
+                rows = (rows + 1) / 2;
+            }
+            wave_sync();  // the previous rows' reads of the table
+            // table: lane = (slot, line); the line's z terms once per octave
+            {
+                int lane_t = lane;  // keeps these terms from being hoisted into the rows' registers
+                asm volatile("" : "+v"(lane_t));
+                const int line = lane_t % LINES, slot = lane_t / LINES;
+                const char *perm = reinterpret_cast<const char *>(S.perm);
+                const char *plut = reinterpret_cast<const char *>(S.plut);
+                auto at4 = [](const char *p, int off) { return *reinterpret_cast<const int *>(p + off); };
+#pragma unroll
+                for (int o = 0; o < OCT; o++) {
+                    const float Z = (float)(oz + g * LINES + line) * fo[o];
+                    const float zl = floorf(Z);
+                    const float z = Z - zl, z1 = z - 1.0f, w = fade(z);
+                    const int Z4 = ((int)zl & 255) * 4;
+                    const int X4 = ((int)floorf((float)ox * fo[o]) & 255) * 4;
+                    const int Y4 = (((int)floorf((float)oy * fo[o]) + (int)S.ycell[o * N + r0]) & 255) * 4;
+                    const char *grad = reinterpret_cast<const char *>(S.grad[o]);
+                    // two planes at a time (the last twice when they are odd):
+                    // each is a chain of dependent LDS reads
+                    auto planes = [&](float4 *dst, auto hashes) {
+                        const int last = np[o] - 1;
+#pragma unroll 1
+                        for (int p = 0; p <= last; p += 2) {
+                            const int q = min(p + 1, last);
+                            int h[4];
+                            hashes(p * 4, h[0], h[1]);
+                            hashes(q * 4, h[2], h[3]);
+                            float4 E[2];
+#pragma unroll
+                            for (int k = 0; k < 2; k++) {
+                                const float4 G0 = *reinterpret_cast<const float4 *>(grad + h[2 * k]);
+                                const float4 G1 = *reinterpret_cast<const float4 *>(grad + h[2 * k + 1]);
+                                const float q0 = G0.y * z, q1 = G1.y * z1;
+                                E[k] = make_float4(fmaf(w, G1.x - G0.x, G0.x), fmaf(w, q1 - q0, q0),
+                                                   fmaf(w, G1.z - G0.z, G0.z), 0.0f);
+                            }
+                            dst[p * lx[o]] = E[0];
+                            dst[q * lx[o]] = E[1];
+                        }
+                    };
+#pragma unroll 1
+                    for (int i = slot; i < lx[o]; i += SLOTS) {
+                        float4 *dst = tab + at[o] + line * (np[o] * lx[o]) + i;
+                        const int px = at4(perm, X4 + i * 4);
+                        if (ref) {  // perm[perm[perm[X] + Z] + Y]
+                            const int a0 = at4(perm, px + Z4) + Y4, a1 = at4(perm, px + Z4 + 4) + Y4;
+                            planes(dst, [&](int p4, int &h0, int &h1) {
+                                h0 = at4(plut, a0 + p4);
+                                h1 = at4(plut, a1 + p4);
+                            });
+                        } else {  // perm[perm[perm[X] + Y] + Z]
+                            const int a0 = px + Y4;
+                            planes(dst, [&](int p4, int &h0, int &h1) {
+                                const int a = at4(perm, a0 + p4) + Z4;
+                                h0 = at4(plut, a);
+                                h1 = at4(plut, a + 4);
+                            });
+                        }
+                    }
+                }
+            }
+            wave_sync();
+            uint64_t chm[OCT], any = 0;
+            {
+                const uint32_t m = lane < rows ? S.ychg[r0 + lane] : 0u;
+#pragma unroll
+                for (int o = 0; o < OCT; o++) {
+                    chm[o] = __ballot((m >> o) & 1u) | 1ull;
+                    any |= chm[o];
+                }
+            }
+            float A0[C][OCT], A1[C][OCT], D0[C][OCT], D1[C][OCT], As[C];
+            uint32_t klo[C], khi[C];
+            uint64_t doubt[C];
+#pragma unroll
+            for (int c = 0; c < C; c++) klo[c] = khi[c] = 0u, doubt[c] = 0ull;
+            int r = 0;
+#pragma unroll 1
+            while (r < rows) {
+                // octaves entering a new y cell at this row
+#pragma unroll
+                for (int o = 0; o < OCT; o++) {
+                    if (!((chm[o] >> r) & 1ull)) continue;
+                    const int p = __builtin_amdgcn_readfirstlane(
+                        (int)S.ycell[o * N + r0 + r] - (int)S.ycell[o * N + r0]);
+                    const float2 xt = S.xcol[o * N + xl];
+                    const float fx = xt.x, x1 = fx - 1.0f, u = xt.y;
+                    const float4 *b = tab + at[o] + p * lx[o] + S.xcell[o * N + xl] + sub * (np[o] * lx[o]);
+#pragma unroll
+                    for (int c = 0; c < C; c++) {
+                        const float4 *e0 = b + c * (L * np[o] * lx[o]), *e1 = e0 + lx[o];
+                        const float4 a = e0[0], q = e0[1], d = e1[0], e = e1[1];
+                        const float l0 = fmaf(a.x, fx, a.y), l1 = fmaf(q.x, x1, q.y);
+                        const float t0 = fmaf(d.x, fx, d.y), t1 = fmaf(e.x, x1, e.y);
+                        const float P0 = fmaf(u, l1 - l0, l0), P1 = fmaf(u, q.z - a.z, a.z);
+                        const float Q0 = fmaf(u, t1 - t0, t0), Q1 = fmaf(u, e.z - d.z, d.z);
+                        A0[c][o] = P0;
+                        A1[c][o] = P1;
+                        D0[c][o] = (Q0 - Q1) - P0;
+                        D1[c][o] = Q1 - P1;
+                        // one column's entries in registers at a time
+                        asm volatile("" ::: "memory");
+                    }
+                }
+#pragma unroll
+                for (int c = 0; c < C; c++) {
+                    As[c] = A0[c][0];
+#pragma unroll
+                    for (int o = 1; o < OCT; o++) As[c] += A0[c][o];
+                }
+                const uint64_t rest = r < 63 ? any >> (r + 1) : 0ull;
+                const int end = rest ? min(rows, r + 1 + __builtin_ctzll(rest)) : rows;
+#pragma unroll 1
+                for (; r < end; r++) {
+                    float2 t[OCT + 1];
+#pragma unroll
+                    for (int o = 0; o <= OCT; o++) t[o] = S.yrow[(r0 + r) * (OCT + 1) + o];
+                    float acc[C], d[C];
+#pragma unroll
+                    for (int c = 0; c < C; c++) acc[c] = As[c];
+#pragma unroll
+                    for (int o = 0; o < OCT; o++) {
+#pragma unroll
+                        for (int c = 0; c < C; c++) d[c] = fmaf(D1[c][o], t[o].x, D0[c][o]);
+#pragma unroll
+                        for (int c = 0; c < C; c++) acc[c] = fmaf(A1[c][o], t[o].x, acc[c]);
+#pragma unroll
+                        for (int c = 0; c < C; c++) acc[c] = fmaf(t[o].y, d[c], acc[c]);
+                    }
+                    uint64_t sure[C], all = ~0ull;
+#pragma unroll
+                    for (int c = 0; c < C; c++) {
+                        const uint64_t above = __ballot(acc[c] > t[OCT].x);
+                        const uint64_t below = __ballot(acc[c] < t[OCT].y);
+                        const uint64_t solid = ref ? below : above;
+                        sure[c] = above | below;
+                        all &= sure[c];
+                        klo[c] = write_lane((uint32_t)solid, (uint32_t)r, klo[c]);
+                        khi[c] = write_lane((uint32_t)(solid >> 32), (uint32_t)r, khi[c]);
+                    }
+                    if (all != ~0ull) {  // uniform, rare
+#pragma unroll
+                        for (int c = 0; c < C; c++)
+                            if (sure[c] != ~0ull) doubt[c] |= 1ull << r;
+                    }
+                }
+            }
+            put_lines<N, MAXN, C>(S, klo, khi, g * LINES, r0 - y_lo, rows, lane);
+            // rows with a voxel too near its threshold, in the oracle's order
+            uint32_t *occ = reinterpret_cast<uint32_t *>(S.occ);
+#pragma unroll 1
+            for (int c = 0; c < C; c++) {
+                uint64_t m = doubt[0];
+#pragma unroll
+                for (int k = 1; k < C; k++) m = c == k ? doubt[k] : m;
+#pragma unroll 1
+                for (; m; m &= m - 1ull) {
+                    const int y = r0 + __builtin_ctzll(m), zl = g * LINES + c * L + sub;
+                    const float wx = (float)(ox + xl), wy = (float)(oy + y), wz = (float)(oz + zl);
+                    const float s = exact_fbm(T, S.perm, wx, ref ? wz : wy, ref ? wy : wz);
+                    const bool solid = ref ? solid_of<true>(s, T, oy + y) : solid_of<false>(s, T, oy + y);
+                    const uint64_t b = __ballot(solid);
+                    wave_sync();  // after the row's first value
+                    if (xl == 0) {
+                        constexpr uint32_t MASK = N >= 32 ? 0xFFFFFFFFu : ((1u << (N & 31)) - 1u);
+                        uint32_t *dst = occ + ((y - y_lo) * N + zl) * RS;
+                        dst[0] = (uint32_t)(b >> (sub * N)) & MASK;
+                        if (N == 64) dst[RS - 1] = (uint32_t)(b >> 32);
+                    }
+                }
+            }
+            r0 += rows;
+        }
+    }
+}
+
+// Lines [z_lo, z_hi) of a 2-D fBm heightmap chunk, with their outputs: h =
+// floor(height_scale * (n + 1) / 2) clamped to [0, height_max]; voxel solid
+// iff wy <= h.  A workgroup takes lines and all their layers, so that a
+// column's noise is evaluated once.  Block ids come from the heights, four
+// columns to a dword: with H = the solid layers of each (0..64) in bytes, bit
+// 7 of 0x80 + H - (y + 1) says whether layer y is one of them.
+template <int N, int MAXN, class SH>
+__device__ void heightmap_lines_out(const FillWork &w, const TerrainDev &T, SH &S, int z_lo, int z_hi) {
+    constexpr int L = 64 / N, W = N == 64 ? 2 : 1, RS = RowStride<MAXN>::v;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lines = z_hi - z_lo;
+    for (int i = tid; i < N * lines; i += kBlock) {
+        const float wx = (float)(w.cx * N + i % N), wz = (float)(w.cz * N + z_lo + i / N);
+        float sum = 0.0f, amp = 1.0f, f = T.frequency;
+#pragma unroll 1
+        for (int o = 0; o < T.octaves; o++) {
+            sum = sum + amp * noise2(S.perm, wx * f, wz * f);
+            f = f * T.lacunarity;
+            amp = amp * T.gain;
+        }
+        const float hf = floorf((T.height_scale * (sum + 1.0f)) / 2.0f);
+        int h;
+        if (!(hf >= 0.0f)) h = 0;
+        else if (hf > (float)T.height_max) h = T.height_max;
+        else h = (int)hf;
+        const int64_t top = (int64_t)h - (int64_t)w.cy * N + 1;  // layers of the chunk up to h
+        S.height[i] = (uint8_t)(top < 0 ? 0 : top > N ? N : top);
+    }
+    __syncthreads();
+    // occupancy rows, line by line: S.occ[y * lines + z - z_lo]
+    uint32_t *occ = reinterpret_cast<uint32_t *>(S.occ);
+    for (int g = wave; g < lines / L; g += kBlock / 64) {
+        const int h = S.height[g * 64 + lane];
+        uint32_t klo = 0u, khi = 0u;
+        for (int y = 0; y < N; y++) {
+            const uint64_t b = __ballot(y < h);
+            klo = write_lane((uint32_t)b, (uint32_t)y, klo);
+            khi = write_lane((uint32_t)(b >> 32), (uint32_t)y, khi);
+        }
+        if (lane < N) {
+            uint32_t *dst = occ + (lane * lines + g * L) * RS;
+            constexpr uint32_t MASK = N >= 32 ? 0xFFFFFFFFu : ((1u << (N & 31)) - 1u);
+            if constexpr (N == 64) {
+                dst[0] = klo;
+                dst[1] = khi;
+            } else {
+                const uint64_t b = (uint64_t)khi << 32 | klo;
+#pragma unroll
+                for (int k = 0; k < L; k++) {
+                    dst[k * RS] = (uint32_t)(b >> (k * N)) & MASK;
+                    if (RS == 2) dst[k * RS + 1] = 0u;
+                }
+            }
+        }
+    }
+    // boundary planes x=0, x=N-1 (bit z per y), eight lines to a byte
+    const GlobalPtr<uint8_t> pb = as_global(reinterpret_cast<uint8_t *>(w.planes));
+    const int bytes = lines / 8;
+    for (int k = tid; k < 2 * N * bytes; k += kBlock) {
+        const int b = k % bytes, y = k / bytes % N, pl = k / (bytes * N);
+        uint32_t v = 0;
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            v |= (uint32_t)(y < (int)S.height[(b * 8 + j) * N + (pl ? N - 1 : 0)]) << j;
+        pb[(pl * N + y) * W * 4 + z_lo / 8 + b] = (uint8_t)v;
+        if (N == 16 && z_lo == 0 && b < 2) pb[(pl * N + y) * W * 4 + 2 + b] = 0;
+        if (N == 16 && z_lo == 0 && bytes == 1) pb[(pl * N + y) * W * 4 + 3] = 0;
+    }
+    // ids, 16 voxels per 16-byte store: a wave takes layers, a lane 16 columns
+    {
+        typedef uint32_t Ids16 __attribute__((ext_vector_type(4)));
+        const GlobalPtr<Ids16> ids = as_global(reinterpret_cast<Ids16 *>(w.ids));
+        const int groups = lines * N / 16;  // of 16 columns
+        const int per = groups < 64 ? 64 / groups : 1;  // layers of a wave pass
+        for (int g = lane % groups; g < groups; g += 64) {
+            const uint4 H = *reinterpret_cast<const uint4 *>(S.height + g * 16);
+            const uint32_t h[4] = {H.x + 0x80808080u, H.y + 0x80808080u, H.z + 0x80808080u,
+                                   H.w + 0x80808080u};
+            for (int y = wave * per + lane / groups; y < N; y += kBlock / 64 * per) {
+                const uint32_t sub = (uint32_t)(y + 1) * 0x01010101u;
+                Ids16 v;
+#pragma unroll
+                for (int k = 0; k < 4; k++) v[k] = ((h[k] - sub) >> 7) & (0x01010101u * kBlockGrass);
+                ids[(y * N + z_lo) * (N / 16) + g] = v;
+            }
+        }
+    }
+    __syncthreads();
+    // rows and boundary planes z=0, z=N-1
+    const GlobalPtr<uint32_t> out = as_global(w.occ), planes = as_global(w.planes);
+    for (int i = tid; i < N * lines * W; i += kBlock) {
+        const int y = i / (lines * W), r = i - y * (lines * W);
+        out[(y * N + z_lo) * W + r] = occ[(y * lines + r / W) * RS + r % W];
+    }
+    for (int k = tid; k < 2 * N * W; k += kBlock) {
+        const int pl = k / (N * W), y = k / W % N, j = k % W;
+        if (pl ? z_hi == N : z_lo == 0)
+            planes[((2 + pl) * N + y) * W + j] = occ[(y * lines + (pl ? lines - 1 : 0)) * RS + j];
+    }
+    if (tid == 0 && z_lo == 0) *as_global(w.meta) = kBlockGrass;
+}
+
+// Rows [y_lo, y_hi), at most fast_slab(MAXN) of them, of a chunk that the
+// host marked for this path, with their outputs.  OCT: octaves compiled for
+// (0: no 3-D noise).
+template <int N, int MAXN, int OCT, class SH>
+__device__ __forceinline__ void fast_rows(const FillWork &w, const TerrainDev &T, const float4 *G,
+                                          SH &S, int y_lo, int y_hi) {
+    using R = typename RowType<MAXN>::T;
+    const int ox = w.cx * N, oy = w.cy * N, oz = w.cz * N;
+    if constexpr (OCT > 0) {
+        build_terms<N, OCT>(T, G, ox, oy, S);
+        __syncthreads();
+        density_rows_fast<N, MAXN, OCT, fast_cols(N, MAXN, OCT)>(T, ox, oy, oz, S, y_lo, y_hi);
+    } else {
+        constexpr uint32_t ROW = N >= 32 ? 0xFFFFFFFFu : ((1u << (N & 31)) - 1u);
+        const R full = T.kind != kSolid ? (R)0 : N == 64 ? (R)~(R)0 : (R)ROW;
+        for (int i = threadIdx.x; i < (y_hi - y_lo) * N; i += kBlock) S.occ[i] = full;
+    }
+    __syncthreads();
+    write_chunk_outputs<N, MAXN>(w, S, true, kBlockGrass, y_lo, y_hi, y_lo);
+}
+
+// Workgroup `part` of `parts` on chunk w, each with N / parts layers (lines of
+// a heightmap); in a
+// batch of several edges a smaller chunk takes the parts that give its
+// workgroups as many rows as a 64^3 chunk's.  A whole chunk of edge up to 32
+// also counts its faces (FillWork.count_out).
+template <int N, int MAXN, class SH>
+__device__ __forceinline__ void fast_part(const FillWork &w, const TerrainDev &T, const float4 *G,
+                                          SH &S, int part, int parts) {
+    if (MAXN == 64 && N < 64) parts = max(1, parts * N / 64);
+    if (T.kind == kHeightmap) parts = min(parts, N / 8);  // whole bytes of the x planes
+    if (part >= parts) return;
+    const int rows = N / parts, y_lo = part * rows, y_hi = y_lo + rows;
+    if (T.kind == kHeightmap) {
+        heightmap_lines_out<N, MAXN>(w, T, S, y_lo, y_hi);
+    } else if (T.kind == kDensity || T.kind == kReference) {
+        switch (w.variant) {
+        case 2: fast_rows<N, MAXN, 2>(w, T, G, S, y_lo, y_hi); break;
+        case 3: fast_rows<N, MAXN, 3>(w, T, G, S, y_lo, y_hi); break;
+        case 4: fast_rows<N, MAXN, 4>(w, T, G, S, y_lo, y_hi); break;
+        case 6: fast_rows<N, MAXN, 6>(w, T, G, S, y_lo, y_hi); break;
+        default: fast_rows<N, MAXN, 8>(w, T, G, S, y_lo, y_hi); break;
+        }
+    } else {
+        fast_rows<N, MAXN, 0>(w, T, G, S, y_lo, y_hi);
+    }
+    if constexpr (MAXN <= 32) {
+        if (w.count_out && parts == 1) {
+            load_neighbours<N, MAXN>(w.cnb, S);
+            __syncthreads();
+            count_loaded<N, MAXN>(S, w.count_out, w.slab_out);
+        }
+    }
+}
+
+template <int MAXN>
+__device__ __forceinline__ void fast_item(const FillWork &w, const TerrainDev *terrains,
+                                          const GradLut *lut, FastShared<MAXN> &S, int part,
+                                          int parts) {
+    const TerrainDev &T = terrains[w.terrain];
+    const bool dens = T.kind == kDensity || T.kind == kReference;
+    if (dens || T.kind == kHeightmap) {
+        for (int i = threadIdx.x; i < (dens ? 768 : 512); i += kBlock) {
+            const int p = T.perm[i & 255];
+            S.perm[i] = dens ? 4 * p : p;
+            if (dens) S.plut[i] = (p & 15) * 16;
+        }
+    }
+    const float4 *G = (T.kind == kReference ? lut->r : lut->c)[0];
+    if (!dens) __syncthreads();  // the density terms' barrier covers its tables
+    switch (w.edge) {
+    case 16: fast_part<16, MAXN>(w, T, G, S, part, parts); break;
+    case 32: if constexpr (MAXN >= 32) fast_part<32, MAXN>(w, T, G, S, part, parts); break;
+    case 64: if constexpr (MAXN >= 64) fast_part<64, MAXN>(w, T, G, S, part, parts); break;
+    default: break;
+    }
+}
+
+// `parts` workgroups per chunk (1, 2, 4 or 8), each on a band of rows.
+template <int MAXN>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
+fill_fast_kernel(const FillWork *__restrict__ work, const int32_t *__restrict__ order, int32_t n,
+                 const TerrainDev *__restrict__ terrains, const GradLut *__restrict__ lut,
+                 int parts, uint32_t *__restrict__ error) {
+    __shared__ FastShared<MAXN> S;
+    const int k = (int)blockIdx.x / parts, part = (int)blockIdx.x - k * parts;
+    const int item = order ? order[k] : k;
+    if (!order_entry_ok(item, n, error)) return;
+    const FillWork &w = work[item];
+    if (!w.variant) return;  // the general kernel's
+    fast_item<MAXN>(w, terrains, lut, S, part, parts);
+}
+
+template <int MAXN>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
+fill_fast_one_kernel(FillWork w, const TerrainDev *__restrict__ terrains,
+                     const GradLut *__restrict__ lut, int parts) {
+    __shared__ FastShared<MAXN> S;
+    fast_item<MAXN>(w, terrains, lut, S, (int)blockIdx.x, parts);
 }
 
 template <int MAXN>
@@ -930,33 +1553,16 @@ struct SlabShared {
 template <class SH, int N> struct RowsOf { static constexpr int v = N * N; };
 template <int N> struct RowsOf<SlabShared, N> { static constexpr int v = kSlabLayers * N; };
 
-// Orders the LDS accesses of one wave: staging written by some lanes is read
-// by others of the same wave (LDS executes one wave's operations in order).
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 template <int N, int MAXN, int BLOCK = kBlock, class SH>
 __device__ __forceinline__ void load_rows(const MeshWork &w, SH &S) {
-    using R = typename RowType<MAXN>::T;
-    constexpr int W = N == 64 ? 2 : 1;
+    using R = typename RowType<N>::T;  // rows in memory: u64 pairs of words at N = 64
     const int tid = threadIdx.x;
     for (int r = tid; r < N * N; r += BLOCK) {
         R v;
-        if (W == 2) v = (R)w.occ[2 * r] | ((R)w.occ[2 * r + 1] << (W == 2 ? 32 : 0));
-        else v = (R)w.occ[r];
+        v = as_global(reinterpret_cast<const R *>(w.occ))[r];
         S.occ[r] = v;
     }
-    for (int i = tid; i < 4 * N; i += BLOCK) {
-        const int k = i / N, y = i - k * N;
-        R v = 0;
-        if (w.nb[k]) {
-            if (W == 2) v = (R)w.nb[k][2 * y] | ((R)w.nb[k][2 * y + 1] << (W == 2 ? 32 : 0));
-            else v = (R)w.nb[k][y];
-        }
-        S.nb[k][y] = v;
-    }
+    load_neighbours<N, MAXN, BLOCK>(w.nb, S);
 }
 
 // face_masks for local layer yl of a slab held in SlabShared (its halo
@@ -1006,7 +1612,7 @@ __device__ __forceinline__ void face_masks(const SH &S, int y, int z,
 // Loads slab `ylo / kSlabLayers` of a 64^3 chunk (rows are u32 pairs, low
 // word first) with its halo layers and neighbour-plane rows.
 __device__ __forceinline__ void load_slab(const MeshWork &w, SlabShared &S, int ylo) {
-    const uint64_t *occ = reinterpret_cast<const uint64_t *>(w.occ);
+    const GlobalPtr<const uint64_t> occ = as_global(reinterpret_cast<const uint64_t *>(w.occ));
     for (int i = threadIdx.x; i < (kSlabLayers + 2) * 64; i += kBlock) {
         const int y = ylo - 1 + (i >> 6);
         S.occ[i] = (y >= 0 && y < 64) ? occ[y * 64 + (i & 63)] : 0ull;
@@ -1014,7 +1620,7 @@ __device__ __forceinline__ void load_slab(const MeshWork &w, SlabShared &S, int 
     for (int i = threadIdx.x; i < 4 * kSlabLayers; i += kBlock) {
         const int k = i / kSlabLayers, yl = i - k * kSlabLayers;
         const uint64_t *p = reinterpret_cast<const uint64_t *>(w.nb[k]);
-        S.nb[k][yl] = p ? p[ylo + yl] : 0ull;
+        S.nb[k][yl] = p ? as_global(p)[ylo + yl] : 0ull;
     }
 }
 
@@ -1458,7 +2064,7 @@ __device__ void emit_rows(const MeshWork &w, uint64_t base, uint32_t F, const Me
                 // compiler would wait for all of the group's stores.
                 uint32_t blk = w.solid_type;
                 if (blk == kBlockMixed) {  // uniform
-                    blk = valid ? (uint32_t)w.ids[(size_t)x + (size_t)N * z + (size_t)N * N * y]
+                    blk = valid ? (uint32_t)as_global(w.ids)[(size_t)x + (size_t)N * z + (size_t)N * N * y]
                                 : (uint32_t)kBlockGrass;
                     blk = min(blk, (uint32_t)kBlockDirt);
                 }
@@ -2126,21 +2732,30 @@ __global__ void __launch_bounds__(kBlock) draw_write_kernel(Planes planes,
 // --------------------------------------------------------------- launchers
 hipError_t launch_fill(const FillWork *work, const int32_t *order, int32_t n, int32_t max_edge,
                        const TerrainDev *terrains, const GradLut *lut, uint32_t *error,
-                       int32_t parts_hint, hipStream_t s) {
+                       int32_t parts_hint, uint32_t kinds, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     if (parts_hint != 0 && parts_hint != 1 && parts_hint != 2 && parts_hint != 4 && parts_hint != 8)
         return hipErrorInvalidValue;
-    // small batches: several workgroups per chunk (density terrains with up
-    // to 4 octaves split their rows; other chunks are filled by the first of
-    // their workgroups; a chunk under 64^3 given 8 uses the first 4)
+    // small batches: several workgroups per chunk, each on a band of rows
     const int parts = fill_parts_for(n, max_edge, parts_hint);
+    const int grid = n * parts;
+    if (kinds & kFillFast) {
+        if (max_edge <= 16)
+            fill_fast_kernel<16><<<grid, kBlock, 0, s>>>(work, order, n, terrains, lut, parts, error);
+        else if (max_edge <= 32)
+            fill_fast_kernel<32><<<grid, kBlock, 0, s>>>(work, order, n, terrains, lut, parts, error);
+        else {  // a workgroup holds 16 layers of a 64^3 chunk
+            const int p = parts < 4 ? 4 : parts;
+            fill_fast_kernel<64><<<n * p, kBlock, 0, s>>>(work, order, n, terrains, lut, p, error);
+        }
+    }
+    if (!(kinds & kFillGeneral)) return hipGetLastError();
     if (parts == 1) {
         if (max_edge <= 16) fill_kernel<16><<<n, kBlock, 0, s>>>(work, order, n, terrains, lut, error);
         else if (max_edge <= 32) fill_kernel<32><<<n, kBlock, 0, s>>>(work, order, n, terrains, lut, error);
         else fill_kernel<64><<<n, kBlock, 0, s>>>(work, order, n, terrains, lut, error);
         return hipGetLastError();
     }
-    const int grid = n * parts;
     if (max_edge <= 16)
         fill_split_kernel<16><<<grid, kBlock, 0, s>>>(work, order, n, terrains, lut, parts, error);
     else if (max_edge <= 32)
@@ -2169,6 +2784,14 @@ hipError_t launch_scan(const uint32_t *counts, int32_t n, const MeshWork *items,
 
 hipError_t launch_fill_one(const FillWork &w, const TerrainDev *terrains, const GradLut *lut,
                            hipStream_t s) {
+    if (!w.noise_out && w.variant) {
+        // one chunk: a workgroup per four rows (two at edge 16)
+        const int parts = 8;
+        if (w.edge <= 16) fill_fast_one_kernel<16><<<parts, kBlock, 0, s>>>(w, terrains, lut, parts);
+        else if (w.edge <= 32) fill_fast_one_kernel<32><<<parts, kBlock, 0, s>>>(w, terrains, lut, parts);
+        else fill_fast_one_kernel<64><<<parts, kBlock, 0, s>>>(w, terrains, lut, parts);
+        return hipGetLastError();
+    }
     if (w.edge <= 16) fill_one_kernel<16><<<1, kBlock, 0, s>>>(w, terrains, lut);
     else if (w.edge <= 32) fill_one_kernel<32><<<1, kBlock, 0, s>>>(w, terrains, lut);
     else fill_one_kernel<64><<<1, kBlock, 0, s>>>(w, terrains, lut);

@@ -353,6 +353,7 @@ int admit(vx_server *S) {
     MeshWork *mw = (MeshWork *)(sl.pinned + up256((size_t)S->max_batch * sizeof(FillWork)));
     int32_t *ord = (int32_t *)((char *)mw + up256((size_t)S->max_batch * sizeof(MeshWork)));
     F->nb_present.resize(n);
+    uint32_t kinds = 0;
     for (int i = 0; i < n; i++) {
         const vx_request &r = F->reqs[i];
         const ChunkLayoutS L = layout_s(r.edge);
@@ -364,6 +365,8 @@ int admit(vx_server *S) {
         f.cz = r.coord.z;
         f.edge = r.edge;
         f.terrain = r.terrain_id;
+        f.variant = fill_variant(ctx->terrains[r.terrain_id], f.cx, f.cy, f.cz, f.edge);
+        kinds |= f.variant ? kFillFast : kFillGeneral;
         f.ids = (uint8_t *)c;
         f.occ = (uint32_t *)(c + L.occ);
         f.planes = (uint32_t *)(c + L.planes);
@@ -415,7 +418,7 @@ int admit(vx_server *S) {
     }
     if (e == hipSuccess)
         e = launch_fill(F->fill_dev, F->order_dev, n, F->max_edge, ctx->terrains_dev, ctx->lut_dev,
-                        F->overflow + 1, 0, s);
+                        F->overflow + 1, 0, kinds, s);
     if (e == hipSuccess) e = launch_count(F->mesh_dev, n, F->max_edge, F->counts, F->slabs, s);
     // the scan rewrites the order array (the fill has consumed it) as the
     // emission order, largest chunks first (emit items when slabbed)
