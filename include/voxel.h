@@ -328,7 +328,7 @@ int vx_batch_set_roles(vx_batch *batch, int32_t ratio);
 /* Tile shape of the VX_BATCH_STAGED form for small batches: workgroups per
  * chunk of the fill (1, 2, 4 or 8; used below 1,024 chunks, where the rule
  * is 2, 4 or 8, and 8 only for 64^3 chunks, which take at least 4) and per item of the emit (1..4;
- * used below 1,280 items, where the rule is 2, 3 or 4); 0 = the rule.
+ * used below 2,560 items, where the rule is 2 to 16); 0 = the rule.
  * Larger batches take one workgroup per chunk and per item whatever is set.
  * Other forms ignore it, and so does VX_BATCH_AUTO once the autotuner has
  * chosen a shape for the batch. */

@@ -1,0 +1,58 @@
+"""Meshes of one chunk, whose faces are shared between workgroups in tiles of
+at least 256: face counts on both sides of a tile, one face's worth of work,
+none, and the worst case; block types found while the ids are read."""
+import numpy as np
+import pytest
+
+import voxel_amd as V
+
+pytestmark = pytest.mark.gpu
+
+
+def isolated(edge, k):
+    """k voxels without neighbours: 6 k faces."""
+    ids = np.zeros((edge, edge, edge), np.uint8)
+    at = [(y, z, x) for y in range(0, edge, 2) for z in range(0, edge, 2) for x in range(0, edge, 2)]
+    for i in np.linspace(0, len(at) - 1, k).astype(int) if k else ():
+        ids[at[i]] = V.GRASS if i % 3 else V.DIRT
+    return ids.reshape(-1)
+
+
+@pytest.mark.parametrize("edge", [16, 32, 64])
+@pytest.mark.parametrize("voxels", [0, 1, 42, 43, 85, 86, 170, 171, 512])
+def test_mesh_parts(ctx, oracle_mod, edge, voxels):
+    print("[case]", edge, voxels, flush=True)
+    ids = isolated(edge, voxels)
+    ch = V.Chunk.from_ids(ctx, (1, 0, -1), edge, ids)
+    assert (ch.ids() == ids).all()
+    assert (ch.occupancy() == oracle_mod.occupancy(ids, edge)).all()
+    mesh = ch.create_mesh()
+    faces, inst, vert, idx = oracle_mod.mesh_buffers(ids, edge, (edge, 0, -edge), [None] * 4)
+    assert mesh.faces == len(faces) == 6 * len(np.unique(np.nonzero(ids)[0]))
+    got = mesh.instances()
+    assert (got["m"].view(np.uint32) == inst["m"].view(np.uint32)).all()
+    assert (got["tex"] == inst["tex"]).all()
+    assert (mesh.vertices().view(np.uint32) == vert.view(np.uint32)).all()
+    assert (mesh.indices() == idx).all()
+
+
+@pytest.mark.parametrize("edge", [16, 32, 64])
+def test_checkerboard_of_both_types(ctx, oracle_mod, edge):
+    y, z, x = np.indices((edge,) * 3)
+    ids = np.where((x + y + z) % 2, 1 + (x // 2 + y) % 2, 0).astype(np.uint8).reshape(-1)
+    mesh = V.Chunk.from_ids(ctx, (0, 0, 0), edge, ids).create_mesh()
+    faces, inst, _, _ = oracle_mod.mesh_buffers(ids, edge, (0, 0, 0), [None] * 4)
+    assert mesh.faces == len(faces) == 3 * edge ** 3
+    got = mesh.instances()
+    assert (got["tex"] == inst["tex"]).all()
+    assert (got["m"].view(np.uint32) == inst["m"].view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("bad", [3, 255])
+def test_ids_out_of_range_are_refused(ctx, bad):
+    for at in (0, 16 ** 3 - 1):
+        ids = np.ones(16 ** 3, np.uint8)
+        ids[at] = bad
+        with pytest.raises(V.VoxelError) as e:
+            V.Chunk.from_ids(ctx, (0, 0, 0), 16, ids)
+        assert e.value.status == V.ERR_INVALID

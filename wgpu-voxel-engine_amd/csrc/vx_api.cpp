@@ -586,8 +586,14 @@ extern "C" int vx_chunk_from_ids(vx_ctx *ctx, vx_coord coord, int32_t edge, cons
     if (!ctx || !out || !ids || !valid_edge(edge) || !coord_in_range(coord, edge))
         return VX_ERR_INVALID;
     const size_t nv = (size_t)edge * edge * edge;
-    for (size_t i = 0; i < nv; i++)
-        if (ids[i] > kBlockDirt) return VX_ERR_INVALID;
+    // one pass without branches: the largest id, and which solid ids occur
+    uint8_t top = 0, grass = 0, dirt = 0;
+    for (size_t i = 0; i < nv; i++) {
+        top = std::max(top, ids[i]);
+        grass |= ids[i] == kBlockGrass;
+        dirt |= ids[i] == kBlockDirt;
+    }
+    if (top > kBlockDirt) return VX_ERR_INVALID;
     std::lock_guard<std::recursive_mutex> g(ctx->mu);
     vx_chunk *c = new_chunk(ctx, coord, edge);
     if (!c) return VX_ERR_NOMEM;
@@ -599,19 +605,14 @@ extern "C" int vx_chunk_from_ids(vx_ctx *ctx, vx_coord coord, int32_t edge, cons
     bind_chunk_ptrs(c, (char *)c->block);
     hipError_t e = hipMemcpyAsync(c->ids, ids, nv, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);  // caller's buffer is pageable
-    if (e == hipSuccess) e = launch_pack_one(fill_work_of(c, -1), ctx->stream);
-    uint32_t meta0 = kBlockMixed;
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(ctx->pinned, c->meta, 4, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    c->solid_type = grass && dirt ? (uint32_t)kBlockMixed : dirt ? kBlockDirt : kBlockGrass;
+    if (e == hipSuccess) e = launch_pack_one(fill_work_of(c, -1), c->solid_type, ctx->stream);
     if (e != hipSuccess) {
         ctx->set_error(e, "vx_chunk_from_ids");
         ctx->dev_free(c->block);
         delete c;
         return VX_ERR_DEVICE;
     }
-    memcpy(&meta0, ctx->pinned, 4);
-    c->solid_type = meta0;
     *out = c;
     return VX_OK;
 }
@@ -758,7 +759,8 @@ extern "C" int vx_chunk_create_mesh(vx_ctx *ctx, vx_chunk *chunk, vx_chunk *cons
     std::lock_guard<std::recursive_mutex> g(ctx->mu);
     const MeshWork w = mesh_work_of(chunk, adj);
     uint32_t *count_dev = (uint32_t *)ctx->small_dev;
-    VX_HIP(ctx, launch_count_one(w, count_dev, ctx->stream));
+    uint32_t *slabs_dev = count_dev + 4;
+    VX_HIP(ctx, launch_count_one(w, count_dev, slabs_dev, ctx->stream));
     VX_HIP(ctx, hipMemcpyAsync(ctx->pinned, count_dev, 4, hipMemcpyDeviceToHost, ctx->stream));
     VX_HIP(ctx, hipStreamSynchronize(ctx->stream));
     uint32_t faces;
@@ -785,7 +787,7 @@ extern "C" int vx_chunk_create_mesh(vx_ctx *ctx, vx_chunk *chunk, vx_chunk *cons
         o.instances = m->instances;
         o.capacity = faces;
         o.formats = formats;
-        hipError_t e = launch_emit_one(w, 0, faces, o, ctx->tables_dev, count_dev + 1, ctx->stream);
+        hipError_t e = launch_emit_one(w, faces, slabs_dev, o, ctx->tables_dev, count_dev + 1, ctx->stream);
         if (e != hipSuccess) {
             ctx->set_error(e, "emit kernel");
             ctx->dev_free(m->block);

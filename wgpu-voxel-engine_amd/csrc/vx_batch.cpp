@@ -996,18 +996,18 @@ extern "C" int vx_batch_autotune(vx_ctx *ctx, vx_batch *b, int32_t reps, vx_tune
     // staged tile shapes for batches small enough that the launchers split
     // chunks (the fill, under kFillGrid chunks) or items (the emit, under
     // kEmitGrid items) over several workgroups: half and twice the fill's
-    // rule, and one or four (two when the rule gives four) emit workgroups
+    // rule, and one or four (two when the rule gives four or more) emit workgroups
     // per item, each beside the other stage's rule
     {
         const int32_t items = emit_items_of(b->n, b->n_items, b->max_edge);
-        const int hf = fill_parts_for(b->n, b->max_edge), he = emit_parts_for(items);
+        const int hf = fill_parts_for(b->n, b->max_edge), he = emit_parts_for(items, b->max_edge);
         if (b->n < kFillGrid) {
             cands.push_back({VX_BATCH_STAGED, 0, 0, hf / 2, 0});
             if (hf * 2 <= (b->max_edge > 32 ? 8 : 4)) cands.push_back({VX_BATCH_STAGED, 0, 0, hf * 2, 0});
         }
         if (items < kEmitGrid) {
             if (he != 1) cands.push_back({VX_BATCH_STAGED, 0, 0, 0, 1});
-            cands.push_back({VX_BATCH_STAGED, 0, 0, 0, he == 4 ? 2 : 4});
+            cands.push_back({VX_BATCH_STAGED, 0, 0, 0, he >= 4 ? 2 : 4});
         }
     }
     if (b->fused_ok) {

@@ -78,7 +78,7 @@ struct vx_ctx {
     vx::TerrainDev *terrains_dev = nullptr;
     vx::GradLut *lut_dev = nullptr;
     vx::MeshTables *tables_dev = nullptr;
-    void *small_dev = nullptr;  // [0] face count, [1] overflow flag of the per-chunk path
+    void *small_dev = nullptr;  // [0] face count, [1] overflow flag, [4..7] slab counts of the per-chunk path
     void *scratch = nullptr;    // staging for host-array entry points
     size_t scratch_bytes = 0;
     unsigned char *pinned = nullptr;  // 4 KiB pinned host staging for readbacks

@@ -13,7 +13,8 @@ namespace vx {
 constexpr int kBlock = 256;        // threads per workgroup (4 wave64)
 constexpr int kMaxOctaves = 8;     // fBm octaves supported by the noise tables
 constexpr int kDescTile = 4096;    // face descriptors staged in LDS per emit tile
-constexpr int kEmitGrid = 1280;    // emit workgroups that fill the GPU (5 per CU)
+constexpr int kEmitGrid = 2560;    // emit workgroups that fill the GPU twice (5 per CU at once)
+constexpr int kEmitGrid64 = 6144;  // the same over slabs of 64^3 chunks (4 per CU at once)
 constexpr int kFillGrid = 1024;    // fill workgroups that fill the GPU (4 per CU)
 
 // Terrain kinds (mirror of vx_terrain.kind in include/voxel.h).
@@ -186,14 +187,19 @@ inline int fill_parts_for(int32_t n, int32_t max_edge, int32_t hint = 0) {
     if (hint > 0) return hint;
     return 2 * n >= kFillGrid ? 2 : (max_edge > 32 && 8 * n <= kFillGrid) ? 8 : 4;
 }
-// Workgroups per emit item: one for kEmitGrid items or more; below that up to
-// 4, so that the grid still covers about kEmitGrid workgroups.  `hint` (1..4;
-// 0 = this rule) replaces the rule for the batches it would split.
-inline int emit_parts_for(int32_t items, int32_t hint = 0) {
+// Workgroups per emit item: one for kEmitGrid items or more; below that as
+// many as make kEmitGrid workgroups (kEmitGrid64 when the items are slabs of
+// 64^3 chunks, which hold more faces), at most 16, so that the last round of
+// workgroups is short.  On one 1,640-chunk batch of 32^3 1 / 2 / 3 / 4 parts
+// ran 184 / 169 / 172 / 177 us a pass, on 512 chunks 1 / 3 / 5 / 8 127 / 95 / 94
+// / 101 us, on 1,292 slabs 1 / 3 / 5 / 8 430 / 386 / 364 / 416 us; two parts at
+// 4,096 chunks or 4,100 mixed items lose 5% and 15%.  `hint` (1..4; 0 = this
+// rule) replaces the rule for the batches it would split.
+inline int emit_parts_for(int32_t items, int32_t max_edge, int32_t hint = 0) {
     if (items >= kEmitGrid) return 1;
     if (hint > 0) return hint;
-    const int p = (kEmitGrid + items - 1) / items;
-    return p < 4 ? p : 4;
+    const int p = ((max_edge > 32 ? kEmitGrid64 : kEmitGrid) + items - 1) / items;
+    return p < 16 ? p : 16;
 }
 // parts_hint: fill_parts_for's hint.  kinds: which chunks the work holds
 // (kFillFast: a FillWork.variant set, kFillGeneral: 0): a kernel for each.
@@ -220,9 +226,12 @@ hipError_t launch_scan(const uint32_t *counts, int32_t n, const MeshWork *items,
                        const uint64_t *base_in = nullptr);
 hipError_t launch_fill_one(const FillWork &w, const TerrainDev *terrains, const GradLut *lut,
                            hipStream_t s);
-hipError_t launch_pack_one(const FillWork &w, hipStream_t s);
-hipError_t launch_count_one(const MeshWork &w, uint32_t *count, hipStream_t s);
-hipError_t launch_emit_one(const MeshWork &w, uint64_t base, uint32_t faces, MeshOut out,
+// solid_type: FillWork.meta[0], from the host's reading of the ids.
+hipError_t launch_pack_one(const FillWork &w, uint32_t solid_type, hipStream_t s);
+// slabs: kSlabs face counts of a 64^3 chunk, written by the count and read by
+// the emit (smaller chunks do not use them).
+hipError_t launch_count_one(const MeshWork &w, uint32_t *count, uint32_t *slabs, hipStream_t s);
+hipError_t launch_emit_one(const MeshWork &w, uint32_t faces, const uint32_t *slabs, MeshOut out,
                            const MeshTables *tables, uint32_t *overflow, hipStream_t s);
 // parts_hint: emit_parts_for's hint.
 hipError_t launch_emit(const MeshWork *work, const int32_t *order, int32_t n, int32_t n_items,

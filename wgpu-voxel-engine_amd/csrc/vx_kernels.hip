@@ -760,36 +760,33 @@ __device__ __forceinline__ void fill_chunk_split(const FillWork &w, const Terrai
 }
 
 // Packs caller-provided u8 ids (already in w.ids) into occupancy rows and
-// boundary planes; meta[0] = the single solid block id, or kBlockMixed.
+// boundary planes of layers [y_lo, y_hi), 16 voxels per load.  meta[0] =
+// solid_type (from the host, which has read the ids).
 template <int N, int MAXN>
-__device__ void pack_chunk(const FillWork &w, FillShared<MAXN> &S) {
-    constexpr int W = N == 64 ? 2 : 1;
+__device__ void pack_chunk(const FillWork &w, FillShared<MAXN> &S, uint32_t solid_type, int y_lo,
+                           int y_hi) {
     constexpr int RS = RowStride<MAXN>::v;
-    __shared__ uint32_t s_types;
-    if (threadIdx.x == 0) s_types = 0;
-    __syncthreads();
-    uint32_t *occ = reinterpret_cast<uint32_t *>(S.occ);
-    uint32_t types = 0;
-    for (int i = threadIdx.x; i < N * N * W; i += kBlock) {
-        const int r = i / W, j = i - r * W;
-        const int xs = j * 32, xe = min(N, xs + 32);
-        const GlobalPtr<const uint8_t> row = as_global<const uint8_t>(w.ids + (size_t)r * N);  // row r = y*N + z -> ids[x + N*z + N*N*y]
+    constexpr int PER_ROW = N / 16;
+    typedef uint32_t Ids16 __attribute__((ext_vector_type(4)));
+    const GlobalPtr<const Ids16> ids = as_global(reinterpret_cast<const Ids16 *>(w.ids));
+    uint16_t *occ = reinterpret_cast<uint16_t *>(S.occ);
+    for (int q = y_lo * N * PER_ROW + threadIdx.x; q < y_hi * N * PER_ROW; q += kBlock) {
+        const Ids16 v = ids[q];
         uint32_t bits = 0;
-        for (int x = xs; x < xe; x++) {
-            const uint32_t b = row[x];
-            if (b != kBlockAir) bits |= 1u << (x - xs);
-            types |= 1u << (b & 7);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            // ids are 0..2: bit 0 of (id | id >> 1) is solid; the four bytes'
+            // bits gathered by one multiply
+            const uint32_t solid = (v[k] | v[k] >> 1) & 0x01010101u;
+            bits |= ((solid * 0x01020408u) >> 24) << (4 * k);
         }
-        occ[r * RS + j] = bits;
-        if (RS == 2 && W == 1) occ[r * RS + 1] = 0u;
+        const int r = q / PER_ROW, part = q - r * PER_ROW;
+        occ[r * RS * 2 + part] = (uint16_t)bits;
+        if (N == 16) occ[r * RS * 2 + 1] = 0;
+        if (RS == 2 && N <= 32 && part == 0) reinterpret_cast<uint32_t *>(S.occ)[r * RS + 1] = 0u;
     }
-    atomicOr(&s_types, types);
     __syncthreads();
-    const uint32_t solid_types = s_types & ~1u;
-    uint32_t st = kBlockMixed;
-    if (solid_types == 0) st = kBlockGrass;  // no solid voxel: type unused
-    else if ((solid_types & (solid_types - 1)) == 0) st = (uint32_t)(__ffs(solid_types) - 1);
-    write_chunk_outputs<N, MAXN>(w, S, false, st);
+    write_chunk_outputs<N, MAXN>(w, S, false, solid_type, y_lo, y_hi);
 }
 
 // SPLIT: the workgroup is part `part` of `parts` on this chunk.
@@ -1475,15 +1472,12 @@ __global__ void __launch_bounds__(kBlock) fill_one_kernel(FillWork w,
     fill_item<MAXN>(w, terrains, lut, S);
 }
 
-template <int MAXN>
-__global__ void __launch_bounds__(kBlock) pack_one_kernel(FillWork w) {
-    __shared__ FillShared<MAXN> S;
-    switch (w.edge) {
-    case 16: pack_chunk<16, MAXN>(w, S); break;
-    case 32: if (MAXN >= 32) pack_chunk<(MAXN >= 32 ? 32 : 16), MAXN>(w, S); break;
-    case 64: if (MAXN >= 64) pack_chunk<(MAXN >= 64 ? 64 : 16), MAXN>(w, S); break;
-    default: break;
-    }
+// One chunk of edge N, a workgroup per N / gridDim.x layers.
+template <int N>
+__global__ void __launch_bounds__(kBlock) pack_one_kernel(FillWork w, uint32_t solid_type) {
+    __shared__ FillShared<N> S;
+    const int rows = N / (int)gridDim.x, y = (int)blockIdx.x * rows;
+    pack_chunk<N, N>(w, S, solid_type, y, y + rows);
 }
 
 // --------------------------------------------------------------- mesh
@@ -1508,10 +1502,9 @@ struct HeavyRows {
     uint32_t n;
 };
 
-// LDS of an emit workgroup of BLOCK threads on a whole chunk (the batch
-// emit uses it up to MAXN = 32; a 64^3 chunk's 32 KB of u64 rows and 16 KB
-// of row firsts would allow only two workgroups per CU, so batches emit
-// those by slabs, and only the single-chunk emit takes MAXN = 64).
+// LDS of an emit workgroup of BLOCK threads on a whole chunk of edge up to 32
+// (a 64^3 chunk's 32 KB of u64 rows and 16 KB of row firsts would allow only
+// two workgroups per CU, so those are emitted by slabs).
 template <int MAXN, int BLOCK = kBlock> struct MeshShared {
     typename RowType<MAXN>::T occ[MAXN * MAXN];
     typename RowType<MAXN>::T nb[4][MAXN];
@@ -1718,9 +1711,10 @@ __global__ void __launch_bounds__(kBlock) count_kernel(const MeshWork *__restric
 }
 
 template <int MAXN>
-__global__ void __launch_bounds__(kBlock) count_one_kernel(MeshWork w, uint32_t *__restrict__ count) {
+__global__ void __launch_bounds__(kBlock) count_one_kernel(MeshWork w, uint32_t *__restrict__ count,
+                                                           uint32_t *__restrict__ slabs) {
     __shared__ CountShared<MAXN> S;
-    count_item<MAXN>(w, S, count, nullptr);
+    count_item<MAXN>(w, S, count, slabs);
 }
 
 // Emission order: chunks by descending face count (buckets of 16 faces,
@@ -1890,9 +1884,9 @@ __device__ __forceinline__ void walk_row_at(SH &S, int r, int x, uint32_t f, uin
 // descriptor walk deals rows to threads round-robin, since a tile's faces
 // often come from a band of consecutive rows (a surface) that consecutive
 // ownership (4 or 16 rows per thread) would leave to a handful of threads.
-// `parts` workgroups may share a chunk (small batches): part p emits tiles
-// p, p + parts, ... and the matching share of the index stores; each part
-// repeats the row scan.  With SlabShared the rows are those of one slab,
+// `parts` workgroups may share a chunk (small batches, one chunk): part p
+// emits tiles p, p + parts, ... and the matching share of the index stores;
+// each part repeats the row scan.  With SlabShared the rows are those of one slab,
 // layers ylo .. ylo + kSlabLayers - 1, whose first face is face `off` of
 // the chunk (indices are chunk-local).
 template <int N, int MAXN, bool INTERLEAVE, int BLOCK = kBlock, bool HEAVY = INTERLEAVE,
@@ -1922,6 +1916,11 @@ __device__ void emit_rows(const MeshWork &w, uint64_t base, uint32_t F, const Me
             dst[q] = v;
         }
     }
+    constexpr uint32_t TILE = sizeof(S.desc) / sizeof(S.desc[0]);
+    // parts share the faces evenly, in tiles of at least a face per thread
+    const uint32_t tile =
+        parts > 1 ? min(TILE, max((uint32_t)BLOCK, ((F + parts - 1) / parts + 63u) & ~63u)) : TILE;
+    if ((uint32_t)part * tile >= F) return;
     const int r0 = tid * RPT;
     uint32_t rc[RPT];
     uint32_t mine = 0;
@@ -1953,9 +1952,8 @@ __device__ void emit_rows(const MeshWork &w, uint64_t base, uint32_t F, const Me
         __syncthreads();
     }
 
-    constexpr uint32_t TILE = sizeof(S.desc) / sizeof(S.desc[0]);
-    for (uint32_t t0 = (uint32_t)part * TILE; t0 < F; t0 += (uint32_t)parts * TILE) {
-        const uint32_t t1 = min(F, t0 + TILE);
+    for (uint32_t t0 = (uint32_t)part * tile; t0 < F; t0 += (uint32_t)parts * tile) {
+        const uint32_t t1 = min(F, t0 + tile);
         if constexpr (INTERLEAVE && !HEAVY) {
 #pragma unroll 1
             for (int r = tid; r < ROWS; r += BLOCK) {
@@ -2204,13 +2202,25 @@ emit_slab_kernel(const MeshWork *__restrict__ work, const int32_t *__restrict__ 
     }
 }
 
+// One chunk, `parts` workgroups on it (on each slab of a 64^3 chunk, whose
+// slab counts count_one_kernel wrote).
 template <int MAXN>
-__global__ void __launch_bounds__(kBlock) emit_one_kernel(MeshWork w, uint64_t base, uint32_t F,
-                                                          MeshOut out,
+__global__ void __launch_bounds__(kBlock) emit_one_kernel(MeshWork w, uint32_t F, MeshOut out,
                                                           const MeshTables *__restrict__ tables,
-                                                          uint32_t *__restrict__ overflow) {
+                                                          uint32_t *__restrict__ overflow, int parts) {
     __shared__ MeshShared<MAXN> S;
-    emit_item<MAXN>(w, base, F, out, tables, overflow, S, 0, 1);
+    emit_item<MAXN>(w, 0, F, out, tables, overflow, S, (int)blockIdx.x, parts);
+}
+
+__global__ void __launch_bounds__(kBlock) emit_slab_one_kernel(MeshWork w,
+                                                               const uint32_t *__restrict__ slabs,
+                                                               MeshOut out,
+                                                               const MeshTables *__restrict__ tables,
+                                                               uint32_t *__restrict__ overflow,
+                                                               int parts) {
+    __shared__ SlabShared S;
+    emit_slab_item(w, 0, slabs, (int)blockIdx.x / parts, out, tables, overflow, S,
+                   (int)blockIdx.x % parts, parts);
 }
 
 // --------------------------------------------------------------- fused
@@ -2798,25 +2808,29 @@ hipError_t launch_fill_one(const FillWork &w, const TerrainDev *terrains, const 
     return hipGetLastError();
 }
 
-hipError_t launch_pack_one(const FillWork &w, hipStream_t s) {
-    if (w.edge <= 16) pack_one_kernel<16><<<1, kBlock, 0, s>>>(w);
-    else if (w.edge <= 32) pack_one_kernel<32><<<1, kBlock, 0, s>>>(w);
-    else pack_one_kernel<64><<<1, kBlock, 0, s>>>(w);
+hipError_t launch_pack_one(const FillWork &w, uint32_t solid_type, hipStream_t s) {
+    if (w.edge <= 16) pack_one_kernel<16><<<4, kBlock, 0, s>>>(w, solid_type);
+    else if (w.edge <= 32) pack_one_kernel<32><<<8, kBlock, 0, s>>>(w, solid_type);
+    else pack_one_kernel<64><<<16, kBlock, 0, s>>>(w, solid_type);
     return hipGetLastError();
 }
 
-hipError_t launch_count_one(const MeshWork &w, uint32_t *count, hipStream_t s) {
-    if (w.edge <= 16) count_one_kernel<16><<<1, kBlock, 0, s>>>(w, count);
-    else if (w.edge <= 32) count_one_kernel<32><<<1, kBlock, 0, s>>>(w, count);
-    else count_one_kernel<64><<<1, kBlock, 0, s>>>(w, count);
+hipError_t launch_count_one(const MeshWork &w, uint32_t *count, uint32_t *slabs, hipStream_t s) {
+    if (w.edge <= 16) count_one_kernel<16><<<1, kBlock, 0, s>>>(w, count, nullptr);
+    else if (w.edge <= 32) count_one_kernel<32><<<1, kBlock, 0, s>>>(w, count, nullptr);
+    else count_one_kernel<64><<<1, kBlock, 0, s>>>(w, count, slabs);
     return hipGetLastError();
 }
 
-hipError_t launch_emit_one(const MeshWork &w, uint64_t base, uint32_t faces, MeshOut out,
+// Workgroups per chunk (per slab of a 64^3 chunk): about 256 faces each, so
+// that every wave of a workgroup writes one group of 64.
+hipError_t launch_emit_one(const MeshWork &w, uint32_t faces, const uint32_t *slabs, MeshOut out,
                            const MeshTables *tables, uint32_t *overflow, hipStream_t s) {
-    if (w.edge <= 16) emit_one_kernel<16><<<1, kBlock, 0, s>>>(w, base, faces, out, tables, overflow);
-    else if (w.edge <= 32) emit_one_kernel<32><<<1, kBlock, 0, s>>>(w, base, faces, out, tables, overflow);
-    else emit_one_kernel<64><<<1, kBlock, 0, s>>>(w, base, faces, out, tables, overflow);
+    const int parts = (int)((faces / (w.edge > 32 ? kSlabs : 1) + 255) / 256);
+    const int p = parts < 1 ? 1 : parts < 64 ? parts : 64;
+    if (w.edge <= 16) emit_one_kernel<16><<<p, kBlock, 0, s>>>(w, faces, out, tables, overflow, p);
+    else if (w.edge <= 32) emit_one_kernel<32><<<p, kBlock, 0, s>>>(w, faces, out, tables, overflow, p);
+    else emit_slab_one_kernel<<<kSlabs * p, kBlock, 0, s>>>(w, slabs, out, tables, overflow, p);
     return hipGetLastError();
 }
 
@@ -2833,7 +2847,7 @@ hipError_t launch_emit(const MeshWork *work, const int32_t *order, int32_t n, in
     // small batches: several workgroups per item, so the grid still covers
     // about a full GPU of workgroups and an item's tiles are emitted side by
     // side
-    const int parts = emit_parts_for(items, parts_hint);
+    const int parts = emit_parts_for(items, max_edge, parts_hint);
     const int grid = items * parts;
     if (max_edge <= 16)
         emit_kernel<16, kBlock><<<grid, kBlock, 0, s>>>(work, order, bases, counts, out, tables,
