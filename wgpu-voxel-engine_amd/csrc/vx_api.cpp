@@ -301,6 +301,29 @@ int vx_ctx::ensure_scratch(size_t bytes) {
     return VX_OK;
 }
 
+constexpr size_t kStageBytes = 1 << 20;
+
+char *vx_ctx::staging(size_t bytes) {
+    if (bytes > kStageBytes) return nullptr;
+    if (!stage) {
+        if (hipHostMalloc((void **)&stage, kStageBytes, hipHostMallocDefault) != hipSuccess ||
+            hipEventCreateWithFlags(&stage_ev, hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            if (stage) (void)hipHostFree(stage);
+            stage = nullptr;
+            stage_ev = nullptr;
+        }
+        return stage;
+    }
+    if (hipEventSynchronize(stage_ev) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return stage;
+}
+
+hipError_t vx_ctx::staging_queued() { return hipEventRecord(stage_ev, stream); }
+
 extern "C" int vx_abi_version(void) { return VX_ABI_VERSION; }
 
 extern "C" const char *vx_status_string(int status) {
@@ -381,6 +404,8 @@ extern "C" int vx_ctx_destroy(vx_ctx *ctx) {
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
+    if (ctx->stage) (void)hipHostFree(ctx->stage);
+    if (ctx->stage_ev) (void)hipEventDestroy(ctx->stage_ev);
     if (ctx->free_fence) (void)hipEventDestroy(ctx->free_fence);
     if (ctx->stream2) (void)hipStreamDestroy(ctx->stream2);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);

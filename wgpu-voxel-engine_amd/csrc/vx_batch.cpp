@@ -9,7 +9,8 @@
 //   store   per chunk i at chunk_off[i]: ids (N^3 B) | occupancy rows
 //           (N^2 * W u32) | 4 boundary planes (4 * N * W u32) | meta (solid block id, u32),
 //           each 256-byte aligned.
-//   ctl     counts[n] u32 | bases[n] u64 | total u64 | overflow u32 |
+//   desc    FillWork[n] | MeshWork[n] | fill order[n] (when not uniform) | control:
+//           counts[n] u32 | bases[n] u64 | total u64 | overflow u32 |
 //           emit_order[n_items] i32 | slabs[4 n] u32 (batches holding 64^3 chunks,
 //           whose emit works on y-slabs: n_items = n + 3 * (number of 64^3 chunks))
 //   arena   instances (68 B/face) | vertices (80 B/face) | indices (24 B/face)
@@ -285,9 +286,12 @@ hipError_t enqueue_all(vx_batch *b) {
     return e;
 }
 
+int ready_form(vx_batch *b);
+
 int capture_graph(vx_batch *b) {
     vx_ctx *ctx = b->ctx;
     drop_graph(b);
+    if (int st = ready_form(b)) return st;
     VX_HIP(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     hipError_t e = enqueue_all(b);
     hipGraph_t g = nullptr;
@@ -302,6 +306,83 @@ int capture_graph(vx_batch *b) {
     return VX_OK;
 }
 
+// Fill and mesh work of every chunk (device pointers into the batch's store
+// and the neighbours' planes).
+void describe(const vx_batch *b, FillWork *fw, MeshWork *mw) {
+    char *store = (char *)b->store;
+    for (int i = 0; i < b->n; i++) {
+        const vx_batch_req &r = b->reqs[i];
+        const Layout L = layout_of(r.edge);
+        char *base = store + b->chunk_off[i];
+        FillWork &f = fw[i];
+        f = FillWork{};
+        f.cx = r.coord.x;
+        f.cy = r.coord.y;
+        f.cz = r.coord.z;
+        f.edge = r.edge;
+        f.terrain = r.terrain_id;
+        f.variant = fill_variant(b->ctx->terrains[r.terrain_id], f.cx, f.cy, f.cz, f.edge);
+        f.ids = (uint8_t *)base;
+        f.occ = (uint32_t *)(base + L.occ);
+        f.planes = (uint32_t *)(base + L.planes);
+        f.meta = (uint32_t *)(base + L.meta);
+    }
+    for (int i = 0; i < b->n; i++) {
+        const vx_batch_req &r = b->reqs[i];
+        MeshWork &m = mw[i];
+        m = MeshWork{};
+        m.ox = r.coord.x * r.edge;
+        m.oy = r.coord.y * r.edge;
+        m.oz = r.coord.z * r.edge;
+        m.edge = r.edge;
+        m.occ = fw[i].occ;
+        m.ids = fw[i].ids;
+        m.solid_type = kBlockGrass;  // generated chunks hold only grass
+        static const int which[4] = {1, 0, 3, 2};  // facing plane of the neighbour
+        const size_t plane = (size_t)r.edge * words_per_row(r.edge);
+        for (int k = 0; k < 4; k++) {
+            const int j = r.nb[k];
+            if (j >= 0) m.nb[k] = fw[j].planes + which[k] * plane;
+            else if (j <= -2) m.nb[k] = b->ext[-2 - j]->planes + which[k] * plane;
+            else m.nb[k] = nullptr;
+        }
+        if (b->fill_counts) {
+            for (int k = 0; k < 4; k++) fw[i].cnb[k] = m.nb[k];
+            fw[i].count_out = b->counts + i;
+            fw[i].slab_out = b->slabs ? b->slabs + (size_t)kSlabs * i : nullptr;
+        }
+    }
+}
+
+// What the form a run takes needs beside the descriptors, made when that form
+// first runs: the persistent forms' work list, the split form's events.
+int ready_form(vx_batch *b) {
+    vx_ctx *ctx = b->ctx;
+    const int form = form_of(b);
+    if (form == VX_BATCH_SPLIT)
+        for (hipEvent_t &ev : b->split_ev)
+            if (!ev) VX_HIP(ctx, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    if (!use_fused(b) || b->fused_made) return VX_OK;
+    std::vector<FillWork> fw(b->n);
+    std::vector<MeshWork> mw(b->n);
+    std::vector<FusedWork> fu(b->n);
+    describe(b, fw.data(), mw.data());
+    for (int i = 0; i < b->n; i++) {
+        fu[i].f = fw[i];
+        fu[i].m = mw[i];
+        for (int k = 0; k < 4; k++) {
+            const int32_t j = b->reqs[i].nb[k];
+            fu[i].halo[k] = j >= 0 ? kHaloRecompute : j <= -2 ? kHaloResident : kHaloAbsent;
+            fu[i].nbi[k] = j >= 0 ? j : -1;
+        }
+    }
+    VX_HIP(ctx, hipMemcpyAsync(b->fused_dev, fu.data(), fu.size() * sizeof(FusedWork),
+                               hipMemcpyHostToDevice, ctx->stream));
+    VX_HIP(ctx, hipStreamSynchronize(ctx->stream));  // fu is pageable
+    b->fused_made = true;
+    return VX_OK;
+}
+
 void free_batch(vx_batch *b) {
     vx_ctx *ctx = b->ctx;
     (void)hipStreamSynchronize(ctx->stream);
@@ -312,11 +393,8 @@ void free_batch(vx_batch *b) {
     ctx->dev_free(b->planes_dev);
     if (b->planes_pin) (void)hipHostFree(b->planes_pin);
     if (b->planes_ev) (void)hipEventDestroy(b->planes_ev);
-    ctx->dev_free(b->fill_dev);
-    ctx->dev_free(b->mesh_dev);
-    ctx->dev_free(b->order_dev);
+    ctx->dev_free(b->desc);
     ctx->dev_free(b->coords_dev);
-    ctx->dev_free(b->ctl);
     ctx->dev_free(b->arena);
     ctx->dev_free(b->fused_dev);
     ctx->dev_free(b->fctl);
@@ -470,69 +548,30 @@ extern "C" int vx_batch_create_ext(vx_ctx *ctx, const vx_batch_req *reqs, int32_
         ext[e]->refs.fetch_add(1);
         b->ext.push_back(ext[e]);
     }
-    if ((st = ctx->dev_alloc((size_t)n * sizeof(FillWork), (void **)&b->fill_dev))) return fail(st);
-    if ((st = ctx->dev_alloc((size_t)n * sizeof(MeshWork), (void **)&b->mesh_dev))) return fail(st);
     const bool slabbed = b->max_edge > 32;
     b->n_items = n;
     if (slabbed)
         for (int i = 0; i < n; i++) b->n_items += reqs[i].edge == 64 ? kSlabs - 1 : 0;
-    const size_t ctl_bytes = up256((size_t)n * 4) + up256((size_t)n * 8) + 256 +
-                             up256((size_t)b->n_items * 4) +
-                             (slabbed ? up256((size_t)kSlabs * n * 4) : 0);
-    if ((st = ctx->dev_alloc(ctl_bytes, &b->ctl))) return fail(st);
-    b->counts = (uint32_t *)b->ctl;
-    b->bases = (uint64_t *)((char *)b->ctl + up256((size_t)n * 4));
-    b->total = (uint64_t *)((char *)b->bases + up256((size_t)n * 8));
+    // one block, one upload: fill work | mesh work | fill order | control
+    const size_t off_mesh = up256((size_t)n * sizeof(FillWork));
+    const size_t off_order = off_mesh + up256((size_t)n * sizeof(MeshWork));
+    const size_t off_ctl = off_order + (b->uniform ? 0 : up256((size_t)n * 4));
+    const size_t off_bases = off_ctl + up256((size_t)n * 4);
+    const size_t off_total = off_bases + up256((size_t)n * 8);
+    const size_t off_emit = off_total + 256;
+    const size_t off_slabs = off_emit + up256((size_t)b->n_items * 4);
+    const size_t desc_bytes = off_slabs + (slabbed ? up256((size_t)kSlabs * n * 4) : 0);
+    if ((st = ctx->dev_alloc(desc_bytes, &b->desc))) return fail(st);
+    char *const desc = (char *)b->desc;
+    b->fill_dev = (FillWork *)desc;
+    b->mesh_dev = (MeshWork *)(desc + off_mesh);
+    if (!b->uniform) b->order_dev = (int32_t *)(desc + off_order);
+    b->counts = (uint32_t *)(desc + off_ctl);
+    b->bases = (uint64_t *)(desc + off_bases);
+    b->total = (uint64_t *)(desc + off_total);
     b->overflow = (uint32_t *)(b->total + 1);  // [0] arena overflow, [1] schedule error
-    b->emit_order = (int32_t *)((char *)b->total + 256);
-    if (slabbed) {
-        b->slabs = (uint32_t *)((char *)b->emit_order + up256((size_t)b->n_items * 4));
-        VX_HIP(ctx, hipMemsetAsync(b->slabs, 0, (size_t)kSlabs * n * 4, ctx->stream));
-    }
-    VX_HIP(ctx, hipMemsetAsync(b->overflow, 0, 8, ctx->stream));
-
-    std::vector<FillWork> fw(n);
-    std::vector<MeshWork> mw(n);
-    char *store = (char *)b->store;
-    for (int i = 0; i < n; i++) {
-        const vx_batch_req &r = reqs[i];
-        const Layout L = layout_of(r.edge);
-        char *base = store + b->chunk_off[i];
-        FillWork &f = fw[i];
-        f = FillWork{};
-        f.cx = r.coord.x;
-        f.cy = r.coord.y;
-        f.cz = r.coord.z;
-        f.edge = r.edge;
-        f.terrain = r.terrain_id;
-        f.variant = fill_variant(ctx->terrains[r.terrain_id], f.cx, f.cy, f.cz, f.edge);
-        b->fill_kinds |= f.variant ? kFillFast : kFillGeneral;
-        f.ids = (uint8_t *)base;
-        f.occ = (uint32_t *)(base + L.occ);
-        f.planes = (uint32_t *)(base + L.planes);
-        f.meta = (uint32_t *)(base + L.meta);
-    }
-    for (int i = 0; i < n; i++) {
-        const vx_batch_req &r = reqs[i];
-        MeshWork &m = mw[i];
-        m = MeshWork{};
-        m.ox = r.coord.x * r.edge;
-        m.oy = r.coord.y * r.edge;
-        m.oz = r.coord.z * r.edge;
-        m.edge = r.edge;
-        m.occ = fw[i].occ;
-        m.ids = fw[i].ids;
-        m.solid_type = kBlockGrass;  // generated chunks hold only grass
-        static const int which[4] = {1, 0, 3, 2};  // facing plane of the neighbour
-        const size_t plane = (size_t)r.edge * words_per_row(r.edge);
-        for (int k = 0; k < 4; k++) {
-            const int j = r.nb[k];
-            if (j >= 0) m.nb[k] = fw[j].planes + which[k] * plane;
-            else if (j <= -2) m.nb[k] = ext[-2 - j]->planes + which[k] * plane;
-            else m.nb[k] = nullptr;
-        }
-    }
-    // fused form: every in-batch neighbour must be the adjacent chunk with the
+    b->emit_order = (int32_t *)(desc + off_emit);
+    if (slabbed) b->slabs = (uint32_t *)(desc + off_slabs);
     // The fill counts the faces itself when every chunk has its own
     // workgroup and no neighbour inside the batch (each neighbour plane is
     // absent or resident before the run): the staged form then has no
@@ -541,12 +580,46 @@ extern "C" int vx_batch_create_ext(vx_ctx *ctx, const vx_batch_req *reqs, int32_
     for (int i = 0; i < n && b->fill_counts; i++)
         for (int k = 0; k < 4; k++)
             if (reqs[i].nb[k] >= 0) b->fill_counts = false;
-    if (b->fill_counts)
-        for (int i = 0; i < n; i++) {
-            for (int k = 0; k < 4; k++) fw[i].cnb[k] = mw[i].nb[k];
-            fw[i].count_out = b->counts + i;
-            fw[i].slab_out = b->slabs ? b->slabs + (size_t)kSlabs * i : nullptr;
+    {
+        // assembled in the context's pinned staging where it fits (the copy is
+        // then asynchronous), else in pageable memory
+        std::vector<char> pageable;
+        char *up = ctx->staging(desc_bytes);
+        if (!up) {
+            pageable.resize(desc_bytes);
+            up = pageable.data();
         }
+        describe(b, (FillWork *)up, (MeshWork *)(up + off_mesh));
+        for (int i = 0; i < n; i++)
+            b->fill_kinds |= ((FillWork *)up)[i].variant ? kFillFast : kFillGeneral;
+        if (!b->uniform) {
+            int32_t *order = (int32_t *)(up + off_order);
+            std::iota(order, order + n, 0);
+            std::stable_sort(order, order + n, [&](int a, int c) { return cost[a] > cost[c]; });
+            if (!is_schedule(order, n)) {
+                ctx->last_error = "batch fill schedule is not a permutation of the requests";
+                return fail(VX_ERR_DEVICE);
+            }
+        }
+        memset(up + off_ctl, 0, off_emit - off_ctl);
+        if (slabbed) memset(up + off_slabs, 0, desc_bytes - off_slabs);
+        // the scan rewrites the emission order every run; start from a valid
+        // one regardless (chunk indices, or every emit item's code chunk << 2
+        // | slab)
+        int32_t *emit = (int32_t *)(up + off_emit);
+        for (int i = 0; i < n; i++) {
+            if (!b->slabs) *emit++ = i;
+            else
+                for (int q = 0; q < (reqs[i].edge == 64 ? kSlabs : 1); q++) *emit++ = i << 2 | q;
+        }
+        hipError_t e = hipMemcpyAsync(b->desc, up, desc_bytes, hipMemcpyHostToDevice, ctx->stream);
+        if (e == hipSuccess)
+            e = pageable.empty() ? ctx->staging_queued() : hipStreamSynchronize(ctx->stream);
+        if (e != hipSuccess) {
+            ctx->set_error(e, "batch descriptors");
+            return fail(VX_ERR_DEVICE);
+        }
+    }
     // split form (edges up to 32): the first half [0, m) and the later chunks
     // it borders, up to m2, are filled first; a batch whose fill counts needs
     // whole-chunk fills (kFillGrid chunks or more) in both fill launches
@@ -559,12 +632,8 @@ extern "C" int vx_batch_create_ext(vx_ctx *ctx, const vx_batch_req *reqs, int32_
         b->split_m2 = m2;
         b->split_ok = !b->fill_counts || (m2 >= kFillGrid && n - m2 >= kFillGrid);
         b->split_total = (uint64_t *)((char *)b->total + 16);  // in the control block's spare words
-        for (int k = 0; k < 3 && b->split_ok; k++)
-            if (hipEventCreateWithFlags(&b->split_ev[k], hipEventDisableTiming) != hipSuccess) {
-                (void)hipGetLastError();
-                b->split_ok = false;
-            }
     }
+    // fused form: every in-batch neighbour must be the adjacent chunk with the
     // same terrain, so its facing plane can be recomputed from noise; the
     // reference-rule terrain is generated by the fill kernels only
     static const int ddx[4] = {-1, 1, 0, 0}, ddz[4] = {0, 0, -1, 1};
@@ -584,19 +653,7 @@ extern "C" int vx_batch_create_ext(vx_ctx *ctx, const vx_batch_req *reqs, int32_
         }
     // pipelined form: edges up to 32 (its LDS holds four workgroups per CU)
     b->pipe_ok = b->fused_ok && b->max_edge <= 32;
-    std::vector<FusedWork> fu;
     if (b->fused_ok) {
-        fu.resize(n);
-        for (int i = 0; i < n; i++) {
-            fu[i].f = fw[i];
-            fu[i].m = mw[i];
-            for (int k = 0; k < 4; k++) {
-                fu[i].halo[k] = reqs[i].nb[k] >= 0    ? kHaloRecompute
-                                : reqs[i].nb[k] <= -2 ? kHaloResident
-                                                      : kHaloAbsent;
-                fu[i].nbi[k] = reqs[i].nb[k] >= 0 ? reqs[i].nb[k] : -1;
-            }
-        }
         if ((st = ctx->dev_alloc((size_t)n * sizeof(FusedWork), (void **)&b->fused_dev)))
             return fail(st);
         // ticket | error | ... | status[n] (u64) | filled[n] (u32)
@@ -613,42 +670,7 @@ extern "C" int vx_batch_create_ext(vx_ctx *ctx, const vx_batch_req *reqs, int32_
         b->fctl_ptrs.bases = b->bases;
         b->fctl_ptrs.total = b->total;
         b->fctl_ptrs.overflow = b->overflow;
-        VX_HIP(ctx, hipMemcpyAsync(b->fused_dev, fu.data(), fu.size() * sizeof(FusedWork),
-                                   hipMemcpyHostToDevice, ctx->stream));
     }
-    {
-        // the scan rewrites it every run; start from a valid order regardless
-        // (chunk indices, or every emit item's code chunk << 2 | slab)
-        std::vector<int32_t> iota_order;
-        iota_order.reserve(b->n_items);
-        for (int i = 0; i < n; i++) {
-            if (!b->slabs) iota_order.push_back(i);
-            else
-                for (int q = 0; q < (reqs[i].edge == 64 ? kSlabs : 1); q++)
-                    iota_order.push_back(i << 2 | q);
-        }
-        VX_HIP(ctx, hipMemcpyAsync(b->emit_order, iota_order.data(), (size_t)b->n_items * 4,
-                                   hipMemcpyHostToDevice, ctx->stream));
-        VX_HIP(ctx, hipStreamSynchronize(ctx->stream));  // pageable source
-    }
-    VX_HIP(ctx, hipMemcpyAsync(b->fill_dev, fw.data(), fw.size() * sizeof(FillWork),
-                               hipMemcpyHostToDevice, ctx->stream));
-    VX_HIP(ctx, hipMemcpyAsync(b->mesh_dev, mw.data(), mw.size() * sizeof(MeshWork),
-                               hipMemcpyHostToDevice, ctx->stream));
-    if (!b->uniform) {
-        std::vector<int32_t> order(n);
-        std::iota(order.begin(), order.end(), 0);
-        std::stable_sort(order.begin(), order.end(),
-                         [&](int a, int c) { return cost[a] > cost[c]; });
-        if (!is_schedule(order.data(), n)) {
-            ctx->last_error = "batch fill schedule is not a permutation of the requests";
-            return fail(VX_ERR_DEVICE);
-        }
-        if ((st = ctx->dev_alloc((size_t)n * 4, (void **)&b->order_dev))) return fail(st);
-        VX_HIP(ctx, hipMemcpyAsync(b->order_dev, order.data(), (size_t)n * 4,
-                                   hipMemcpyHostToDevice, ctx->stream));
-    }
-    VX_HIP(ctx, hipStreamSynchronize(ctx->stream));  // host vectors are pageable
     uint64_t cap = face_capacity;
     if (cap == 0) {
         for (int i = 0; i < n; i++) cap += 4ull * reqs[i].edge * reqs[i].edge;
@@ -738,11 +760,17 @@ extern "C" int vx_batch_get_mode(vx_batch *b, int32_t *mode) {
 extern "C" int vx_batch_run(vx_ctx *ctx, vx_batch *b) {
     if (!ctx || !b || b->ctx != ctx) return VX_ERR_INVALID;
     std::lock_guard<std::recursive_mutex> g(ctx->mu);
-    if (!b->graph_exec) {
-        int st = capture_graph(b);
-        if (st) return st;
+    if (!b->graph_exec && !b->launched) {
+        // the first run launches the kernels themselves; the graph is captured
+        // while the GPU works on them (vx_batch_wait), or by the second run
+        if (int st = ready_form(b)) return st;
+        VX_HIP(ctx, enqueue_all(b));
+    } else {
+        if (!b->graph_exec)
+            if (int st = capture_graph(b)) return st;
+        VX_HIP(ctx, hipGraphLaunch(b->graph_exec, ctx->stream));
     }
-    VX_HIP(ctx, hipGraphLaunch(b->graph_exec, ctx->stream));
+    b->launched = true;
     b->ran = true;
     b->results = false;
     return VX_OK;
@@ -773,8 +801,10 @@ extern "C" int vx_batch_wait(vx_ctx *ctx, vx_batch *b, uint64_t *total_faces) {
     if (!ctx || !b || b->ctx != ctx) return VX_ERR_INVALID;
     std::lock_guard<std::recursive_mutex> g(ctx->mu);
     if (!b->ran) return VX_ERR_NOT_READY;
-    VX_HIP(ctx, hipMemcpyAsync(ctx->pinned, b->total, 8, hipMemcpyDeviceToHost, ctx->stream));
-    VX_HIP(ctx, hipMemcpyAsync(ctx->pinned + 8, b->overflow, 8, hipMemcpyDeviceToHost, ctx->stream));
+    // total | overflow, schedule error: 16 contiguous bytes
+    VX_HIP(ctx, hipMemcpyAsync(ctx->pinned, b->total, 16, hipMemcpyDeviceToHost, ctx->stream));
+    if (!b->graph_exec && b->launched)
+        if (int st = capture_graph(b)) return st;  // beside the first run
     VX_HIP(ctx, hipStreamSynchronize(ctx->stream));
     uint32_t sched_err;
     memcpy(&sched_err, ctx->pinned + 12, 4);
@@ -1112,6 +1142,7 @@ extern "C" int vx_batch_profile(vx_ctx *ctx, vx_batch *b, int32_t reps, float ms
     // one-launch forms and the split form: the whole run as one figure
     const bool whole = use_fused(b) || form_of(b) == VX_BATCH_SPLIT;
     for (int r = 0; r < reps && !st && whole; r++) {
+        if ((st = ready_form(b))) break;
         hipError_t e = hipEventRecord(ev[0], ctx->stream);
         if (e == hipSuccess) e = enqueue_all(b);
         if (e == hipSuccess) e = hipEventRecord(ev[1], ctx->stream);

@@ -87,6 +87,16 @@ struct vx_ctx {
     int32_t draw_counts_cap = 0;
     uint32_t *draw_scratch = nullptr; // this device's static draw-list scratch
 
+    char *stage = nullptr;            // pinned staging of asynchronous uploads (made on first use)
+    hipEvent_t stage_ev = nullptr;    // the last upload from it has been consumed
+
+    // The staging buffer for an upload of `bytes`, once the previous upload from
+    // it is through, or null when it does not fit (or cannot be had): the
+    // caller then uploads from pageable memory.  staging_queued() follows the
+    // copy on `stream`.
+    char *staging(size_t bytes);
+    hipError_t staging_queued();
+
     void set_error(hipError_t e, const char *what);
     int dev_alloc(size_t n, void **out);
     void dev_free(void *p);
@@ -141,9 +151,8 @@ struct vx_batch {
     vx::MeshWork *mesh_dev = nullptr;
     uint32_t fill_kinds = 0;        // kFillFast / kFillGeneral: the chunks' fill kernels
     int32_t *order_dev = nullptr;   // longest-first schedule (null when uniform)
+    void *desc = nullptr;           // block of the descriptors, the schedules and the control words
     int32_t *coords_dev = nullptr;  // chunk coordinates (draw lists), made on first use
-    void *ctl = nullptr;            // counts[n] | bases[n] | total | overflow | emit_order[n_items]
-                                    // | slabs[kSlabs * n] (batches holding 64^3 chunks)
     int32_t *emit_order = nullptr;  // emission order written by the scan (largest first)
     int32_t n_items = 0;            // emit items: n, or with slabs kSlabs per 64^3 chunk
     uint32_t *slabs = nullptr;      // per-slab face counts of 64^3 chunks (null when none)
@@ -173,10 +182,12 @@ struct vx_batch {
     hipEvent_t split_ev[3] = {};    // fill, scan of the first half; the second half's end
     int32_t pipe_lag = 0;           // farthest in-batch neighbour index ahead of a chunk
     vx::FusedWork *fused_dev = nullptr;
+    bool fused_made = false;        // fused_dev has been written
     void *fctl = nullptr;           // ticket | error | status[n]
     vx::FusedCtl fctl_ptrs{};
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
+    bool launched = false;          // some run has been queued (the first without a graph)
     bool ran = false;
     bool results = false;           // host copies below are current
     uint64_t h_total = 0;

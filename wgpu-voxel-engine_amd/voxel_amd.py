@@ -521,6 +521,12 @@ class Frustum:
                 b.free()
 
 
+# BatchReq as an array of records
+_REQ_DTYPE = np.dtype([("coord", "<i4", (3,)), ("edge", "<i4"), ("terrain_id", "<i4"),
+                       ("nb", "<i4", (4,))])
+assert _REQ_DTYPE.itemsize == C.sizeof(BatchReq)
+
+
 class Batch:
     """Many Chunk::new + create_mesh requests as one graph-replayed launch
     sequence (fill -> count -> scan -> emit)."""
@@ -533,17 +539,12 @@ class Batch:
         tids = np.broadcast_to(np.asarray(terrain_ids, np.int32), (n,))
         nb = (np.full((n, 4), -1, np.int32) if neighbours is None
               else np.asarray(neighbours, np.int32).reshape(n, 4))
-        reqs = (BatchReq * n)()
-        for i in range(n):
-            reqs[i].coord = Coord(*map(int, coords[i]))
-            reqs[i].edge = int(edges[i])
-            reqs[i].terrain_id = int(tids[i])
-            for k in range(4):
-                reqs[i].nb[k] = int(nb[i, k])
+        reqs = np.empty(n, _REQ_DTYPE)
+        reqs["coord"], reqs["edge"], reqs["terrain_id"], reqs["nb"] = coords, edges, tids, nb
         h = P()
         ext = list(ext or [])
         ext_arr = (P * max(1, len(ext)))(*[c.h for c in ext])
-        ctx.check(ctx.L.vx_batch_create_ext(ctx.h, C.cast(reqs, P), n, C.cast(ext_arr, P), len(ext),
+        ctx.check(ctx.L.vx_batch_create_ext(ctx.h, _p(reqs), n, C.cast(ext_arr, P), len(ext),
                                             formats, face_capacity, C.byref(h)),
                   "vx_batch_create_ext")
         self.ctx, self.h, self.n, self.formats = ctx, h, n, formats
