@@ -167,17 +167,22 @@ hipError_t enqueue_fill(vx_batch *b) {
     return launch_fill(b->fill_dev, b->order_dev, b->n, b->max_edge, ctx->terrains_dev,
                        ctx->lut_dev, b->overflow + 1, fill_split_of(b), b->fill_kinds, ctx->stream);
 }
-hipError_t enqueue_count(vx_batch *b) {
-    return launch_count(b->mesh_dev, b->n, b->max_edge, b->counts, b->slabs, b->ctx->stream);
+// Batches of few chunks have no scan: the emit sums the counts itself.
+bool self_scan(const vx_batch *b) { return b->n <= kSelfScan && !b->fill_counts; }
+
+hipError_t enqueue_count(vx_batch *b, const CullJob &cull = CullJob{}) {
+    return launch_count(b->mesh_dev, b->n, b->max_edge, b->counts, b->slabs,
+                        self_scan(b) ? b->overflow : nullptr, cull, b->ctx->stream);
 }
 hipError_t enqueue_scan(vx_batch *b) {
     return launch_scan(b->counts, b->n, b->slabs ? b->mesh_dev : nullptr, b->bases, b->total,
                        b->overflow, b->emit_order, b->ctx->stream);
 }
 hipError_t enqueue_emit(vx_batch *b) {
-    return launch_emit(b->mesh_dev, b->emit_order, b->n, b->n_items, b->max_edge, b->bases,
-                       b->counts, b->slabs, b->out, b->ctx->tables_dev, b->overflow,
-                       emit_split_of(b), b->ctx->stream);
+    const bool self = self_scan(b);
+    return launch_emit(b->mesh_dev, self ? nullptr : b->emit_order, b->n, b->n_items, b->max_edge,
+                       b->bases, b->counts, b->slabs, b->out, b->ctx->tables_dev, b->overflow,
+                       emit_split_of(b), self ? b->total : nullptr, b->ctx->stream);
 }
 
 // The form a run takes.  VX_BATCH_AUTO runs the staged form unless the
@@ -247,21 +252,22 @@ hipError_t enqueue_split(vx_batch *b) {
     // first half on the second stream
     if (e == hipSuccess) e = hipStreamWaitEvent(s1, b->split_ev[0], 0);
     if (e == hipSuccess && !b->fill_counts)
-        e = launch_count(b->mesh_dev, m, b->max_edge, b->counts, nullptr, s1);
+        e = launch_count(b->mesh_dev, m, b->max_edge, b->counts, nullptr, nullptr, CullJob{}, s1);
     if (e == hipSuccess)
         e = launch_scan(b->counts, m, nullptr, b->bases, b->split_total, b->overflow,
                         b->emit_order, s1);
     if (e == hipSuccess) e = hipEventRecord(b->split_ev[1], s1);
     if (e == hipSuccess)
         e = launch_emit(b->mesh_dev, b->emit_order, m, m, b->max_edge, b->bases, b->counts,
-                        nullptr, b->out, ctx->tables_dev, b->overflow, es, s1);
+                        nullptr, b->out, ctx->tables_dev, b->overflow, es, nullptr, s1);
     if (e == hipSuccess) e = hipEventRecord(b->split_ev[2], s1);
     // second half on the context stream
     if (e == hipSuccess)
         e = launch_fill(b->fill_dev + m2, nullptr, n - m2, b->max_edge, ctx->terrains_dev,
                         ctx->lut_dev, b->overflow + 1, fs, b->fill_kinds, s0);
     if (e == hipSuccess && !b->fill_counts)
-        e = launch_count(b->mesh_dev + m, n - m, b->max_edge, b->counts + m, nullptr, s0);
+        e = launch_count(b->mesh_dev + m, n - m, b->max_edge, b->counts + m, nullptr, nullptr,
+                         CullJob{}, s0);
     if (e == hipSuccess) e = hipStreamWaitEvent(s0, b->split_ev[1], 0);
     // the overflow word was cleared by the first half's scan: not again here
     if (e == hipSuccess)
@@ -270,7 +276,7 @@ hipError_t enqueue_split(vx_batch *b) {
     if (e == hipSuccess)
         e = launch_emit(b->mesh_dev + m, b->emit_order + m, n - m, n - m, b->max_edge,
                         b->bases + m, b->counts + m, nullptr, b->out, ctx->tables_dev,
-                        b->overflow, es, s0);
+                        b->overflow, es, nullptr, s0);
     if (e == hipSuccess) e = hipStreamWaitEvent(s0, b->split_ev[2], 0);
     return e;
 }
@@ -278,10 +284,11 @@ hipError_t enqueue_split(vx_batch *b) {
 hipError_t enqueue_all(vx_batch *b) {
     if (use_fused(b)) return enqueue_fused(b);
     if (form_of(b) == VX_BATCH_SPLIT) return enqueue_split(b);
-    hipError_t e = launch_cull(b->cull, b->ctx->stream);
+    // the cull runs beside the count, or alone when the fill counts
+    hipError_t e = b->fill_counts ? launch_cull(b->cull, b->ctx->stream) : hipSuccess;
     if (e == hipSuccess) e = enqueue_fill(b);
-    if (e == hipSuccess && !b->fill_counts) e = enqueue_count(b);
-    if (e == hipSuccess) e = enqueue_scan(b);
+    if (e == hipSuccess && !b->fill_counts) e = enqueue_count(b, b->cull);
+    if (e == hipSuccess && !self_scan(b)) e = enqueue_scan(b);
     if (e == hipSuccess) e = enqueue_emit(b);
     return e;
 }
@@ -391,8 +398,6 @@ void free_batch(vx_batch *b) {
     for (vx_chunk *c : b->ext)
         if (c->refs.fetch_sub(1) == 1) vx_chunk_destroy_locked(c);
     ctx->dev_free(b->planes_dev);
-    if (b->planes_pin) (void)hipHostFree(b->planes_pin);
-    if (b->planes_ev) (void)hipEventDestroy(b->planes_ev);
     ctx->dev_free(b->desc);
     ctx->dev_free(b->coords_dev);
     ctx->dev_free(b->arena);
@@ -786,12 +791,12 @@ extern "C" int vx_batch_run_per_chunk(vx_ctx *ctx, vx_batch *b) {
     auto slabs_of = [&](int i) { return b->slabs ? b->slabs + (size_t)kSlabs * i : nullptr; };
     for (int i = 0; i < n; i++)
         VX_HIP(ctx, launch_count(b->mesh_dev + i, 1, b->reqs[i].edge, b->counts + i, slabs_of(i),
-                                 ctx->stream));
+                                 nullptr, CullJob{}, ctx->stream));
     VX_HIP(ctx, enqueue_scan(b));
     for (int i = 0; i < n; i++)
         VX_HIP(ctx, launch_emit(b->mesh_dev + i, nullptr, 1, 0, b->reqs[i].edge, b->bases + i,
                                 b->counts + i, slabs_of(i), b->out, ctx->tables_dev, b->overflow,
-                                0, ctx->stream));
+                                0, nullptr, ctx->stream));
     b->ran = true;
     b->results = false;
     return VX_OK;
@@ -841,9 +846,10 @@ extern "C" int vx_batch_wait(vx_ctx *ctx, vx_batch *b, uint64_t *total_faces) {
             b->results = false;
             return st;
         }
-        // a persistent form writes no slab counts: count again first
-        if (b->slabs) VX_HIP(ctx, enqueue_count(b));
-        VX_HIP(ctx, enqueue_scan(b));
+        // a persistent form writes no slab counts: count again first; without
+        // a scan it is the count that clears the overflow word
+        if (b->slabs || self_scan(b)) VX_HIP(ctx, enqueue_count(b));
+        if (!self_scan(b)) VX_HIP(ctx, enqueue_scan(b));
         VX_HIP(ctx, enqueue_emit(b));
         VX_HIP(ctx, hipMemcpyAsync(ctx->pinned + 8, b->overflow, 8, hipMemcpyDeviceToHost,
                                    ctx->stream));
@@ -951,15 +957,10 @@ extern "C" int vx_batch_set_cull(vx_batch *b, const vx_frustum *f, const int32_t
     if (!b->planes_dev) {
         int st = ctx->dev_alloc(sizeof(f->planes), (void **)&b->planes_dev);
         if (st) return st;
-        VX_HIP(ctx, hipHostMalloc((void **)&b->planes_pin, sizeof(f->planes), hipHostMallocDefault));
-        VX_HIP(ctx, hipEventCreateWithFlags(&b->planes_ev, hipEventDisableTiming));
-    } else {
-        VX_HIP(ctx, hipEventSynchronize(b->planes_ev));  // previous frame's copy has run
     }
-    memcpy(b->planes_pin, f->planes, sizeof(f->planes));
-    VX_HIP(ctx, hipMemcpyAsync(b->planes_dev, b->planes_pin, sizeof(f->planes),
-                               hipMemcpyHostToDevice, ctx->stream));
-    VX_HIP(ctx, hipEventRecord(b->planes_ev, ctx->stream));
+    Planes P;
+    memcpy(P.p, f->planes, sizeof(P.p));
+    VX_HIP(ctx, launch_set_planes(P, b->planes_dev, ctx->stream));
     CullJob job{b->planes_dev, coords_dev, mask_dev, n, edge};
     if (job.coords != b->cull.coords || job.mask != b->cull.mask || job.n != b->cull.n ||
         job.edge != b->cull.edge) {
@@ -1162,7 +1163,7 @@ extern "C" int vx_batch_profile(vx_ctx *ctx, vx_batch *b, int32_t reps, float ms
         if (e == hipSuccess) e = hipEventRecord(ev[1], ctx->stream);
         if (e == hipSuccess && !b->fill_counts) e = enqueue_count(b);
         if (e == hipSuccess) e = hipEventRecord(ev[2], ctx->stream);
-        if (e == hipSuccess) e = enqueue_scan(b);
+        if (e == hipSuccess && !self_scan(b)) e = enqueue_scan(b);
         if (e == hipSuccess) e = hipEventRecord(ev[3], ctx->stream);
         if (e == hipSuccess) e = enqueue_emit(b);
         if (e == hipSuccess) e = hipEventRecord(ev[4], ctx->stream);

@@ -145,8 +145,6 @@ struct vx_batch {
     std::vector<vx_chunk *> ext;    // resident neighbours named by requests (retained)
     vx::CullJob cull{};             // optional frustum job run with the batch
     float *planes_dev = nullptr;    // device copy of the cull planes
-    float *planes_pin = nullptr;    // pinned staging for per-frame planes
-    hipEvent_t planes_ev = nullptr; // the staging copy has been consumed
     vx::FillWork *fill_dev = nullptr;
     vx::MeshWork *mesh_dev = nullptr;
     uint32_t fill_kinds = 0;        // kFillFast / kFillGeneral: the chunks' fill kernels

@@ -217,8 +217,10 @@ inline bool fill_whole_chunks(int32_t n) { return n >= kFillGrid; }
 // (the batch's mesh work) the scan's order lists item codes chunk << 2 |
 // slab, at most kSlabs * n of them; launch_emit takes their number.
 constexpr int kSlabs = 4;
+// clear (may be null): a word the count sets to 0 (the overflow word of an
+// emit that follows without a scan).  cull: a frustum job run beside it.
 hipError_t launch_count(const MeshWork *work, int32_t n, int32_t max_edge, uint32_t *counts,
-                        uint32_t *slabs, hipStream_t s);
+                        uint32_t *slabs, uint32_t *clear, const CullJob &cull, hipStream_t s);
 // base_in (device, may be null): faces before these chunks, added to every
 // base and to the total (the second half of a split batch).
 hipError_t launch_scan(const uint32_t *counts, int32_t n, const MeshWork *items, uint64_t *bases,
@@ -233,11 +235,14 @@ hipError_t launch_pack_one(const FillWork &w, uint32_t solid_type, hipStream_t s
 hipError_t launch_count_one(const MeshWork &w, uint32_t *count, uint32_t *slabs, hipStream_t s);
 hipError_t launch_emit_one(const MeshWork &w, uint32_t faces, const uint32_t *slabs, MeshOut out,
                            const MeshTables *tables, uint32_t *overflow, hipStream_t s);
-// parts_hint: emit_parts_for's hint.
+// parts_hint: emit_parts_for's hint.  total (null: bases come from the scan):
+// the emit sums the counts before each chunk itself, in batch order (order =
+// null), and writes bases and *total; for batches of at most kSelfScan chunks.
 hipError_t launch_emit(const MeshWork *work, const int32_t *order, int32_t n, int32_t n_items,
-                       int32_t max_edge, const uint64_t *bases, const uint32_t *counts,
+                       int32_t max_edge, uint64_t *bases, const uint32_t *counts,
                        const uint32_t *slabs, MeshOut out, const MeshTables *tables,
-                       uint32_t *overflow, int32_t parts_hint, hipStream_t s);
+                       uint32_t *overflow, int32_t parts_hint, uint64_t *total, hipStream_t s);
+constexpr int kSelfScan = 512;
 // Emit items of a batch: its chunks, or for batches that hold 64^3 chunks
 // kSlabs per 64^3 chunk and one per other chunk.
 inline int32_t emit_items_of(int32_t n, int32_t n_items, int32_t max_edge) {
@@ -259,6 +264,7 @@ hipError_t launch_pipe(const FusedWork *work, int32_t n, int32_t max_edge, int32
                        FusedCtl ctl, MeshOut out, const CullJob &cull, int32_t grid, int32_t ratio,
                        hipStream_t s);
 hipError_t launch_cull(const CullJob &job, hipStream_t s);
+hipError_t launch_set_planes(const Planes &planes, float *dst, hipStream_t s);
 hipError_t launch_copy(void *dst, const void *src, uint64_t bytes, hipStream_t s);
 hipError_t launch_frustum(const Planes &planes, const int32_t *coords, int32_t n, int32_t edge,
                           uint8_t *mask, hipStream_t s);

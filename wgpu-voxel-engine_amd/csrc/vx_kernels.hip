@@ -1602,6 +1602,40 @@ __device__ __forceinline__ void face_masks(const SH &S, int y, int z,
     }
 }
 
+// Frustum test of chunk AABBs (frustum_culling.rs:16-40; dist = ((a*x + b*y) + c*z) + d, NaN passes).
+__device__ __forceinline__ uint8_t aabb_visible(const float *pl, int cx, int cy, int cz, int edge) {
+    // exact 64-bit products rounded to f32: equal to the 32-bit product
+    // wherever that does not overflow, defined for every coordinate
+    const float px = (float)((long long)cx * edge), py = (float)((long long)cy * edge),
+                pz = (float)((long long)cz * edge);
+    const float e = (float)edge;
+    const float xs[2] = {px, px + e}, ys[2] = {py, py + e}, zs[2] = {pz, pz + e};
+    uint32_t any = 0;
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        const float x = xs[c & 1], y = ys[(c >> 2) & 1], z = zs[(c >> 1) & 1];
+        uint32_t inside = 1;
+#pragma unroll
+        for (int k = 0; k < 6; k++) {
+            const float dist = pl[4 * k] * x + pl[4 * k + 1] * y + pl[4 * k + 2] * z + pl[4 * k + 3];
+            inside &= !(dist < 0.0f);
+        }
+        any |= inside;
+    }
+    return (uint8_t)any;
+}
+
+// Slice `block` of `blocks` of a cull job (in the fused launches every
+// workgroup takes one before its chunk tickets).
+__device__ __forceinline__ void cull_slice(const CullJob &job, int block, int blocks) {
+    float pl[24];
+#pragma unroll
+    for (int i = 0; i < 24; i++) pl[i] = job.planes[i];
+    for (int i = block * kBlock + threadIdx.x; i < job.n; i += blocks * kBlock)
+        job.mask[i] = aabb_visible(pl, job.coords[3 * i], job.coords[3 * i + 1],
+                                   job.coords[3 * i + 2], job.edge);
+}
+
 // Loads slab `ylo / kSlabLayers` of a 64^3 chunk (rows are u32 pairs, low
 // word first) with its halo layers and neighbour-plane rows.
 __device__ __forceinline__ void load_slab(const MeshWork &w, SlabShared &S, int ylo) {
@@ -1701,11 +1735,20 @@ __device__ __forceinline__ void count_item(const MeshWork &w, CountShared<MAXN> 
     }
 }
 
+// One workgroup per chunk; workgroups from n on cull (a frustum job beside the
+// batch: neither kernel alone fills the GPU).  `clear` (may be null): the
+// arena-overflow word, for an emit that takes its bases itself.
 template <int MAXN>
 __global__ void __launch_bounds__(kBlock) count_kernel(const MeshWork *__restrict__ work,
                                                        uint32_t *__restrict__ counts,
-                                                       uint32_t *__restrict__ slabs) {
+                                                       uint32_t *__restrict__ slabs, int32_t n,
+                                                       uint32_t *__restrict__ clear, CullJob cull) {
     __shared__ CountShared<MAXN> S;
+    if ((int)blockIdx.x >= n) {
+        cull_slice(cull, (int)blockIdx.x - n, (int)gridDim.x - n);
+        return;
+    }
+    if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0u;
     count_item<MAXN>(work[blockIdx.x], S, counts + blockIdx.x,
                      slabs ? slabs + (size_t)kSlabs * blockIdx.x : nullptr);
 }
@@ -2130,21 +2173,39 @@ __device__ __forceinline__ void emit_item(const MeshWork &w, uint64_t base, uint
     }
 }
 
+// First face of chunk `item` from the counts before it, summed by the
+// workgroup itself: small batches need no scan kernel (4 to 5 us with its
+// launch, against about 1 us here).  The writer (one workgroup per chunk) also
+// leaves bases[item] and, for the last chunk, the batch's total.
+__device__ __forceinline__ uint64_t self_base(const uint32_t *counts, int item, int n,
+                                              uint64_t *bases, uint64_t *total, uint32_t *red,
+                                              bool writer) {
+    uint32_t c = 0;
+    for (int j = threadIdx.x; j < item; j += kBlock) c += counts[j];
+    const uint64_t base = block_sum(c, red);
+    if (writer && threadIdx.x == 0) {
+        bases[item] = base;
+        if (item == n - 1) *total = base + counts[item];
+    }
+    return base;
+}
+
 // Register cap: five waves per SIMD (96 VGPRs), matching the five
 // workgroups per CU that the 29 KB of LDS allows at MAXN = 32, so more
 // workgroups overlap their descriptor and store phases.
 template <int MAXN, int BLOCK>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8)))
 emit_kernel(const MeshWork *__restrict__ work, const int32_t *__restrict__ order,
-            const uint64_t *__restrict__ bases, const uint32_t *__restrict__ counts, MeshOut out,
+            uint64_t *__restrict__ bases, const uint32_t *__restrict__ counts, MeshOut out,
             const MeshTables *__restrict__ tables, uint32_t *__restrict__ overflow, int parts,
-            int32_t n) {
+            int32_t n, uint64_t *__restrict__ total) {
     __shared__ MeshShared<MAXN, BLOCK> S;
     const int k = (int)blockIdx.x / parts, part = (int)blockIdx.x - k * parts;
     const int item = order ? order[k] : k;
     if (!order_entry_ok(item, n, overflow + 1)) return;
-    emit_item<MAXN, BLOCK>(work[item], bases[item], counts[item], out, tables, overflow, S, part,
-                           parts);
+    const uint64_t base =
+        total ? self_base(counts, item, n, bases, total, S.red, part == 0) : bases[item];
+    emit_item<MAXN, BLOCK>(work[item], base, counts[item], out, tables, overflow, S, part, parts);
 }
 
 // One slab of a 64^3 chunk: its faces start `off` faces into the chunk,
@@ -2181,24 +2242,28 @@ union EmitShared64 {
 
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
 emit_slab_kernel(const MeshWork *__restrict__ work, const int32_t *__restrict__ order,
-                 const uint64_t *__restrict__ bases, const uint32_t *__restrict__ counts,
+                 uint64_t *__restrict__ bases, const uint32_t *__restrict__ counts,
                  const uint32_t *__restrict__ slabs, MeshOut out,
                  const MeshTables *__restrict__ tables, uint32_t *__restrict__ overflow, int parts,
-                 int32_t n) {
+                 int32_t n, uint64_t *__restrict__ total) {
     __shared__ EmitShared64 S;
     const int k = (int)blockIdx.x / parts, part = (int)blockIdx.x - k * parts;
     const int code = order ? order[k] : k;
     const int item = code >> 2, slab = code & 3;
     if (!order_entry_ok(item, n, overflow + 1)) return;
     const MeshWork &w = work[item];
+    if (w.edge != 64 && slab > 0) {
+        if (order && threadIdx.x == 0) atomicOr(overflow + 1, 1u);
+        return;
+    }
+    const uint64_t base = total ? self_base(counts, item, n, bases, total, S.slab.red,
+                                            slab == 0 && part == 0)
+                                : bases[item];
     if (w.edge == 64) {
-        emit_slab_item(w, bases[item], slabs + (size_t)kSlabs * item, slab, out, tables, overflow,
+        emit_slab_item(w, base, slabs + (size_t)kSlabs * item, slab, out, tables, overflow,
                        S.slab, part, parts);
-    } else if (slab == 0) {
-        emit_item<32, kBlock>(w, bases[item], counts[item], out, tables, overflow, S.small, part,
-                              parts);
-    } else if (order && threadIdx.x == 0) {
-        atomicOr(overflow + 1, 1u);
+    } else {
+        emit_item<32, kBlock>(w, base, counts[item], out, tables, overflow, S.small, part, parts);
     }
 }
 
@@ -2360,40 +2425,6 @@ __device__ void fused_chunk(const FusedWork &W, const TerrainDev &T, int t, int 
     __syncthreads();
 }
 
-// Frustum test of resident chunk AABBs folded into the fused launch: every
-// workgroup culls a grid-stride slice before it takes chunk tickets
-// (frustum_culling.rs:16-40; dist = ((a*x + b*y) + c*z) + d, NaN passes).
-__device__ __forceinline__ uint8_t aabb_visible(const float *pl, int cx, int cy, int cz, int edge) {
-    // exact 64-bit products rounded to f32: equal to the 32-bit product
-    // wherever that does not overflow, defined for every coordinate
-    const float px = (float)((long long)cx * edge), py = (float)((long long)cy * edge),
-                pz = (float)((long long)cz * edge);
-    const float e = (float)edge;
-    const float xs[2] = {px, px + e}, ys[2] = {py, py + e}, zs[2] = {pz, pz + e};
-    uint32_t any = 0;
-#pragma unroll
-    for (int c = 0; c < 8; c++) {
-        const float x = xs[c & 1], y = ys[(c >> 2) & 1], z = zs[(c >> 1) & 1];
-        uint32_t inside = 1;
-#pragma unroll
-        for (int k = 0; k < 6; k++) {
-            const float dist = pl[4 * k] * x + pl[4 * k + 1] * y + pl[4 * k + 2] * z + pl[4 * k + 3];
-            inside &= !(dist < 0.0f);
-        }
-        any |= inside;
-    }
-    return (uint8_t)any;
-}
-
-__device__ __forceinline__ void cull_slice(const CullJob &job) {
-    float pl[24];
-#pragma unroll
-    for (int i = 0; i < 24; i++) pl[i] = job.planes[i];
-    for (int i = blockIdx.x * kBlock + threadIdx.x; i < job.n; i += gridDim.x * kBlock)
-        job.mask[i] = aabb_visible(pl, job.coords[3 * i], job.coords[3 * i + 1],
-                                   job.coords[3 * i + 2], job.edge);
-}
-
 // Register cap: three waves per SIMD (the noise and emit phases together
 // otherwise need ~185 VGPRs at MAXN = 32 and leave two).
 template <int MAXN>
@@ -2406,7 +2437,7 @@ fused_kernel(const FusedWork *__restrict__ work, int32_t n,
                                                        CullJob cull) {
     __shared__ FusedShared<MAXN> S;
     const int tid = threadIdx.x;
-    if (cull.n > 0) cull_slice(cull);
+    if (cull.n > 0) cull_slice(cull, (int)blockIdx.x, (int)gridDim.x);
     for (int i = tid; i < 8 * 16; i += kBlock) S.lut[i >> 4][i & 15] = lut->c[i >> 4][i & 15];
     for (int i = tid; i < 6 * 3 * 2 * 4; i += kBlock) (&S.P[0][0][0][0])[i] = (&tables->P[0][0][0][0])[i];
     for (int i = tid; i < 6 * 2 * 3 * 4; i += kBlock) (&S.Mb[0][0][0][0])[i] = (&tables->Mb[0][0][0][0])[i];
@@ -2589,7 +2620,7 @@ pipe_kernel(const FusedWork *__restrict__ work, int32_t n, int32_t lag,
     static_assert(MAXN <= 32, "64^3 chunks take the fused or staged form");
     __shared__ PipeShared<MAXN> S;
     const int tid = threadIdx.x;
-    if (cull.n > 0) cull_slice(cull);
+    if (cull.n > 0) cull_slice(cull, (int)blockIdx.x, (int)gridDim.x);
     for (int i = tid; i < 8 * 16; i += kBlock) S.lut[i >> 4][i & 15] = lut->c[i >> 4][i & 15];
     for (int i = tid; i < 6 * 3 * 2 * 4; i += kBlock) (&S.P[0][0][0][0])[i] = (&tables->P[0][0][0][0])[i];
     for (int i = tid; i < 6 * 2 * 3 * 4; i += kBlock) (&S.Mb[0][0][0][0])[i] = (&tables->Mb[0][0][0][0])[i];
@@ -2776,11 +2807,12 @@ hipError_t launch_fill(const FillWork *work, const int32_t *order, int32_t n, in
 }
 
 hipError_t launch_count(const MeshWork *work, int32_t n, int32_t max_edge, uint32_t *counts,
-                        uint32_t *slabs, hipStream_t s) {
+                        uint32_t *slabs, uint32_t *clear, const CullJob &cull, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    if (max_edge <= 16) count_kernel<16><<<n, kBlock, 0, s>>>(work, counts, nullptr);
-    else if (max_edge <= 32) count_kernel<32><<<n, kBlock, 0, s>>>(work, counts, nullptr);
-    else count_kernel<64><<<n, kBlock, 0, s>>>(work, counts, slabs);
+    const int grid = n + (cull.n > 0 ? (cull.n + kBlock - 1) / kBlock : 0);
+    if (max_edge <= 16) count_kernel<16><<<grid, kBlock, 0, s>>>(work, counts, nullptr, n, clear, cull);
+    else if (max_edge <= 32) count_kernel<32><<<grid, kBlock, 0, s>>>(work, counts, nullptr, n, clear, cull);
+    else count_kernel<64><<<grid, kBlock, 0, s>>>(work, counts, slabs, n, clear, cull);
     return hipGetLastError();
 }
 
@@ -2835,29 +2867,29 @@ hipError_t launch_emit_one(const MeshWork &w, uint32_t faces, const uint32_t *sl
 }
 
 hipError_t launch_emit(const MeshWork *work, const int32_t *order, int32_t n, int32_t n_items,
-                       int32_t max_edge, const uint64_t *bases, const uint32_t *counts,
+                       int32_t max_edge, uint64_t *bases, const uint32_t *counts,
                        const uint32_t *slabs, MeshOut out, const MeshTables *tables,
-                       uint32_t *overflow, int32_t parts_hint, hipStream_t s) {
+                       uint32_t *overflow, int32_t parts_hint, uint64_t *total, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     if (parts_hint < 0 || parts_hint > 4) return hipErrorInvalidValue;
     // items: chunks, or for batches that hold 64^3 chunks the scan's emit
     // items (kSlabs codes per chunk without an order)
     const int items = max_edge <= 32 ? n : order ? n_items : kSlabs * n;
-    if (items <= 0) return hipErrorInvalidValue;
+    if (items <= 0 || (total && order)) return hipErrorInvalidValue;
     // small batches: several workgroups per item, so the grid still covers
     // about a full GPU of workgroups and an item's tiles are emitted side by
     // side
-    const int parts = emit_parts_for(items, max_edge, parts_hint);
+    const int parts = emit_parts_for(max_edge <= 32 ? n : n_items > 0 ? n_items : items, max_edge, parts_hint);
     const int grid = items * parts;
     if (max_edge <= 16)
         emit_kernel<16, kBlock><<<grid, kBlock, 0, s>>>(work, order, bases, counts, out, tables,
-                                                        overflow, parts, n);
+                                                        overflow, parts, n, total);
     else if (max_edge <= 32)
         emit_kernel<32, kBlock><<<grid, kBlock, 0, s>>>(work, order, bases, counts, out, tables,
-                                                        overflow, parts, n);
+                                                        overflow, parts, n, total);
     else
         emit_slab_kernel<<<grid, kBlock, 0, s>>>(work, order, bases, counts, slabs, out, tables,
-                                                 overflow, parts, n);
+                                                 overflow, parts, n, total);
     return hipGetLastError();
 }
 
@@ -2882,7 +2914,14 @@ hipError_t launch_fused(const FusedWork *work, int32_t n, int32_t max_edge,
     return hipGetLastError();
 }
 
-__global__ void __launch_bounds__(kBlock) cull_kernel(CullJob job) { cull_slice(job); }
+__global__ void __launch_bounds__(kBlock) cull_kernel(CullJob job) {
+    cull_slice(job, (int)blockIdx.x, (int)gridDim.x);
+}
+
+// Planes of a cull job, passed by value: no staging to wait for.
+__global__ void __launch_bounds__(64) set_planes_kernel(Planes p, float *__restrict__ dst) {
+    if (threadIdx.x < 24) dst[threadIdx.x] = p.p[threadIdx.x];
+}
 
 // Plain device copy, 16 bytes per lane per step (also the reference point
 // for calibrating HBM byte counters: it reads and writes exactly `n16` x 16 B).
@@ -2923,6 +2962,11 @@ hipError_t launch_pipe(const FusedWork *work, int32_t n, int32_t max_edge, int32
 hipError_t launch_cull(const CullJob &job, hipStream_t s) {
     if (job.n <= 0) return hipSuccess;
     cull_kernel<<<(job.n + kBlock - 1) / kBlock, kBlock, 0, s>>>(job);
+    return hipGetLastError();
+}
+
+hipError_t launch_set_planes(const Planes &planes, float *dst, hipStream_t s) {
+    set_planes_kernel<<<1, 64, 0, s>>>(planes, dst);
     return hipGetLastError();
 }
 
