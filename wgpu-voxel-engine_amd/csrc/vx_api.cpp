@@ -938,7 +938,22 @@ int vx_draw_list_locked(vx_ctx *ctx, const vx_frustum *f, const int32_t *coords_
                         const uint32_t *faces_dev, const uint64_t *first_dev, int32_t n,
                         int32_t edge, uint32_t mode, vx_draw_indexed *args_dev,
                         uint32_t *count_dev) {
+    Planes P;
+    memcpy(P.p, f->planes, sizeof(P.p));
     const int32_t nb = draw_blocks(n);
+    if (n <= kDrawOne) {
+        // one launch; its state words are zeroed once (every launch leaves
+        // them zero)
+        if (!ctx->draw_state) {
+            const size_t bytes = 4 * (size_t)kDrawStateWords;
+            int st = ctx->dev_alloc(bytes, (void **)&ctx->draw_state);
+            if (st) return st;
+            VX_HIP(ctx, hipMemsetAsync(ctx->draw_state, 0, bytes, ctx->stream));
+        }
+        VX_HIP(ctx, launch_draw_one(P, coords_dev, faces_dev, first_dev, n, edge, mode, ctx->draw_state,
+                                    reinterpret_cast<DrawArgs *>(args_dev), count_dev, ctx->stream));
+        return VX_OK;
+    }
     if (nb > ctx->draw_counts_cap) {
         if (ctx->draw_counts) {
             VX_HIP(ctx, hipStreamSynchronize(ctx->stream));  // earlier lists may still read it
@@ -951,8 +966,6 @@ int vx_draw_list_locked(vx_ctx *ctx, const vx_frustum *f, const int32_t *coords_
         if (st) return st;
         ctx->draw_counts_cap = cap;
     }
-    Planes P;
-    memcpy(P.p, f->planes, sizeof(P.p));
     VX_HIP(ctx, launch_draw_list(P, coords_dev, faces_dev, first_dev, n, edge, mode,
                                  ctx->draw_counts, reinterpret_cast<DrawArgs *>(args_dev),
                                  count_dev, ctx->stream));
