@@ -101,3 +101,25 @@ def test_whole_chunks(ctx, oracle_mod, edge):
         faces = oracle_mod.mesh_buffers(ref, edge, (0, 0, 0), [None] * 4)[0]
         assert b.chunk_faces(i)[1] == len(faces), i
     b.close()
+
+
+@pytest.mark.parametrize("n", [127, 130, 1030])
+@pytest.mark.parametrize("kind", ["four octaves", "six octaves", "reference rule", "heightmap"])
+def test_tiles_beside_64(ctx, oracle_mod, kind, n):
+    """Batches with 64^3 chunks on both sides of their tiles' rule (16, 8 and
+    4 workgroups a chunk), smaller chunks among them."""
+    t = CASES[kind]
+    ot = oracle_terrain(oracle_mod, t)
+    edges = [64 if i % 8 == 3 else (32, 16)[i % 2] for i in range(n)]
+    coords = [(i % 13 - 6, 0, i // 13) for i in range(n)]
+    b = V.Batch(ctx, coords, edges, ctx.terrain(t))
+    b.run()
+    b.wait()
+    for i in [0, 1, 2, 3, n // 2, n - 2, n - 1] + [k for k in range(3, n, 8)][-2:]:
+        ref = oracle_mod.chunk_fill(ot, *coords[i], edges[i])
+        assert (b.ids(i) == ref).all(), i
+        ch = b.chunk(i)
+        assert (ch.occupancy() == oracle_mod.occupancy(ref, edges[i])).all(), i
+        ch.release()
+        assert b.chunk_faces(i)[1] == len(oracle_mod.mesh_buffers(ref, edges[i], (0, 0, 0), [None] * 4)[0]), i
+    b.close()

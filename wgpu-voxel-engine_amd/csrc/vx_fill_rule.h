@@ -23,9 +23,16 @@ constexpr int fast_cols(int edge, int max_edge, int variant) {
 // beside a 64^3 slab) let four workgroups share a CU's 160 KB of LDS.
 constexpr int fast_tab(int max_edge) { return max_edge == 64 ? 208 : 368; }
 
-// Rows of a chunk that a workgroup holds at once: a 64^3 chunk's layers are
-// filled 16 at a time (8 KB of rows instead of 32 KB), smaller chunks whole.
-constexpr int fast_slab(int max_edge) { return max_edge == 64 ? 16 : max_edge; }
+// Rows (layers times lines) of a chunk that a workgroup holds at once: a
+// quarter of a 64^3 chunk's (8 KB instead of 32 KB), a smaller chunk's all.
+constexpr int fast_rows(int max_edge) { return max_edge == 64 ? 1024 : max_edge * max_edge; }
+
+// Workgroups per 64^3 chunk of the fast fill in a batch of n chunks, 4 at least
+// (fast_rows).  1,024 run at once: at 323 chunks 4 are 1,292, a second round
+// that is nearly empty; 8 take 103 us, 16 107 us.  A ragged batch of 2,048
+// takes 73 us with 4 and 13 us more with 8: nothing is left to even out, and
+// each workgroup lays its terms out anew.
+constexpr int fill64_parts_for(int n) { return n >= 1024 ? 4 : n >= 128 ? 8 : 16; }
 
 // The variant that takes a density chunk, or 0 for the general kernels.  The
 // fast fill needs

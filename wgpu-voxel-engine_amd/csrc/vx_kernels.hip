@@ -43,6 +43,8 @@ template <class T> __device__ __forceinline__ GlobalPtr<T> as_global(T *p) {
     return (GlobalPtr<T>)p;
 }
 
+typedef uint32_t Ids16 __attribute__((ext_vector_type(4)));  // 16 block ids
+
 // Exclusive scan of one u32 per thread over a BLOCK-thread workgroup.
 template <int BLOCK = kBlock>
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t *s_wave,
@@ -79,13 +81,6 @@ __device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t *s_wave) {
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
-}
-
-// v with lane `lane` replaced by the uniform value x (v_writelane_b32, which
-// this compiler exposes as an intrinsic only).
-extern "C" __device__ int vx_llvm_writelane(int x, int lane, int v) __asm("llvm.amdgcn.writelane.i32");
-__device__ __forceinline__ uint32_t write_lane(uint32_t x, uint32_t lane, uint32_t v) {
-    return (uint32_t)vx_llvm_writelane((int)x, (int)lane, (int)v);
 }
 
 // 2-D improved-noise gradient: x+y, -x+y, x-y, -x-y, x, -x, y, -y.
@@ -601,7 +596,7 @@ __device__ void generate_rows(const TerrainDev &T, int ox, int oy, int oz, const
 }
 
 // Writes the layers y_lo <= y < y_hi of a chunk whose occupancy rows for
-// them are in S.occ (which starts at layer y_base): occupancy and boundary planes always, u8 ids (all solid
+// them are in S.occ: occupancy and boundary planes always, u8 ids (all solid
 // voxels = kBlockGrass) when write_ids; meta[0] = solid block id from the
 // workgroup that writes layer 0.  COHERENT: the occupancy rows and boundary
 // planes, which other workgroups of the same launch read, are written with
@@ -609,10 +604,10 @@ __device__ void generate_rows(const TerrainDev &T, int ox, int oy, int oz, const
 // write-back; a plain store may stay in the writing XCD's L2).
 template <int N, int MAXN, bool COHERENT = false, class SH>
 __device__ void write_chunk_outputs(const FillWork &w, SH &S, bool write_ids, uint32_t solid_type,
-                                    int y_lo = 0, int y_hi = N, int y_base = 0) {
+                                    int y_lo = 0, int y_hi = N) {
     constexpr int W = N == 64 ? 2 : 1;
     constexpr int RS = RowStride<MAXN>::v;
-    const uint32_t *occ = reinterpret_cast<const uint32_t *>(S.occ) - y_base * N * RS;
+    const uint32_t *occ = reinterpret_cast<const uint32_t *>(S.occ);
     const int tid = threadIdx.x;
     const int span = y_hi - y_lo;
     auto put = [](uint32_t *p, uint32_t v) {
@@ -650,7 +645,6 @@ __device__ void write_chunk_outputs(const FillWork &w, SH &S, bool write_ids, ui
     if (write_ids) {
         // u8 block ids, 16 voxels per 16-byte store
         constexpr int PER_ROW = N / 16;
-        typedef uint32_t Ids16 __attribute__((ext_vector_type(4)));
         const GlobalPtr<Ids16> ids4 = as_global(reinterpret_cast<Ids16 *>(w.ids));
         for (int q = y_lo * N * PER_ROW + tid; q < y_hi * N * PER_ROW; q += kBlock) {
             const int r = q / PER_ROW, part = q - r * PER_ROW;
@@ -767,7 +761,6 @@ __device__ void pack_chunk(const FillWork &w, FillShared<MAXN> &S, uint32_t soli
                            int y_hi) {
     constexpr int RS = RowStride<MAXN>::v;
     constexpr int PER_ROW = N / 16;
-    typedef uint32_t Ids16 __attribute__((ext_vector_type(4)));
     const GlobalPtr<const Ids16> ids = as_global(reinterpret_cast<const Ids16 *>(w.ids));
     uint16_t *occ = reinterpret_cast<uint16_t *>(S.occ);
     for (int q = y_lo * N * PER_ROW + threadIdx.x; q < y_hi * N * PER_ROW; q += kBlock) {
@@ -890,13 +883,13 @@ fill_split_kernel(const FillWork *__restrict__ work, const int32_t *__restrict__
 // infinities satisfy neither comparison and so take the exact row.
 //
 // Bound by VALU issue at four waves per SIMD: per 64 voxels of four octaves 12
-// FMAs, two comparisons and two lane writes (a comparison, a lane write, a
+// FMAs, two comparisons and a 64-bit move (a comparison, a lane write, a
 // shift or an SGPR operand issues in 4 cycles, an FMA, add or right shift in
 // 2), about 10 more for the columns' coefficients and the tables.  4096 chunks
-// of 32^3, four octaves: 128 us, against 376 us for the octave-inner loop of
+// of 32^3, four octaves: 126 us, against 376 us for the octave-inner loop of
 // the general kernels (152 VALU per 64 voxels); 1640 chunks under the
-// reference rule 49 against 146 us, 323 chunks of 64^3 136 against 381 us, 1023
-// chunks of six octaves 127 against 400 us.  Two columns per lane at five or
+// reference rule 49 against 146 us, 323 chunks of 64^3 103 against 381 us, 1023
+// chunks of six octaves 122 against 400 us.  Two columns per lane at five or
 // six waves per SIMD, or reading the next row's terms early, changed nothing
 // (143, 142, 139 against 136 us at that stage).
 template <int MAXN> struct FastShared {
@@ -912,13 +905,13 @@ template <int MAXN> struct FastShared {
     float4 grad[kMaxOctaves][16];  // amplitude * gradient (x, col, row) by hash
     union {
         float4 tab[kBlock / 64][fast_tab(MAXN)];
-        alignas(16) uint8_t height[fast_slab(MAXN) * MAXN];  // heightmaps: solid layers per column
+        alignas(16) uint8_t height[fast_rows(MAXN)];  // heightmaps: solid layers per column
     };
     float2 yrow[MAXN * (kMaxOctaves + 1)];
     float2 xcol[kMaxOctaves * MAXN];  // (fx, fade(fx)) per octave and x
     uint8_t ycell[kMaxOctaves * MAXN], xcell[kMaxOctaves * MAXN];
     uint32_t ychg[MAXN];
-    typename RowType<MAXN>::T occ[fast_slab(MAXN) * MAXN];
+    typename RowType<MAXN>::T occ[fast_rows(MAXN)];
     uint32_t red[kBlock / 64];
 };
 
@@ -1008,45 +1001,83 @@ __device__ __forceinline__ void build_terms(const TerrainDev &T, const float4 *G
     }
 }
 
-// Stores the rows of C * 64 / N lines from line z0: lane r < rows holds the
-// ballots of row y0 + r (klo, khi: C halves of 64 / N lines each).
-template <int N, int MAXN, int C, class SH>
-__device__ __forceinline__ void put_lines(SH &S, const uint32_t (&klo)[C], const uint32_t (&khi)[C],
-                                          int z0, int y0, int rows, int lane) {
+// v with lane `lane` replaced by the uniform value x (v_writelane_b32, which
+// this compiler exposes as an intrinsic only).
+extern "C" __device__ int vx_llvm_writelane(int x, int lane, int v) __asm("llvm.amdgcn.writelane.i32");
+
+// Puts the uniform 64-bit values v[c] into k[c] of lane r.  Called with every
+// lane of the wave active.  Four values: 64-bit moves with one lane enabled,
+// half the cost of two lane writes each (4.6 against 9 cycles; grid of 4,096
+// 32^3 chunks filled in 131 us against 133); fewer gain nothing from it, and a
+// heightmap's loop, which can overlap its lane writes, loses (ragged batch of
+// 2,048 in 77 us against 73).
+template <int C>
+__device__ __forceinline__ void keep_rows(uint64_t (&k)[C], const uint64_t (&v)[C], int r) {
+    if constexpr (C == 4) {
+        uint64_t all;
+        asm volatile("s_mov_b64 %4, exec\n\ts_mov_b64 exec, %5\n\ts_nop 1\n\tv_mov_b64 %0, %6\n\t"
+                     "v_mov_b64 %1, %7\n\tv_mov_b64 %2, %8\n\tv_mov_b64 %3, %9\n\ts_mov_b64 exec, %4"
+                     : "+v"(k[0]), "+v"(k[1]), "+v"(k[2]), "+v"(k[3]), "=&s"(all)
+                     : "s"(1ull << r), "s"(v[0]), "s"(v[1]), "s"(v[2]), "s"(v[3]));
+    } else {
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            const int lo = vx_llvm_writelane((int)(uint32_t)v[c], r, (int)(uint32_t)k[c]);
+            const int hi = vx_llvm_writelane((int)(v[c] >> 32), r, (int)(k[c] >> 32));
+            k[c] = (uint64_t)(uint32_t)hi << 32 | (uint32_t)lo;
+        }
+    }
+}
+
+// A tile of a chunk that a fast-fill workgroup holds: layers [y_lo, y_hi) of
+// 1 << LS lines from z_lo (LS < 0: 1 << ls of them), its row (y, z) at
+// S.occ[(y - y_lo) * lines + z - z_lo].
+template <int LS>
+struct FillTile {
+    int y_lo, y_hi, z_lo, ls;
+    __device__ __forceinline__ int shift() const { return LS < 0 ? ls : LS; }
+    __device__ __forceinline__ int lines() const { return 1 << shift(); }
+    __device__ __forceinline__ int rows() const { return (y_hi - y_lo) << shift(); }
+    __device__ __forceinline__ int row(int y, int z) const { return ((y - y_lo) << shift()) + z - z_lo; }
+};
+// log2 of a chunk's lines
+constexpr int line_bits(int edge) { return edge == 16 ? 4 : edge == 32 ? 5 : 6; }
+
+// Stores the rows of C * 64 / N lines from line z: lane r < rows holds the
+// ballots of row y + r.
+template <int N, int MAXN, int C, class SH, class TILE>
+__device__ __forceinline__ void put_lines(SH &S, const TILE &t, const uint64_t (&k)[C], int z, int y,
+                                          int rows, int lane) {
     constexpr int RS = RowStride<MAXN>::v;
     if (lane >= rows) return;
-    uint32_t *dst = reinterpret_cast<uint32_t *>(S.occ) + ((y0 + lane) * N + z0) * RS;
+    uint32_t *dst = reinterpret_cast<uint32_t *>(S.occ) + t.row(y + lane, z) * RS;
+    constexpr uint32_t MASK = N >= 32 ? 0xFFFFFFFFu : ((1u << (N & 31)) - 1u);
 #pragma unroll
     for (int c = 0; c < C; c++) {
         if constexpr (N == 64) {
-            dst[2 * c] = klo[c];
-            dst[2 * c + 1] = khi[c];
-        } else if constexpr (N == 32) {
-            dst[2 * c * RS] = klo[c];
-            dst[(2 * c + 1) * RS] = khi[c];
-            if (RS == 2) dst[2 * c * RS + 1] = dst[(2 * c + 1) * RS + 1] = 0u;
+            dst[2 * c] = (uint32_t)k[c];
+            dst[2 * c + 1] = (uint32_t)(k[c] >> 32);
         } else {
-            const uint32_t v[4] = {klo[c] & 0xFFFFu, klo[c] >> 16, khi[c] & 0xFFFFu, khi[c] >> 16};
+            constexpr int L = 64 / N;
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                dst[(4 * c + k) * RS] = v[k];
-                if (RS == 2) dst[(4 * c + k) * RS + 1] = 0u;
+            for (int j = 0; j < L; j++) {
+                dst[(L * c + j) * RS] = (uint32_t)(k[c] >> (j * N)) & MASK;
+                if (RS == 2) dst[(L * c + j) * RS + 1] = 0u;
             }
         }
     }
 }
 
-// Rows [y_lo, y_hi) of a density (or reference-rule) chunk into S.occ (from
-// its start).  A wave
+// The rows of a tile of a density (or reference-rule) chunk into S.occ.  A wave
 // takes C * 64 / N lines along x, so a lane holds C columns (same x, lines
 // 64 / N apart) and reads each row's terms once for the C of them.  Per
 // octave the lines' lattice gradients are blended along z once into a table
 // of the wave (one entry per line, y plane and lattice x: value slope qx,
 // offset q0 and row slope qy); a column that enters a y cell blends four
 // entries along x into its A0, A1, D0, D1.
-template <int N, int MAXN, int OCT, int C, class SH>
-__device__ void density_rows_fast(const TerrainDev &T, int ox, int oy, int oz, SH &S, int y_lo,
-                                  int y_hi) {
+template <int N, int MAXN, int OCT, int C, class SH, class TILE>
+__device__ void density_rows_fast(const TerrainDev &T, int ox, int oy, int oz, SH &S,
+                                  const TILE &tile) {
     constexpr int L = 64 / N, LINES = L * C, RS = RowStride<MAXN>::v;
     constexpr int SLOTS = 64 / LINES;
     const bool ref = T.kind == kReference;
@@ -1065,12 +1096,12 @@ __device__ void density_rows_fast(const TerrainDev &T, int ox, int oy, int oz, S
             f = f * T.lacunarity;
         }
     }
-    for (int g = wave; g < N / LINES; g += kBlock / 64) {
-        int r0 = y_lo;
+    for (int z0 = tile.z_lo + wave * LINES; z0 < tile.z_lo + tile.lines(); z0 += kBlock / 64 * LINES) {
+        int r0 = tile.y_lo;
 #pragma unroll 1
-        while (r0 < y_hi) {
+        while (r0 < tile.y_hi) {
             // as many rows as the wave's table holds the planes of
-            int rows = y_hi - r0;
+            int rows = tile.y_hi - r0;
             int np[OCT], at[OCT];
             for (;;) {
                 int e = 0;
@@ -1095,20 +1126,26 @@ __device__ void density_rows_fast(const TerrainDev &T, int ox, int oy, int oz, S
                 auto at4 = [](const char *p, int off) { return *reinterpret_cast<const int *>(p + off); };
 #pragma unroll
                 for (int o = 0; o < OCT; o++) {
-                    const float Z = (float)(oz + g * LINES + line) * fo[o];
+                    const float Z = (float)(oz + z0 + line) * fo[o];
                     const float zl = floorf(Z);
                     const float z = Z - zl, z1 = z - 1.0f, w = fade(z);
                     const int Z4 = ((int)zl & 255) * 4;
                     const int X4 = ((int)floorf((float)ox * fo[o]) & 255) * 4;
                     const int Y4 = (((int)floorf((float)oy * fo[o]) + (int)S.ycell[o * N + r0]) & 255) * 4;
                     const char *grad = reinterpret_cast<const char *>(S.grad[o]);
-                    // two planes at a time (the last twice when they are odd):
-                    // each is a chain of dependent LDS reads
+                    // slots: lattice x (a power of two of them) times groups of
+                    // planes, each of which takes every groups-th plane, two at
+                    // a time (a chain of dependent LDS reads each; past the end
+                    // the last plane again).  With a slot per lattice x alone
+                    // most idle where cells are large (1,023 chunks of six
+                    // octaves: 128 us, against 122)
+                    const int sh = 32 - __builtin_clz(lx[o] - 1);
+                    const int groups = max(SLOTS >> sh, 1), last = np[o] - 1;
+                    const int pg = (slot >> sh) & (groups - 1);
                     auto planes = [&](float4 *dst, auto hashes) {
-                        const int last = np[o] - 1;
 #pragma unroll 1
-                        for (int p = 0; p <= last; p += 2) {
-                            const int q = min(p + 1, last);
+                        for (int p0 = pg; p0 <= last; p0 += 2 * groups) {
+                            const int p = p0, q = min(p0 + groups, last);
                             int h[4];
                             hashes(p * 4, h[0], h[1]);
                             hashes(q * 4, h[2], h[3]);
@@ -1126,7 +1163,7 @@ __device__ void density_rows_fast(const TerrainDev &T, int ox, int oy, int oz, S
                         }
                     };
 #pragma unroll 1
-                    for (int i = slot; i < lx[o]; i += SLOTS) {
+                    for (int i = slot & ((1 << sh) - 1); i < lx[o]; i += SLOTS) {
                         float4 *dst = tab + at[o] + line * (np[o] * lx[o]) + i;
                         const int px = at4(perm, X4 + i * 4);
                         if (ref) {  // perm[perm[perm[X] + Z] + Y]
@@ -1157,10 +1194,9 @@ __device__ void density_rows_fast(const TerrainDev &T, int ox, int oy, int oz, S
                 }
             }
             float A0[C][OCT], A1[C][OCT], D0[C][OCT], D1[C][OCT], As[C];
-            uint32_t klo[C], khi[C];
-            uint64_t doubt[C];
+            uint64_t kept[C], doubt[C];
 #pragma unroll
-            for (int c = 0; c < C; c++) klo[c] = khi[c] = 0u, doubt[c] = 0ull;
+            for (int c = 0; c < C; c++) kept[c] = doubt[c] = 0ull;
             int r = 0;
 #pragma unroll 1
             while (r < rows) {
@@ -1214,17 +1250,16 @@ __device__ void density_rows_fast(const TerrainDev &T, int ox, int oy, int oz, S
 #pragma unroll
                         for (int c = 0; c < C; c++) acc[c] = fmaf(t[o].y, d[c], acc[c]);
                     }
-                    uint64_t sure[C], all = ~0ull;
+                    uint64_t sure[C], solid[C], all = ~0ull;
 #pragma unroll
                     for (int c = 0; c < C; c++) {
                         const uint64_t above = __ballot(acc[c] > t[OCT].x);
                         const uint64_t below = __ballot(acc[c] < t[OCT].y);
-                        const uint64_t solid = ref ? below : above;
+                        solid[c] = ref ? below : above;
                         sure[c] = above | below;
                         all &= sure[c];
-                        klo[c] = write_lane((uint32_t)solid, (uint32_t)r, klo[c]);
-                        khi[c] = write_lane((uint32_t)(solid >> 32), (uint32_t)r, khi[c]);
                     }
+                    keep_rows(kept, solid, r);
                     if (all != ~0ull) {  // uniform, rare
 #pragma unroll
                         for (int c = 0; c < C; c++)
@@ -1232,7 +1267,7 @@ __device__ void density_rows_fast(const TerrainDev &T, int ox, int oy, int oz, S
                     }
                 }
             }
-            put_lines<N, MAXN, C>(S, klo, khi, g * LINES, r0 - y_lo, rows, lane);
+            put_lines<N, MAXN, C>(S, tile, kept, z0, r0, rows, lane);
             // rows with a voxel too near its threshold, in the oracle's order
             uint32_t *occ = reinterpret_cast<uint32_t *>(S.occ);
 #pragma unroll 1
@@ -1242,7 +1277,7 @@ __device__ void density_rows_fast(const TerrainDev &T, int ox, int oy, int oz, S
                 for (int k = 1; k < C; k++) m = c == k ? doubt[k] : m;
 #pragma unroll 1
                 for (; m; m &= m - 1ull) {
-                    const int y = r0 + __builtin_ctzll(m), zl = g * LINES + c * L + sub;
+                    const int y = r0 + __builtin_ctzll(m), zl = z0 + c * L + sub;
                     const float wx = (float)(ox + xl), wy = (float)(oy + y), wz = (float)(oz + zl);
                     const float s = exact_fbm(T, S.perm, wx, ref ? wz : wy, ref ? wy : wz);
                     const bool solid = ref ? solid_of<true>(s, T, oy + y) : solid_of<false>(s, T, oy + y);
@@ -1250,7 +1285,7 @@ __device__ void density_rows_fast(const TerrainDev &T, int ox, int oy, int oz, S
                     wave_sync();  // after the row's first value
                     if (xl == 0) {
                         constexpr uint32_t MASK = N >= 32 ? 0xFFFFFFFFu : ((1u << (N & 31)) - 1u);
-                        uint32_t *dst = occ + ((y - y_lo) * N + zl) * RS;
+                        uint32_t *dst = occ + tile.row(y, zl) * RS;
                         dst[0] = (uint32_t)(b >> (sub * N)) & MASK;
                         if (N == 64) dst[RS - 1] = (uint32_t)(b >> 32);
                     }
@@ -1261,19 +1296,82 @@ __device__ void density_rows_fast(const TerrainDev &T, int ox, int oy, int oz, S
     }
 }
 
-// Lines [z_lo, z_hi) of a 2-D fBm heightmap chunk, with their outputs: h =
-// floor(height_scale * (n + 1) / 2) clamped to [0, height_max]; voxel solid
-// iff wy <= h.  A workgroup takes lines and all their layers, so that a
-// column's noise is evaluated once.  Block ids come from the heights, four
-// columns to a dword: with H = the solid layers of each (0..64) in bytes, bit
-// 7 of 0x80 + H - (y + 1) says whether layer y is one of them.
-template <int N, int MAXN, class SH>
-__device__ void heightmap_lines_out(const FillWork &w, const TerrainDev &T, SH &S, int z_lo, int z_hi) {
-    constexpr int L = 64 / N, W = N == 64 ? 2 : 1, RS = RowStride<MAXN>::v;
+// Planes x=0, x=N-1 (bit z per y) of a tile whose rows are in S.occ: ballots
+// of 64 rows, a byte per 8 lines.
+template <int N, int MAXN, class SH, class TILE>
+__device__ void write_x_planes(const FillWork &w, SH &S, const TILE &t) {
+    constexpr int W = N == 64 ? 2 : 1, RS = RowStride<MAXN>::v;
+    const uint32_t *occ = reinterpret_cast<const uint32_t *>(S.occ);
+    const GlobalPtr<uint8_t> planes = as_global(reinterpret_cast<uint8_t *>(w.planes));
+    const int ls = t.shift(), per = t.lines() / 8, rows = t.rows();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, pl = lane >> 3, q = lane & 7;
+    for (int r0 = wave * 64; r0 < rows; r0 += kBlock) {
+        const uint32_t *row = occ + min(r0 + lane, rows - 1) * RS;
+        const uint64_t first = __ballot(row[0] & 1u);
+        const uint64_t last = __ballot((row[W - 1] >> ((N < 32 ? N : 32) - 1)) & 1u);
+        const int y = t.y_lo + ((r0 + 8 * q) >> ls);
+        if (pl < 2 && r0 + 8 * q < rows) {
+            const int at = (pl * N + y) * W * 4;
+            planes[at + t.z_lo / 8 + q % per] = (uint8_t)((pl ? last : first) >> (8 * q));
+            if (N == 16 && t.z_lo == 0 && q % per == 0) {  // a word's upper half
+                planes[at + 2] = 0;
+                planes[at + 3] = 0;
+            }
+        }
+    }
+}
+
+// Occupancy rows, planes z=0, z=N-1 and meta of a tile whose rows are in S.occ.
+template <int N, int MAXN, class SH, class TILE>
+__device__ void write_rows(const FillWork &w, SH &S, const TILE &t) {
+    constexpr int W = N == 64 ? 2 : 1, RS = RowStride<MAXN>::v;
+    const uint32_t *occ = reinterpret_cast<const uint32_t *>(S.occ);
+    const int tid = threadIdx.x, ls = t.shift(), lines = t.lines(), n = t.rows() * W;
+    const GlobalPtr<uint32_t> out = as_global(w.occ), planes = as_global(w.planes);
+    for (int i = tid; i < n; i += kBlock) {
+        const int r = i / W;
+        out[((t.y_lo + (r >> ls)) * N + t.z_lo + (r & (lines - 1))) * W + i % W] = occ[r * RS + i % W];
+    }
+    for (int k = tid; k < 2 * (t.y_hi - t.y_lo) * W; k += kBlock) {
+        const int pl = k & 1, y = t.y_lo + (k >> 1) / W, j = (k >> 1) % W;
+        if (pl ? t.z_lo + lines == N : t.z_lo == 0)
+            planes[((2 + pl) * N + y) * W + j] = occ[t.row(y, pl ? N - 1 : 0) * RS + j];
+    }
+    if (tid == 0 && t.y_lo == 0 && t.z_lo == 0) *as_global(w.meta) = kBlockGrass;
+}
+
+// Block ids of a tile from its rows, 16 voxels per 16-byte store: a nibble of
+// a row times 1 + 2^7 + 2^14 + 2^21 has its bits at the four bytes' bit 0.
+template <int N, int MAXN, class SH, class TILE>
+__device__ void write_ids(const FillWork &w, SH &S, const TILE &t) {
+    constexpr int RS = RowStride<MAXN>::v, PER = N / 16;
+    const uint16_t *occ = reinterpret_cast<const uint16_t *>(S.occ);
+    const int ls = t.shift(), n = t.rows() * PER;
+    const GlobalPtr<Ids16> ids = as_global(reinterpret_cast<Ids16 *>(w.ids));
+    for (int q = threadIdx.x; q < n; q += kBlock) {
+        const int r = q / PER;
+        const uint32_t bits = occ[r * RS * 2 + q % PER];
+        Ids16 v;
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            v[k] = (__umul24((bits >> (4 * k)) & 15u, 0x00204081u) & 0x01010101u) * kBlockGrass;
+        ids[((t.y_lo + (r >> ls)) * N + t.z_lo) * PER + q - (r >> ls << ls) * PER] = v;
+    }
+}
+
+// Lines of a 2-D fBm heightmap chunk (all layers of them, so that a column's
+// noise is evaluated once), with their outputs: h = floor(height_scale * (n +
+// 1) / 2) clamped to [0, height_max]; voxel solid iff wy <= h.  Block ids come
+// from the heights, four columns to a dword: with H = the solid layers of each
+// (0..64) in bytes, bit 7 of 0x80 + H - (y + 1) says whether layer y is one of
+// them.
+template <int N, int MAXN, class SH, class TILE>
+__device__ void heightmap_tile(const FillWork &w, const TerrainDev &T, SH &S, const TILE &t) {
+    constexpr int L = 64 / N;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int lines = z_hi - z_lo;
+    const int lines = t.lines();
     for (int i = tid; i < N * lines; i += kBlock) {
-        const float wx = (float)(w.cx * N + i % N), wz = (float)(w.cz * N + z_lo + i / N);
+        const float wx = (float)(w.cx * N + i % N), wz = (float)(w.cz * N + t.z_lo + i / N);
         float sum = 0.0f, amp = 1.0f, f = T.frequency;
 #pragma unroll 1
         for (int o = 0; o < T.octaves; o++) {
@@ -1290,124 +1388,105 @@ __device__ void heightmap_lines_out(const FillWork &w, const TerrainDev &T, SH &
         S.height[i] = (uint8_t)(top < 0 ? 0 : top > N ? N : top);
     }
     __syncthreads();
-    // occupancy rows, line by line: S.occ[y * lines + z - z_lo]
-    uint32_t *occ = reinterpret_cast<uint32_t *>(S.occ);
     for (int g = wave; g < lines / L; g += kBlock / 64) {
         const int h = S.height[g * 64 + lane];
-        uint32_t klo = 0u, khi = 0u;
+        uint64_t kept[1] = {0ull};
         for (int y = 0; y < N; y++) {
-            const uint64_t b = __ballot(y < h);
-            klo = write_lane((uint32_t)b, (uint32_t)y, klo);
-            khi = write_lane((uint32_t)(b >> 32), (uint32_t)y, khi);
+            const uint64_t b[1] = {__ballot(y < h)};
+            keep_rows(kept, b, y);
         }
-        if (lane < N) {
-            uint32_t *dst = occ + (lane * lines + g * L) * RS;
-            constexpr uint32_t MASK = N >= 32 ? 0xFFFFFFFFu : ((1u << (N & 31)) - 1u);
-            if constexpr (N == 64) {
-                dst[0] = klo;
-                dst[1] = khi;
-            } else {
-                const uint64_t b = (uint64_t)khi << 32 | klo;
-#pragma unroll
-                for (int k = 0; k < L; k++) {
-                    dst[k * RS] = (uint32_t)(b >> (k * N)) & MASK;
-                    if (RS == 2) dst[k * RS + 1] = 0u;
-                }
-            }
-        }
+        put_lines<N, MAXN, 1>(S, t, kept, t.z_lo + g * L, 0, N, lane);
     }
-    // boundary planes x=0, x=N-1 (bit z per y), eight lines to a byte
-    const GlobalPtr<uint8_t> pb = as_global(reinterpret_cast<uint8_t *>(w.planes));
-    const int bytes = lines / 8;
-    for (int k = tid; k < 2 * N * bytes; k += kBlock) {
-        const int b = k % bytes, y = k / bytes % N, pl = k / (bytes * N);
+    // planes x=0, x=N-1 (bit z per y), eight lines to a byte
+    const GlobalPtr<uint8_t> planes = as_global(reinterpret_cast<uint8_t *>(w.planes));
+    for (int k = tid; k < 2 * N * (lines / 8); k += kBlock) {
+        const int b = k % (lines / 8), y = k / (lines / 8) % N, pl = k / (lines / 8 * N);
+        const int at = (pl * N + y) * (N == 64 ? 8 : 4);
         uint32_t v = 0;
 #pragma unroll
         for (int j = 0; j < 8; j++)
             v |= (uint32_t)(y < (int)S.height[(b * 8 + j) * N + (pl ? N - 1 : 0)]) << j;
-        pb[(pl * N + y) * W * 4 + z_lo / 8 + b] = (uint8_t)v;
-        if (N == 16 && z_lo == 0 && b < 2) pb[(pl * N + y) * W * 4 + 2 + b] = 0;
-        if (N == 16 && z_lo == 0 && bytes == 1) pb[(pl * N + y) * W * 4 + 3] = 0;
+        planes[at + t.z_lo / 8 + b] = (uint8_t)v;
+        if (N == 16 && t.z_lo == 0 && b == 0) {  // a word's upper half
+            planes[at + 2] = 0;
+            planes[at + 3] = 0;
+        }
     }
-    // ids, 16 voxels per 16-byte store: a wave takes layers, a lane 16 columns
-    {
-        typedef uint32_t Ids16 __attribute__((ext_vector_type(4)));
-        const GlobalPtr<Ids16> ids = as_global(reinterpret_cast<Ids16 *>(w.ids));
-        const int groups = lines * N / 16;  // of 16 columns
-        const int per = groups < 64 ? 64 / groups : 1;  // layers of a wave pass
-        for (int g = lane % groups; g < groups; g += 64) {
-            const uint4 H = *reinterpret_cast<const uint4 *>(S.height + g * 16);
-            const uint32_t h[4] = {H.x + 0x80808080u, H.y + 0x80808080u, H.z + 0x80808080u,
-                                   H.w + 0x80808080u};
-            for (int y = wave * per + lane / groups; y < N; y += kBlock / 64 * per) {
-                const uint32_t sub = (uint32_t)(y + 1) * 0x01010101u;
-                Ids16 v;
+    // a wave takes layers, a lane 16 columns
+    const GlobalPtr<Ids16> ids = as_global(reinterpret_cast<Ids16 *>(w.ids));
+    const int groups = lines * N / 16, per = groups < 64 ? 64 / groups : 1;
+    for (int g = lane % groups; g < groups; g += 64) {
+        const uint4 H = *reinterpret_cast<const uint4 *>(S.height + g * 16);
+        const uint32_t h[4] = {H.x + 0x80808080u, H.y + 0x80808080u, H.z + 0x80808080u,
+                               H.w + 0x80808080u};
+        for (int y = wave * per + lane / groups; y < N; y += kBlock / 64 * per) {
+            const uint32_t sub = (uint32_t)(y + 1) * 0x01010101u;
+            Ids16 v;
 #pragma unroll
-                for (int k = 0; k < 4; k++) v[k] = ((h[k] - sub) >> 7) & (0x01010101u * kBlockGrass);
-                ids[(y * N + z_lo) * (N / 16) + g] = v;
-            }
+            for (int k = 0; k < 4; k++) v[k] = ((h[k] - sub) >> 7) & (0x01010101u * kBlockGrass);
+            ids[(y * N + t.z_lo) * (N / 16) + g] = v;
         }
     }
     __syncthreads();
-    // rows and boundary planes z=0, z=N-1
-    const GlobalPtr<uint32_t> out = as_global(w.occ), planes = as_global(w.planes);
-    for (int i = tid; i < N * lines * W; i += kBlock) {
-        const int y = i / (lines * W), r = i - y * (lines * W);
-        out[(y * N + z_lo) * W + r] = occ[(y * lines + r / W) * RS + r % W];
-    }
-    for (int k = tid; k < 2 * N * W; k += kBlock) {
-        const int pl = k / (N * W), y = k / W % N, j = k % W;
-        if (pl ? z_hi == N : z_lo == 0)
-            planes[((2 + pl) * N + y) * W + j] = occ[(y * lines + (pl ? lines - 1 : 0)) * RS + j];
-    }
-    if (tid == 0 && z_lo == 0) *as_global(w.meta) = kBlockGrass;
+    write_rows<N, MAXN>(w, S, t);
 }
 
-// Rows [y_lo, y_hi), at most fast_slab(MAXN) of them, of a chunk that the
-// host marked for this path, with their outputs.  OCT: octaves compiled for
-// (0: no 3-D noise).
-template <int N, int MAXN, int OCT, class SH>
-__device__ __forceinline__ void fast_rows(const FillWork &w, const TerrainDev &T, const float4 *G,
-                                          SH &S, int y_lo, int y_hi) {
+// A tile of a chunk that the host marked for this path, with its outputs.
+// OCT: octaves compiled for (0: no noise, all air or all solid).
+template <int N, int MAXN, int OCT, class SH, class TILE>
+__device__ __forceinline__ void fast_tile(const FillWork &w, const TerrainDev &T, const float4 *G,
+                                          SH &S, const TILE &t) {
     using R = typename RowType<MAXN>::T;
     const int ox = w.cx * N, oy = w.cy * N, oz = w.cz * N;
     if constexpr (OCT > 0) {
         build_terms<N, OCT>(T, G, ox, oy, S);
         __syncthreads();
-        density_rows_fast<N, MAXN, OCT, fast_cols(N, MAXN, OCT)>(T, ox, oy, oz, S, y_lo, y_hi);
+        density_rows_fast<N, MAXN, OCT, fast_cols(N, MAXN, OCT)>(T, ox, oy, oz, S, t);
     } else {
         constexpr uint32_t ROW = N >= 32 ? 0xFFFFFFFFu : ((1u << (N & 31)) - 1u);
         const R full = T.kind != kSolid ? (R)0 : N == 64 ? (R)~(R)0 : (R)ROW;
-        for (int i = threadIdx.x; i < (y_hi - y_lo) * N; i += kBlock) S.occ[i] = full;
+        for (int i = threadIdx.x; i < t.rows(); i += kBlock) S.occ[i] = full;
     }
     __syncthreads();
-    write_chunk_outputs<N, MAXN>(w, S, true, kBlockGrass, y_lo, y_hi, y_lo);
+    write_rows<N, MAXN>(w, S, t);
+    write_x_planes<N, MAXN>(w, S, t);
+    write_ids<N, MAXN>(w, S, t);
 }
 
-// Workgroup `part` of `parts` on chunk w, each with N / parts layers (lines of
-// a heightmap); in a
-// batch of several edges a smaller chunk takes the parts that give its
-// workgroups as many rows as a 64^3 chunk's.  A whole chunk of edge up to 32
-// also counts its faces (FillWork.count_out).
+// Workgroup `part` of `parts` (a power of two) on chunk w.  64^3 chunks of
+// noise and heightmaps are cut into lines, eight at least (all layers of a
+// line share its tables or heights), the former into layers beyond that: 323
+// chunks of 64^3 in 103 us, against 136 for four slabs of 16 layers, which read
+// each table for 16 rows only.  Other chunks are cut into layers (the lines of
+// a smaller one are one group per wave, and air and solid ones store whole
+// layers: in tiles of lines a ragged batch's fill took 78 us against 73), in a
+// batch that holds 64^3 chunks fewer of the smaller ones.  A whole chunk of edge up to 32 also counts its faces
+// (FillWork.count_out).
 template <int N, int MAXN, class SH>
 __device__ __forceinline__ void fast_part(const FillWork &w, const TerrainDev &T, const float4 *G,
                                           SH &S, int part, int parts) {
-    if (MAXN == 64 && N < 64) parts = max(1, parts * N / 64);
-    if (T.kind == kHeightmap) parts = min(parts, N / 8);  // whole bytes of the x planes
+    constexpr int LS = line_bits(N);
+    const bool noise = T.kind == kDensity || T.kind == kReference;
+    if (MAXN == 64 && N < 64 && T.kind != kHeightmap) parts = max(1, parts * N / 64);
+    // the lines' cuts
+    const int cut = T.kind == kHeightmap || (N == 64 && noise) ? min(__builtin_ctz(parts), LS - 3) : 0;
+    if (T.kind == kHeightmap) parts = 1 << cut;
     if (part >= parts) return;
-    const int rows = N / parts, y_lo = part * rows, y_hi = y_lo + rows;
+    const int rows = N / (parts >> cut), ls = LS - cut;
+    const int z_lo = (part & ((1 << cut) - 1)) << ls, y_lo = (part >> cut) * rows;
     if (T.kind == kHeightmap) {
-        heightmap_lines_out<N, MAXN>(w, T, S, y_lo, y_hi);
-    } else if (T.kind == kDensity || T.kind == kReference) {
+        heightmap_tile<N, MAXN>(w, T, S, FillTile<-1>{0, N, z_lo, ls});
+    } else if (noise) {
+        const FillTile<N == 64 ? -1 : LS> t{y_lo, y_lo + rows, z_lo, ls};
         switch (w.variant) {
-        case 2: fast_rows<N, MAXN, 2>(w, T, G, S, y_lo, y_hi); break;
-        case 3: fast_rows<N, MAXN, 3>(w, T, G, S, y_lo, y_hi); break;
-        case 4: fast_rows<N, MAXN, 4>(w, T, G, S, y_lo, y_hi); break;
-        case 6: fast_rows<N, MAXN, 6>(w, T, G, S, y_lo, y_hi); break;
-        default: fast_rows<N, MAXN, 8>(w, T, G, S, y_lo, y_hi); break;
+        case 2: fast_tile<N, MAXN, 2>(w, T, G, S, t); break;
+        case 3: fast_tile<N, MAXN, 3>(w, T, G, S, t); break;
+        case 4: fast_tile<N, MAXN, 4>(w, T, G, S, t); break;
+        case 6: fast_tile<N, MAXN, 6>(w, T, G, S, t); break;
+        default: fast_tile<N, MAXN, 8>(w, T, G, S, t); break;
         }
     } else {
-        fast_rows<N, MAXN, 0>(w, T, G, S, y_lo, y_hi);
+        fast_tile<N, MAXN, 0>(w, T, G, S, FillTile<LS>{y_lo, y_lo + rows, z_lo, ls});
     }
     if constexpr (MAXN <= 32) {
         if (w.count_out && parts == 1) {
@@ -2851,8 +2930,8 @@ hipError_t launch_fill(const FillWork *work, const int32_t *order, int32_t n, in
             fill_fast_kernel<16><<<grid, kBlock, 0, s>>>(work, order, n, terrains, lut, parts, error);
         else if (max_edge <= 32)
             fill_fast_kernel<32><<<grid, kBlock, 0, s>>>(work, order, n, terrains, lut, parts, error);
-        else {  // a workgroup holds 16 layers of a 64^3 chunk
-            const int p = parts < 4 ? 4 : parts;
+        else {
+            const int p = parts_hint ? max(parts, 4) : fill64_parts_for(n);
             fill_fast_kernel<64><<<n * p, kBlock, 0, s>>>(work, order, n, terrains, lut, p, error);
         }
     }
@@ -2893,11 +2972,11 @@ hipError_t launch_scan(const uint32_t *counts, int32_t n, const MeshWork *items,
 hipError_t launch_fill_one(const FillWork &w, const TerrainDev *terrains, const GradLut *lut,
                            hipStream_t s) {
     if (!w.noise_out && w.variant) {
-        // one chunk: a workgroup per four rows (two at edge 16)
-        const int parts = 8;
-        if (w.edge <= 16) fill_fast_one_kernel<16><<<parts, kBlock, 0, s>>>(w, terrains, lut, parts);
-        else if (w.edge <= 32) fill_fast_one_kernel<32><<<parts, kBlock, 0, s>>>(w, terrains, lut, parts);
-        else fill_fast_one_kernel<64><<<parts, kBlock, 0, s>>>(w, terrains, lut, parts);
+        // one chunk: a workgroup per four layers (two at edge 16), or per 8
+        // lines and 16 layers of a 64^3 chunk
+        if (w.edge <= 16) fill_fast_one_kernel<16><<<8, kBlock, 0, s>>>(w, terrains, lut, 8);
+        else if (w.edge <= 32) fill_fast_one_kernel<32><<<8, kBlock, 0, s>>>(w, terrains, lut, 8);
+        else fill_fast_one_kernel<64><<<32, kBlock, 0, s>>>(w, terrains, lut, 32);
         return hipGetLastError();
     }
     if (w.edge <= 16) fill_one_kernel<16><<<1, kBlock, 0, s>>>(w, terrains, lut);
