@@ -56,3 +56,29 @@ def test_ids_out_of_range_are_refused(ctx, bad):
         with pytest.raises(V.VoxelError) as e:
             V.Chunk.from_ids(ctx, (0, 0, 0), 16, ids)
         assert e.value.status == V.ERR_INVALID
+
+
+@pytest.mark.parametrize("edge,n", [(16, 17), (16, 64), (16, 400), (16, 639), (16, 641), (16, 1281), (32, 700),
+                                    (32, 1279), (32, 1281), (32, 1792), (64, 21), (64, 400)])
+def test_batch_parts(ctx, oracle_mod, edge, n):
+    """Batches on both sides of the rule for workgroups per emit item."""
+    print("[case]", edge, n, flush=True)
+    t = V.Terrain(kind=V.TERRAIN_HEIGHTMAP, seed=3, octaves=2, frequency=1 / 24, lacunarity=2.0, gain=0.5,
+                  height_scale=14.0, height_max=15)
+    ot = oracle_mod.terrain(kind=t.kind, seed=t.seed, octaves=t.octaves, frequency=t.frequency,
+                            lacunarity=t.lacunarity, gain=t.gain, height_scale=t.height_scale,
+                            height_max=t.height_max, y_scale=t.y_scale)
+    coords = [(i % 31 - 15, 0, i // 31) for i in range(n)]
+    b = V.Batch(ctx, coords, edge, ctx.terrain(t), None, formats=V.FMT_INSTANCES)
+    b.run()
+    b.wait()
+    inst = b.mesh(V.FMT_INSTANCES)
+    for i in [0, 1, 7, n // 2, n - 2, n - 1]:
+        ids = oracle_mod.chunk_fill(ot, *coords[i], edge)
+        faces, ei, _, _ = oracle_mod.mesh_buffers(ids, edge, tuple(v * edge for v in coords[i]), [None] * 4)
+        first, cnt = b.chunk_faces(i)
+        assert cnt == len(faces), i
+        got = inst[first:first + cnt]
+        assert (got["m"].view(np.uint32) == ei["m"].view(np.uint32)).all(), i
+        assert (got["tex"] == ei["tex"]).all(), i
+    b.close()

@@ -14,6 +14,7 @@ constexpr int kBlock = 256;        // threads per workgroup (4 wave64)
 constexpr int kMaxOctaves = 8;     // fBm octaves supported by the noise tables
 constexpr int kDescTile = 4096;    // face descriptors staged in LDS per emit tile
 constexpr int kEmitGrid = 2560;    // emit workgroups that fill the GPU twice (5 per CU at once)
+constexpr int kEmitThree = 1792;   // chunks of edge 32 up to which three workgroups each pay
 constexpr int kEmitGrid64 = 6144;  // the same over slabs of 64^3 chunks (4 per CU at once)
 constexpr int kFillGrid = 1024;    // fill workgroups that fill the GPU (4 per CU)
 
@@ -181,25 +182,39 @@ inline int words_per_row(int edge) { return (edge + 31) / 32; }
 // more; below that 2, 4 or 8 so that the grid still covers about kFillGrid
 // workgroups (8 only for batches of at most kFillGrid / 8 chunks that hold
 // 64^3 chunks).  `hint` (1, 2, 4 or 8; 0 = this rule) replaces the rule
-// for the batches it would split.
+// for the batches it would split.  (64^3 chunks on the fast path:
+// fill64_parts_for.)
 inline int fill_parts_for(int32_t n, int32_t max_edge, int32_t hint = 0) {
     if (n >= kFillGrid) return 1;
     if (hint > 0) return hint;
     return 2 * n >= kFillGrid ? 2 : (max_edge > 32 && 8 * n <= kFillGrid) ? 8 : 4;
 }
-// Workgroups per emit item: one for kEmitGrid items or more; below that as
-// many as make kEmitGrid workgroups (kEmitGrid64 when the items are slabs of
-// 64^3 chunks, which hold more faces), at most 16, so that the last round of
-// workgroups is short.  On one 1,640-chunk batch of 32^3 1 / 2 / 3 / 4 parts
-// ran 184 / 169 / 172 / 177 us a pass, on 512 chunks 1 / 3 / 5 / 8 127 / 95 / 94
-// / 101 us, on 1,292 slabs 1 / 3 / 5 / 8 430 / 386 / 364 / 416 us; two parts at
-// 4,096 chunks or 4,100 mixed items lose 5% and 15%.  `hint` (1..4; 0 = this
-// rule) replaces the rule for the batches it would split.
+// Workgroups per emit item, so that the last round of the 1,280 workgroups
+// that run at once is short without many that only repeat an item's set-up.
+// Edge 16 (700 faces an item, the set-up is most of it): one round, and at
+// most four or a workgroup per CU; emits of 132 / 256 / 400 / 600 / 800 chunks
+// take 15 / 17 / 18 / 19 / 23 us at 4 / 4 / 3 / 2 / 1 parts, against 22 / 21 / 24 /
+// 25 / 31 at the rule of edge 32.  Edge 32: kEmitGrid workgroups, at most 15
+// parts (512 chunks at 1 / 3 / 5 / 8 parts 127 / 95 / 94 / 101 us a pass), three up
+// to kEmitThree (1,640 chunks whose faces differ much at 1 / 2 / 3 / 4 parts
+// 184 / 169 / 172 / 177, alike ones 308 / 319 / 307), one beyond (1,980 alike ones
+// 353 / 374 / 353, 2,450 424 / 463 / 429).  Slabs of 64^3 chunks hold more faces:
+// kEmitGrid64 (1,292 slabs at 1 / 3 / 5 / 8 parts 430 / 386 / 364 / 416); one at
+// kEmitGrid items or more (two at 4,100 mixed items lose 15%).  Odd numbers:
+// workgroups go round the 8 XCDs, and an even number puts the same parts and
+// slabs, which are not alike, on the same ones (1,600 slabs at 2 / 3 / 4 parts
+// 347 / 304 / 346).  `hint` (1..4; 0 = this rule) replaces the rule below
+// kEmitGrid items.
 inline int emit_parts_for(int32_t items, int32_t max_edge, int32_t hint = 0) {
     if (items >= kEmitGrid) return 1;
     if (hint > 0) return hint;
+    if (max_edge <= 16) {
+        const int round = kEmitGrid / 2 / items, cus = 256 / items, most = cus > 4 ? cus : 4;
+        return round < 1 ? 1 : round < most ? round : most;
+    }
+    if (max_edge <= 32 && 2 * items >= kEmitGrid) return items < kEmitThree ? 3 : 1;
     const int p = ((max_edge > 32 ? kEmitGrid64 : kEmitGrid) + items - 1) / items;
-    return p < 16 ? p : 16;
+    return p < 16 ? (p - 1) | 1 : 15;
 }
 // parts_hint: fill_parts_for's hint.  kinds: which chunks the work holds
 // (kFillFast: a FillWork.variant set, kFillGeneral: 0): a kernel for each.
