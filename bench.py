@@ -565,7 +565,8 @@ def main():
     stages = {
         "fill": {"ms": round(float(stage_ms[0]), 4),
                  "GB/s": round(fill_bytes / (stage_ms[0] * 1e-3) / 1e9, 1),
-                 "TFLOP/s": round(fill_flops / (stage_ms[0] * 1e-3) / 1e12, 2)},
+                 "TFLOP/s": round(fill_flops / (stage_ms[0] * 1e-3) / 1e12, 2),
+                 "TFLOP/s_counts": "the restated noise's operations; the kernel executes fewer"},
         "count": {"ms": round(float(stage_ms[1]), 4)},
         "scan": {"ms": round(float(stage_ms[2]), 4)},
         "emit": {"ms": round(float(stage_ms[3]), 4),
@@ -593,16 +594,14 @@ def main():
                 "ms": round(k_ms, 4), "hbm_GB/s": round(f_gbs, 1),
                 "hbm_frac": round(f_gbs / HBM_PEAK_GBS, 4)}
     elif stage_ms[0] >= stage_ms[3]:
-        ach = fill_flops / (stage_ms[0] * 1e-3) / 1e12
-        roof = {"kernel": "fill_kernel<32> (noise+fill)", "bound": "valu", "achieved": round(ach, 2),
-                "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(ach / FP32_PEAK_TFLOPS, 4),
-                "traffic": measured_traffic("fill_kernel<32>", total_faces),
+        # executed VALU stream against the SIMDs' issue rate (the restated
+        # noise's operations are more than the kernel executes)
+        vi = measured_counter("fill_fast_kernel<32>", total_faces, "valu_insts")
+        ach = vi * 64 / (stage_ms[0] * 1e-3) / 1e12 if vi else 0.0
+        roof = {"kernel": "fill_fast_kernel<32> (noise+fill)", "bound": "valu", "achieved": round(ach, 2),
+                "peak": VALU_LANE_OPS_T, "unit": "T lane-ops/s", "frac": round(ach / VALU_LANE_OPS_T, 4),
+                "traffic": measured_traffic("fill_fast_kernel<32>", total_faces),
                 "ms": round(float(stage_ms[0]), 4)}
-        vi = measured_counter("fill_kernel<32>", total_faces, "valu_insts")
-        if vi:  # executed VALU stream against the SIMDs' issue rate
-            lane_ops = vi * 64 / (stage_ms[0] * 1e-3) / 1e12
-            roof["valu_issue"] = {"insts_per_launch": vi, "lane_ops_T_per_s": round(lane_ops, 2),
-                                  "peak": VALU_LANE_OPS_T, "frac": round(lane_ops / VALU_LANE_OPS_T, 4)}
     else:
         ach = emit_bytes / (stage_ms[3] * 1e-3) / 1e9
         roof = {"kernel": "emit_kernel<32> (cull+compact+emit)", "bound": "hbm",
@@ -614,7 +613,7 @@ def main():
         roof["traffic_source"] = ("read from profiles/traffic_uniform4096x32.txt: rocprofv3 "
                                   "FETCH_SIZE + WRITE_SIZE of this kernel on this workload, scaled "
                                   "by a plain copy kernel's counters; not measured in this run")
-    stages["fill"]["traffic"] = measured_traffic("fill_kernel<32>", total_faces)
+    stages["fill"]["traffic"] = measured_traffic("fill_fast_kernel<32>", total_faces)
     stages["emit"]["traffic"] = measured_traffic("emit_kernel<32>", total_faces)
 
     plain = None

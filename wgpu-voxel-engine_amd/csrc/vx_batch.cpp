@@ -186,10 +186,9 @@ hipError_t enqueue_emit(vx_batch *b) {
 }
 
 // The form a run takes.  VX_BATCH_AUTO runs the staged form unless the
-// autotuner chose a persistent form (fused or pipelined) for this batch
-// shape: the plain fused kernel measured as slow or slower than the staged
-// graph at every size, from 64 chunks (0.20 vs 0.21 ms) through a 512-chunk
-// frame with its cull job (0.23 vs 0.24 ms) to 4096 chunks (0.76 vs 1.1 ms).
+// autotuner chose another for this batch shape: at 4096 chunks of 32^3 the
+// staged graph takes 0.40 ms, split 0.43, pipelined 0.71, fused 0.93 (the
+// persistent forms keep the general fill), and smaller batches are alike.
 int form_of(const vx_batch *b) {
     int m = b->mode;
     if (m == VX_BATCH_AUTO) {
