@@ -8,7 +8,8 @@ import voxel_amd as V
 
 pytestmark = pytest.mark.gpu
 
-SIZES = {"16, workgroups": ([16], 37), "16, waves": ([16], 2049), "32, workgroups": ([32], 37),
+SIZES = {"16, workgroups": ([16], 37), "16, fewest waves": ([16], 514), "16, waves": ([16], 2049),
+         "32, workgroups": ([32], 37),
          "32, waves": ([32], 2050), "32 and 16, waves": ([32, 16], 2051), "64": ([64], 9),
          "64, 32 and 16": ([64, 32, 16], 30)}
 

@@ -3035,10 +3035,11 @@ hipError_t launch_count(const MeshWork *work, int32_t n, int32_t max_edge, uint3
                         uint32_t *slabs, uint32_t *clear, const CullJob &cull, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     // a wave per chunk of edge up to 32 where there are enough of them to fill
-    // the chip: 4,096 in 8.2 us, against 10.6 for a workgroup each; 1,640 take
-    // 5.6 either way, 512 gain 0.4 us from the workgroup
+    // the chip: 4,096 of 32^3 in 8.2 us, against 10.6 for a workgroup each; 1,640
+    // take 5.6 either way, 512 gain 0.4 us from the workgroup.  Of 16^3, whose
+    // workgroups mostly read halos, 900 to 1,980 gain 0.2 to 0.5 us a wave each
     constexpr int kWaves = kBlock / 64;
-    const bool wave = max_edge <= 32 && n >= 2048;
+    const bool wave = n >= (max_edge <= 16 ? 512 : 2048) && max_edge <= 32;
     const int grid = (wave ? (n + kWaves - 1) / kWaves : n) + (cull.n > 0 ? (cull.n + kBlock - 1) / kBlock : 0);
     auto launch = [&](auto kernel) {
         kernel<<<grid, kBlock, 0, s>>>(work, counts, max_edge <= 32 ? nullptr : slabs, n, clear, cull);
