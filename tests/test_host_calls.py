@@ -1,0 +1,76 @@
+"""What the library's host code queues, and in which order, without a GPU: its
+HIP calls bind to tests/host_calls/hip_calls.cpp, which logs them.  Each
+scenario runs in a process of its own."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+STUB = os.path.join(ROOT, "tests", "host_calls", "hip_calls.cpp")
+
+PRELUDE = r"""
+import ctypes as C, sys
+hip = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+hip.calls_log.restype = C.c_char_p
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+import voxel_amd as V
+ctx = V.Context(0)
+stream = V.P()
+ctx.check(ctx.L.vx_ctx_stream(ctx.h, C.byref(stream)), "vx_ctx_stream")
+def calls():
+    "The calls since the last look."
+    out = hip.calls_log().decode().split("\n")[:-1]
+    hip.calls_clear()
+    return out
+def terrain(**k):
+    return V.Terrain(**dict(dict(kind=V.TERRAIN_DENSITY, seed=7, octaves=4, frequency=1 / 64,
+                                 lacunarity=2.0, gain=0.5, y_scale=1 / 128), **k))
+def batch(n, edge=32, t=None, **k):
+    return V.Batch(ctx, [(i, 0, 0) for i in range(n)], edge, ctx.terrain(t or terrain()), **k)
+calls()
+"""
+
+
+@pytest.fixture(scope="module")
+def scenario(tmp_path_factory):
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        pytest.skip("no host C++ compiler")
+    so = tmp_path_factory.mktemp("calls") / "hip_calls.so"
+    subprocess.run([cxx, "-std=c++17", "-O1", "-shared", "-fPIC", STUB, "-o", str(so)], check=True)
+
+    def run(code, **env):
+        p = subprocess.run([sys.executable, "-c", PRELUDE + code, str(so),
+                            os.path.join(ROOT, "wgpu-voxel-engine_amd")],
+                           capture_output=True, text=True, timeout=120, env=dict(os.environ, **env))
+        assert p.returncode == 0, p.stdout + p.stderr
+    return run
+
+
+DRAW = r"""
+frustum = V.Frustum(np.eye(4, dtype=np.float32).ravel())
+def draw(n):
+    return ctx.L.vx_frustum_draw_list(ctx.h, C.byref(frustum.c), bufs[0].ptr, bufs[1].ptr, bufs[2].ptr,
+                                      n, 32, V.DRAW_INSTANCED, bufs[3].ptr, bufs[4].ptr)
+bufs = [V.DeviceBuffer(ctx, b) for b in (100000 * 12, 100000 * 4, 100000 * 8, 100000 * 20, 8)]
+"""
+
+
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("warm", [[], [100000]])
+def test_captured_draw_list_records_kernels_only(scenario, mode, warm):
+    """The first list of up to 65,536 meshes may be a captured one, after a
+    longer list or none: nothing is allocated or cleared in its capture."""
+    scenario(DRAW + f"""
+for n in {warm}:
+    assert draw(n) == V.OK
+calls()
+assert hip.hipStreamBeginCapture(stream, {mode}) == 0
+assert draw(4000) == V.OK
+got = [c for c in calls() if c != "hipStreamBeginCapture"]
+assert got and all(c.startswith("captured:draw_") for c in got), got
+""")

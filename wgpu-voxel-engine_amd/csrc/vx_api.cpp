@@ -380,7 +380,8 @@ extern "C" int vx_ctx_create(const vx_ctx_desc *desc, vx_ctx **out) {
     if ((st = c->dev_alloc(sizeof(GradLut), (void **)&c->lut_dev)) ||
         (st = c->dev_alloc(sizeof(MeshTables), (void **)&c->tables_dev)) ||
         (st = c->dev_alloc(kMaxTerrains * sizeof(TerrainDev), (void **)&c->terrains_dev)) ||
-        (st = c->dev_alloc(64, (void **)&c->small_dev))) {
+        (st = c->dev_alloc(64, (void **)&c->small_dev)) ||
+        (st = c->dev_alloc(4 * (size_t)kDrawStateWords, (void **)&c->draw_state))) {
         vx_ctx_destroy(c);
         return st;
     }
@@ -391,6 +392,7 @@ extern "C" int vx_ctx_create(const vx_ctx_desc *desc, vx_ctx **out) {
     }
     if (hipMemcpyAsync(c->lut_dev, &lut, sizeof(lut), hipMemcpyHostToDevice, c->stream) != hipSuccess ||
         hipMemcpyAsync(c->tables_dev, &tabs, sizeof(tabs), hipMemcpyHostToDevice, c->stream) != hipSuccess ||
+        hipMemsetAsync(c->draw_state, 0, 4 * (size_t)kDrawStateWords, c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess) {
         vx_ctx_destroy(c);
         return VX_ERR_DEVICE;
@@ -942,14 +944,8 @@ int vx_draw_list_locked(vx_ctx *ctx, const vx_frustum *f, const int32_t *coords_
     memcpy(P.p, f->planes, sizeof(P.p));
     const int32_t nb = draw_blocks(n);
     if (n <= kDrawOne) {
-        // one launch; its state words are zeroed once (every launch leaves
-        // them zero)
-        if (!ctx->draw_state) {
-            const size_t bytes = 4 * (size_t)kDrawStateWords;
-            int st = ctx->dev_alloc(bytes, (void **)&ctx->draw_state);
-            if (st) return st;
-            VX_HIP(ctx, hipMemsetAsync(ctx->draw_state, 0, bytes, ctx->stream));
-        }
+        // one launch; its state words are zero since the context was made
+        // (every launch leaves them zero)
         VX_HIP(ctx, launch_draw_one(P, coords_dev, faces_dev, first_dev, n, edge, mode, ctx->draw_state,
                                     reinterpret_cast<DrawArgs *>(args_dev), count_dev, ctx->stream));
         return VX_OK;
