@@ -96,3 +96,43 @@ def test_captured_draw_list(ctx):
         hip.hipGraphDestroy(graph)
         for b in bufs + [args, cnt]:
             b.free()
+
+
+def test_captured_draw_list_beside_eager_ones(ctx):
+    """Replays of a captured list on another stream, eager lists of other
+    lengths meanwhile: both stay right, and so do later ones."""
+    hip = C.CDLL("libamdhip64.so.7")
+    s, s2 = V.P(), V.P()
+    ctx.check(ctx.L.vx_ctx_stream(ctx.h, C.byref(s)), "vx_ctx_stream")
+    assert hip.hipStreamCreateWithFlags(C.byref(s2), 1) == 0  # non-blocking
+    n, f = 65536, frustum((0.0, 40.0, 0.0), (0.5, -0.1, 0.7), 900.0)
+    rng = np.random.default_rng(3)
+    coords = np.ascontiguousarray(rng.integers(-30, 30, (n, 3)) * [1, 0, 1], np.int32)
+    faces = rng.integers(0, 900, n).astype(np.uint32)
+    first = np.concatenate([[0], np.cumsum(faces[:-1], dtype=np.uint64)]).astype(np.uint64)
+    mask = f.mask(ctx, coords)
+    want = expected(mask, faces, first, V.DRAW_INSTANCED)
+    bufs = [V.DeviceBuffer.of(ctx, v) for v in (coords, faces, first)]
+    args, cnt = V.DeviceBuffer(ctx, n * 20), V.DeviceBuffer(ctx, 8)
+    graph, ex = V.P(), V.P()
+    assert hip.hipStreamBeginCapture(s, 1) == 0
+    st = ctx.L.vx_frustum_draw_list(ctx.h, C.byref(f.c), bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, n, 32,
+                                    V.DRAW_INSTANCED, args.ptr, cnt.ptr)
+    assert hip.hipStreamEndCapture(s, C.byref(graph)) == 0 and st == V.OK
+    assert hip.hipGraphInstantiate(C.byref(ex), graph, None, None, C.c_size_t(0)) == 0
+    try:
+        for k, m in enumerate((65536, 512, 30000, 65536, 1, 65000, 4096, 65536)):
+            print("[case] replay beside a list of", m, flush=True)
+            for _ in range(3):
+                assert hip.hipGraphLaunch(ex, s2) == 0
+            got = f.draw_list(ctx, coords[:m], faces[:m], first[:m])
+            assert hip.hipStreamSynchronize(s2) == 0
+            assert (got == expected(mask[:m], faces[:m], first[:m], V.DRAW_INSTANCED)).all()
+            assert cnt.download(np.uint32, 2).tolist() == [len(want), 0]
+            assert (args.download(np.uint8, len(want) * 20).view(V.DRAW_DTYPE) == want).all()
+    finally:
+        hip.hipGraphExecDestroy(ex)
+        hip.hipGraphDestroy(graph)
+        hip.hipStreamDestroy(s2)
+        for b in bufs + [args, cnt]:
+            b.free()

@@ -57,6 +57,7 @@ def draw(n):
     return ctx.L.vx_frustum_draw_list(ctx.h, C.byref(frustum.c), bufs[0].ptr, bufs[1].ptr, bufs[2].ptr,
                                       n, 32, V.DRAW_INSTANCED, bufs[3].ptr, bufs[4].ptr)
 bufs = [V.DeviceBuffer(ctx, b) for b in (100000 * 12, 100000 * 4, 100000 * 8, 100000 * 20, 8)]
+calls()
 """
 
 
@@ -73,4 +74,23 @@ assert hip.hipStreamBeginCapture(stream, {mode}) == 0
 assert draw(4000) == V.OK
 got = [c for c in calls() if c != "hipStreamBeginCapture"]
 assert got and all(c.startswith("captured:draw_") for c in got), got
+""")
+
+
+def test_captured_draw_list_keeps_no_state(scenario):
+    """A list queued at once takes one launch, whose status words are that
+    call's own; a captured one, whose replays would share them with later
+    calls, the two passes that overwrite all they read."""
+    scenario(DRAW + """
+for _ in range(2):
+    assert draw(4000) == V.OK
+assert calls() == ["draw_one_kernel 8"] * 2
+assert hip.hipStreamBeginCapture(stream, 1) == 0
+assert draw(4000) == V.OK
+graph = V.P()
+assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+assert calls() == ["hipStreamBeginCapture", "captured:draw_count_kernel 16", "captured:draw_write_kernel 16",
+                   "hipStreamEndCapture"]
+assert draw(4000) == V.OK
+assert calls() == ["draw_one_kernel 8"]
 """)

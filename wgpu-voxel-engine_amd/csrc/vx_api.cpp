@@ -381,10 +381,12 @@ extern "C" int vx_ctx_create(const vx_ctx_desc *desc, vx_ctx **out) {
         (st = c->dev_alloc(sizeof(MeshTables), (void **)&c->tables_dev)) ||
         (st = c->dev_alloc(kMaxTerrains * sizeof(TerrainDev), (void **)&c->terrains_dev)) ||
         (st = c->dev_alloc(64, (void **)&c->small_dev)) ||
-        (st = c->dev_alloc(4 * (size_t)kDrawStateWords, (void **)&c->draw_state))) {
+        (st = c->dev_alloc(8 * (size_t)kDrawStateWords, (void **)&c->draw_state)) ||
+        (st = c->dev_alloc(4 * (size_t)draw_blocks(kDrawOne), (void **)&c->draw_counts))) {
         vx_ctx_destroy(c);
         return st;
     }
+    c->draw_counts_cap = draw_blocks(kDrawOne);
     if (hipHostMalloc((void **)&c->pinned, 4096, hipHostMallocDefault) != hipSuccess) {
         c->pinned = nullptr;
         vx_ctx_destroy(c);
@@ -392,7 +394,7 @@ extern "C" int vx_ctx_create(const vx_ctx_desc *desc, vx_ctx **out) {
     }
     if (hipMemcpyAsync(c->lut_dev, &lut, sizeof(lut), hipMemcpyHostToDevice, c->stream) != hipSuccess ||
         hipMemcpyAsync(c->tables_dev, &tabs, sizeof(tabs), hipMemcpyHostToDevice, c->stream) != hipSuccess ||
-        hipMemsetAsync(c->draw_state, 0, 4 * (size_t)kDrawStateWords, c->stream) != hipSuccess ||
+        hipMemsetAsync(c->draw_state, 0, 8 * (size_t)kDrawStateWords, c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess) {
         vx_ctx_destroy(c);
         return VX_ERR_DEVICE;
@@ -943,11 +945,14 @@ int vx_draw_list_locked(vx_ctx *ctx, const vx_frustum *f, const int32_t *coords_
     Planes P;
     memcpy(P.p, f->planes, sizeof(P.p));
     const int32_t nb = draw_blocks(n);
-    if (n <= kDrawOne) {
-        // one launch; its state words are zero since the context was made
-        // (every launch leaves them zero)
+    // One launch for a short list, unless it is captured: a replay would come
+    // with the tag of its capture, maybe on another stream beside later calls.
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (n <= kDrawOne) VX_HIP(ctx, hipStreamIsCapturing(ctx->stream, &capturing));
+    if (n <= kDrawOne && capturing == hipStreamCaptureStatusNone) {
         VX_HIP(ctx, launch_draw_one(P, coords_dev, faces_dev, first_dev, n, edge, mode, ctx->draw_state,
-                                    reinterpret_cast<DrawArgs *>(args_dev), count_dev, ctx->stream));
+                                    ++ctx->draw_tag, reinterpret_cast<DrawArgs *>(args_dev), count_dev,
+                                    ctx->stream));
         return VX_OK;
     }
     if (nb > ctx->draw_counts_cap) {

@@ -85,7 +85,8 @@ struct vx_ctx {
     hipEvent_t free_fence = nullptr;  // recorded on `stream` at every dev_free
     uint32_t *draw_counts = nullptr;  // per-workgroup counts of draw-list passes
     int32_t draw_counts_cap = 0;
-    uint32_t *draw_state = nullptr;   // state words of one-launch draw lists (zero between launches)
+    uint64_t *draw_state = nullptr;   // status words of one-launch draw lists
+    uint64_t draw_tag = 0;            // one-launch draw lists queued
     uint32_t *draw_scratch = nullptr; // this device's static draw-list scratch
 
     char *stage = nullptr;            // pinned staging of asynchronous uploads (made on first use)

@@ -284,12 +284,14 @@ hipError_t launch_copy(void *dst, const void *src, uint64_t bytes, hipStream_t s
 hipError_t launch_frustum(const Planes &planes, const int32_t *coords, int32_t n, int32_t edge,
                           uint8_t *mask, hipStream_t s);
 // Draw lists of up to kDrawOne meshes can take one launch; `state` holds
-// kDrawStateWords words, zero before the first use and left zero.
+// kDrawStateWords words that no other launch uses at the same time, zero before
+// the first use; `tag` is a number (1 to 2^48 - 1) that no earlier launch on them had.
 constexpr int32_t kDrawOne = 65536;
-constexpr int32_t kDrawStateWords = 1 + kDrawOne / 512;
+constexpr int32_t kDrawStateWords = kDrawOne / 512;
 hipError_t launch_draw_one(const Planes &planes, const int32_t *coords, const uint32_t *faces,
                            const uint64_t *first, int32_t n, int32_t edge, uint32_t mode,
-                           uint32_t *state, DrawArgs *args, uint32_t *count, hipStream_t s);
+                           uint64_t *state, uint64_t tag, DrawArgs *args, uint32_t *count,
+                           hipStream_t s);
 // Workgroups (and block_counts entries) a draw list of n meshes uses.
 int32_t draw_blocks(int32_t n);
 // The draw-list scratch array of the allocation-free entry point: device

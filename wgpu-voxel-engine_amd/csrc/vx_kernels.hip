@@ -2938,60 +2938,71 @@ __global__ void __launch_bounds__(kBlock) draw_write_kernel(Planes planes,
 
 // Both passes in one launch for lists of up to kDrawOne meshes (at most 128
 // workgroups of 512 threads), whose two launches cost more than their work: a
-// workgroup publishes its count, then sums the counts of the workgroups
-// before it as they appear.  state[0] counts finished
-// workgroups (low half) and range errors (high half); the last one reports
-// the errors and clears every word, so that the state is zero between
-// launches, replays of a captured one included.  Waits are only on workgroups
-// dispatched earlier, and bounded: a wait that runs out (state shared by
-// overlapping calls) ends as a range error.
-// 700 / 8,000 / 65,536 meshes: 4.5 / 5.3 / 7.1 us a pass, against 7.8 / 7.8 / 7.7
-// in two launches of one mesh per thread and 8.9 / 10.5 / 10.4 of four; at
-// 200,000 the waits cost more than the launch (12.8 against 7.9).
+// workgroup publishes its count, then sums the counts of the workgroups before
+// it as they appear.  A status word is the call's tag << 16 | kDrawBad if an
+// offset does not fit | the count: one word carries everything a reader needs,
+// so no store has to be ordered with another, and a word of any earlier call
+// has another tag, so none is ever cleared or taken for this call's.  Waits
+// are only on workgroups dispatched earlier, and bounded: where one runs out
+// the thread counts those boxes itself, so the list is right whatever else
+// holds the GPU.
+// 700 / 8,000 / 30,000 / 65,536 meshes: 4.1 / 4.6 / 5.7 / 5.9 us a call, against
+// 6.2 / 6.2 / 6.2 / 6.3 in two launches of one mesh per thread.  The waits grow
+// with the list: 131,072 take 6.2 against 6.4, 262,144 7.2 either way.
+constexpr uint32_t kDrawBad = 0x8000u;
+constexpr uint32_t kDrawSpins = 1u << 14;  // about 10 ms
+static_assert(kDrawOneBlock < (int)kDrawBad && kDrawStateWords * kDrawOneBlock >= kDrawOne &&
+              kDrawStateWords <= kDrawOneBlock, "a thread per earlier workgroup");
+
 __global__ void __launch_bounds__(kDrawOneBlock) draw_one_kernel(Planes planes,
                                                           const int32_t *__restrict__ coords,
                                                           const uint32_t *__restrict__ faces,
                                                           const uint64_t *__restrict__ first,
                                                           int32_t n, int32_t edge, uint32_t mode,
-                                                          uint32_t *__restrict__ state,
+                                                          uint64_t *__restrict__ status, uint64_t tag,
                                                           DrawArgs *__restrict__ args,
                                                           uint32_t *__restrict__ count) {
     __shared__ uint32_t red[kDrawOneBlock / 64];
-    __shared__ uint32_t s_last;
-    uint32_t *status = state + 1;
     const int tid = threadIdx.x, blk = (int)blockIdx.x, i = blk * kDrawOneBlock + tid;
-    const uint32_t vis =
-        i < n ? aabb_visible(planes.p, coords[3 * i], coords[3 * i + 1], coords[3 * i + 2], edge) : 0u;
+    uint32_t vis = 0;
+    bool range = true;
+    DrawArgs a{};
+    if (i < n) {
+        vis = aabb_visible(planes.p, coords[3 * i], coords[3 * i + 1], coords[3 * i + 2], edge);
+        a = draw_args(mode, faces[i], first[i], range);
+    }
     uint32_t total;
     const uint32_t pos = block_exclusive_scan<kDrawOneBlock>(vis, red, &total);
+    const uint32_t own = total | (__syncthreads_or(vis && !range) ? kDrawBad : 0u);
     if (tid == 0)
-        __hip_atomic_store(status + blk, 0x80000000u | total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(status + blk, tag << 16 | own, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     uint32_t before = 0;
-    bool ok = true;
-    for (int j = tid; j < blk; j += kDrawOneBlock) {
-        uint32_t v, spins = 0;
-        while (!((v = __hip_atomic_load(status + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >> 31)) {
-            if (++spins > (1u << 20)) {
-                ok = false;
-                break;
-            }
+    if (tid < blk) {
+        uint64_t v;
+        uint32_t spins = 0;
+        while ((v = __hip_atomic_load(status + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >> 16 !=
+                   tag && spins++ < kDrawSpins)
             __builtin_amdgcn_s_sleep(1);
+        before = (uint32_t)v & 0xFFFFu;
+        if (v >> 16 != tag) {
+            before = 0;
+            bool fits = true;
+            for (int m = tid * kDrawOneBlock; m < (tid + 1) * kDrawOneBlock; m++) {
+                if (!aabb_visible(planes.p, coords[3 * m], coords[3 * m + 1], coords[3 * m + 2], edge))
+                    continue;
+                before++;
+                draw_args(mode, faces[m], first[m], fits);
+            }
+            if (!fits) before |= kDrawBad;
         }
-        before += v & 0x7FFFFFFFu;
     }
+    const bool bad = __syncthreads_or((before | own) & kDrawBad);
     uint32_t off;
-    block_exclusive_scan<kDrawOneBlock>(before, red, &off);
-    if (vis && off + pos < (uint32_t)n) args[off + pos] = draw_args(mode, faces[i], first[i], ok);
-    if (blk == (int)gridDim.x - 1 && tid == 0) count[0] = off + total;
-    const uint32_t bad = __syncthreads_or(!ok) ? 0x10000u : 0u;
-    if (tid == 0) s_last = atomicAdd(state, 1u + bad) + 1u + bad;
-    __syncthreads();
-    if ((s_last & 0xFFFFu) != gridDim.x) return;
-    for (int j = tid; j < (int)gridDim.x; j += kDrawOneBlock)
-        __hip_atomic_store(status + j, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (tid == 0) {
-        __hip_atomic_store(state, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        count[1] = s_last >> 16 ? 1u : 0u;
+    block_exclusive_scan<kDrawOneBlock>(before & (kDrawBad - 1), red, &off);
+    if (vis) args[off + pos] = a;
+    if (blk == (int)gridDim.x - 1 && tid == 0) {
+        count[0] = off + total;
+        count[1] = bad ? 1u : 0u;
     }
 }
 
@@ -3254,11 +3265,12 @@ hipError_t launch_clear_words(uint32_t *p, int32_t n, hipStream_t s) {
 
 hipError_t launch_draw_one(const Planes &planes, const int32_t *coords, const uint32_t *faces,
                            const uint64_t *first, int32_t n, int32_t edge, uint32_t mode,
-                           uint32_t *state, DrawArgs *args, uint32_t *count, hipStream_t s) {
+                           uint64_t *state, uint64_t tag, DrawArgs *args, uint32_t *count,
+                           hipStream_t s) {
     if (n <= 0) return hipSuccess;
     if (n > kDrawOne) return hipErrorInvalidValue;
-    draw_one_kernel<<<(n + kDrawOneBlock - 1) / kDrawOneBlock, kDrawOneBlock, 0, s>>>(planes, coords, faces, first, n, edge, mode, state,
-                                                      args, count);
+    draw_one_kernel<<<(n + kDrawOneBlock - 1) / kDrawOneBlock, kDrawOneBlock, 0, s>>>(
+        planes, coords, faces, first, n, edge, mode, state, tag, args, count);
     return hipGetLastError();
 }
 
