@@ -131,8 +131,9 @@ bool check_schedules() {
     return on;
 }
 
-int form_of(const vx_batch *b);
-
+// emit_order holds what the last scan wrote there: one order of the batch, or
+// after the split form one per half, with indices relative to the half.  A
+// later run in a form without a scan leaves it.
 bool schedules_ok(vx_batch *b) {
     std::vector<int32_t> h((size_t)std::max(b->n, b->n_items));
     auto fetch = [&](const int32_t *a, int32_t m) {
@@ -142,7 +143,7 @@ bool schedules_ok(vx_batch *b) {
     };
     if (b->order_dev && !(fetch(b->order_dev, b->n) && is_schedule(h.data(), b->n))) return false;
     if (!fetch(b->emit_order, b->n_items)) return false;
-    if (form_of(b) == VX_BATCH_SPLIT)  // each half's order, indices relative to the half
+    if (b->order_halves)
         return is_schedule(h.data(), b->split_m) &&
                is_schedule(h.data() + b->split_m, b->n - b->split_m);
     if (!b->slabs) return is_schedule(h.data(), b->n);
@@ -175,6 +176,7 @@ hipError_t enqueue_count(vx_batch *b, const CullJob &cull = CullJob{}) {
                         self_scan(b) ? b->overflow : nullptr, cull, b->ctx->stream);
 }
 hipError_t enqueue_scan(vx_batch *b) {
+    b->order_halves = false;
     return launch_scan(b->counts, b->n, b->slabs ? b->mesh_dev : nullptr, b->bases, b->total,
                        b->overflow, b->emit_order, b->ctx->stream);
 }
@@ -236,6 +238,7 @@ hipError_t enqueue_fused(vx_batch *b) {
 // and emits it, and waits for the second stream before the run ends.  Each
 // half's emission order holds indices relative to the half.
 hipError_t enqueue_split(vx_batch *b) {
+    b->order_halves = true;
     vx_ctx *ctx = b->ctx;
     hipError_t e = hipSuccess;
     if (!ctx->stream2) e = hipStreamCreateWithFlags(&ctx->stream2, hipStreamNonBlocking);
@@ -292,6 +295,13 @@ hipError_t enqueue_all(vx_batch *b) {
     return e;
 }
 
+// Queues a replay of the captured graph (of the form a run takes).
+hipError_t launch_graph(vx_batch *b) {
+    if (form_of(b) == VX_BATCH_SPLIT) b->order_halves = true;
+    else if (!use_fused(b) && !self_scan(b)) b->order_halves = false;
+    return hipGraphLaunch(b->graph_exec, b->ctx->stream);
+}
+
 int ready_form(vx_batch *b);
 
 int capture_graph(vx_batch *b) {
@@ -299,7 +309,9 @@ int capture_graph(vx_batch *b) {
     drop_graph(b);
     if (int st = ready_form(b)) return st;
     VX_HIP(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
+    const bool halves = b->order_halves;
     hipError_t e = enqueue_all(b);
+    b->order_halves = halves;  // nothing has run
     hipGraph_t g = nullptr;
     hipError_t e2 = hipStreamEndCapture(ctx->stream, &g);
     if (e != hipSuccess || e2 != hipSuccess) {
@@ -607,9 +619,8 @@ extern "C" int vx_batch_create_ext(vx_ctx *ctx, const vx_batch_req *reqs, int32_
         }
         memset(up + off_ctl, 0, off_emit - off_ctl);
         if (slabbed) memset(up + off_slabs, 0, desc_bytes - off_slabs);
-        // the scan rewrites the emission order every run; start from a valid
-        // one regardless (chunk indices, or every emit item's code chunk << 2
-        // | slab)
+        // a scan rewrites the emission order; start from a valid one
+        // regardless (chunk indices, or every emit item's code chunk << 2 | slab)
         int32_t *emit = (int32_t *)(up + off_emit);
         for (int i = 0; i < n; i++) {
             if (!b->slabs) *emit++ = i;
@@ -772,7 +783,7 @@ extern "C" int vx_batch_run(vx_ctx *ctx, vx_batch *b) {
     } else {
         if (!b->graph_exec)
             if (int st = capture_graph(b)) return st;
-        VX_HIP(ctx, hipGraphLaunch(b->graph_exec, ctx->stream));
+        VX_HIP(ctx, launch_graph(b));
     }
     b->launched = true;
     b->ran = true;
@@ -1073,10 +1084,10 @@ extern "C" int vx_batch_autotune(vx_ctx *ctx, vx_batch *b, int32_t reps, vx_tune
             b->fill_split = cands[c].fill_split;
             b->emit_split = cands[c].emit_split;
             if ((st = capture_graph(b))) break;
-            hipError_t e = hipGraphLaunch(b->graph_exec, ctx->stream);  // warm-up
+            hipError_t e = launch_graph(b);  // warm-up
             if (e == hipSuccess) e = hipEventRecord(e0, ctx->stream);
             for (int i = 0; i < reps && e == hipSuccess; i++)
-                e = hipGraphLaunch(b->graph_exec, ctx->stream);
+                e = launch_graph(b);
             if (e == hipSuccess) e = hipEventRecord(e1, ctx->stream);
             if (e == hipSuccess) e = hipEventSynchronize(e1);
             if (e != hipSuccess) {
@@ -1183,7 +1194,7 @@ extern "C" int vx_batch_profile(vx_ctx *ctx, vx_batch *b, int32_t reps, float ms
         if (!st) {
             hipError_t e = hipEventRecord(ev[0], ctx->stream);
             for (int r = 0; r < reps && e == hipSuccess; r++)
-                e = hipGraphLaunch(b->graph_exec, ctx->stream);
+                e = launch_graph(b);
             if (e == hipSuccess) e = hipEventRecord(ev[5], ctx->stream);
             if (e == hipSuccess) e = hipEventSynchronize(ev[5]);
             if (e != hipSuccess) {

@@ -154,6 +154,7 @@ struct vx_batch {
     void *desc = nullptr;           // block of the descriptors, the schedules and the control words
     int32_t *coords_dev = nullptr;  // chunk coordinates (draw lists), made on first use
     int32_t *emit_order = nullptr;  // emission order written by the scan (largest first)
+    bool order_halves = false;      // it holds the split form's two orders
     int32_t n_items = 0;            // emit items: n, or with slabs kSlabs per 64^3 chunk
     uint32_t *slabs = nullptr;      // per-slab face counts of 64^3 chunks (null when none)
     uint32_t *counts = nullptr;
