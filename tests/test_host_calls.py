@@ -94,3 +94,23 @@ assert calls() == ["hipStreamBeginCapture", "captured:draw_count_kernel 16", "ca
 assert draw(4000) == V.OK
 assert calls() == ["draw_one_kernel 8"]
 """)
+
+
+@pytest.mark.parametrize("mode", ["STAGED", "SPLIT"])
+@pytest.mark.parametrize("call", ["hipStreamBeginCapture", "hipStreamEndCapture", "hipGraphInstantiate"])
+def test_wait_outlives_a_failed_capture(scenario, mode, call):
+    """A run that succeeded is waited for and its results are returned whether
+    or not the graph of later runs can be captured; the next run tries again."""
+    scenario(f"""
+b = batch(4)
+b.set_mode(V.BATCH_{mode})
+b.run()
+calls()
+hip.calls_fail(b"{call}")
+assert b.wait() == 0
+assert "hipStreamSynchronize" in calls()
+assert b.chunk_faces(3) == (0, 0)
+b.run()
+got = calls()
+assert "hipGraphInstantiate" in got and got[-1] == "hipGraphLaunch", got
+""")

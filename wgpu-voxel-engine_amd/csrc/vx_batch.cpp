@@ -818,8 +818,9 @@ extern "C" int vx_batch_wait(vx_ctx *ctx, vx_batch *b, uint64_t *total_faces) {
     if (!b->ran) return VX_ERR_NOT_READY;
     // total | overflow, schedule error: 16 contiguous bytes
     VX_HIP(ctx, hipMemcpyAsync(ctx->pinned, b->total, 16, hipMemcpyDeviceToHost, ctx->stream));
-    if (!b->graph_exec && b->launched)
-        if (int st = capture_graph(b)) return st;  // beside the first run
+    // the graph of later runs, beside the first; if that fails, the run is
+    // still waited for, and the next tries again and reports it
+    if (!b->graph_exec && b->launched) (void)capture_graph(b);
     VX_HIP(ctx, hipStreamSynchronize(ctx->stream));
     uint32_t sched_err;
     memcpy(&sched_err, ctx->pinned + 12, 4);
