@@ -19,6 +19,7 @@ constexpr int kOk = 0, kFailed = 999, kUnsupported = 900;
 std::string g_log, g_fail;
 std::map<const void *, std::string> g_kernels;
 void *g_capturing = nullptr;  // the capturing stream
+void *g_captured = nullptr;   // the last that was
 int g_capture_mode = 0;
 Dim3 g_grid, g_block;
 size_t g_shared;
@@ -44,6 +45,7 @@ extern "C" {
 const char *calls_log() { return g_log.c_str(); }
 void calls_clear() { g_log.clear(); }
 void calls_fail(const char *name) { g_fail = name; }  // the next call of that name fails
+void *calls_capture_stream() { return g_captured; }
 
 // ---- HIP
 int hipGetDeviceCount(int *n) { return *n = 1, kOk; }
@@ -88,7 +90,7 @@ int hipEventSynchronize(void *) { return call("hipEventSynchronize") ? kFailed :
 int hipEventElapsedTime(float *ms, void *, void *) { return *ms = 1.0f, kOk; }
 int hipStreamBeginCapture(void *s, int mode) {
     if (call("hipStreamBeginCapture") || g_capturing) return kFailed;
-    g_capturing = s;
+    g_capturing = g_captured = s;
     g_capture_mode = mode;
     return kOk;
 }

@@ -114,3 +114,32 @@ b.run()
 got = calls()
 assert "hipGraphInstantiate" in got and got[-1] == "hipGraphLaunch", got
 """)
+
+
+def test_graphs_are_captured_on_a_private_stream(scenario):
+    """A caller, or another thread, may queue work on the context's stream at
+    any moment: no call captures that stream."""
+    scenario("""
+hip.calls_capture_stream.restype = C.c_void_p
+for mode in (V.BATCH_STAGED, V.BATCH_SPLIT):
+    b = batch(4)
+    b.set_mode(mode)
+    b.run()
+    b.wait()
+    assert hip.calls_capture_stream() not in (None, stream.value)
+    got = [c for c in calls() if c.startswith("captured:")]
+    assert any("emit_kernel" in c for c in got)
+# and a run in the caller's own capture records work, with a graph or without
+for runs in (0, 1, 2):
+    b = batch(4)
+    for _ in range(runs):
+        b.run()
+        b.wait()
+    calls()
+    assert hip.hipStreamBeginCapture(stream, 1) == 0
+    b.run()
+    graph = V.P()
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    got = calls()[1:-1]
+    assert got and all(c.startswith("captured:") for c in got), (runs, got)
+""")

@@ -412,6 +412,7 @@ extern "C" int vx_ctx_destroy(vx_ctx *ctx) {
     if (ctx->stage_ev) (void)hipEventDestroy(ctx->stage_ev);
     if (ctx->free_fence) (void)hipEventDestroy(ctx->free_fence);
     if (ctx->stream2) (void)hipStreamDestroy(ctx->stream2);
+    if (ctx->capture_stream) (void)hipStreamDestroy(ctx->capture_stream);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;  // DeviceHeap frees every device block
     return VX_OK;

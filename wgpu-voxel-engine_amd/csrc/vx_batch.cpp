@@ -163,28 +163,28 @@ int32_t emit_split_of(const vx_batch *b) {
     return tuned_auto(b) ? b->tuned_emit_split : b->emit_split;
 }
 
-hipError_t enqueue_fill(vx_batch *b) {
+hipError_t enqueue_fill(vx_batch *b, hipStream_t s) {
     vx_ctx *ctx = b->ctx;
     return launch_fill(b->fill_dev, b->order_dev, b->n, b->max_edge, ctx->terrains_dev,
-                       ctx->lut_dev, b->overflow + 1, fill_split_of(b), b->fill_kinds, ctx->stream);
+                       ctx->lut_dev, b->overflow + 1, fill_split_of(b), b->fill_kinds, s);
 }
 // Batches of few chunks have no scan: the emit sums the counts itself.
 bool self_scan(const vx_batch *b) { return b->n <= kSelfScan && !b->fill_counts; }
 
-hipError_t enqueue_count(vx_batch *b, const CullJob &cull = CullJob{}) {
+hipError_t enqueue_count(vx_batch *b, const CullJob &cull, hipStream_t s) {
     return launch_count(b->mesh_dev, b->n, b->max_edge, b->counts, b->slabs,
-                        self_scan(b) ? b->overflow : nullptr, cull, b->ctx->stream);
+                        self_scan(b) ? b->overflow : nullptr, cull, s);
 }
-hipError_t enqueue_scan(vx_batch *b) {
+hipError_t enqueue_scan(vx_batch *b, hipStream_t s) {
     b->order_halves = false;
     return launch_scan(b->counts, b->n, b->slabs ? b->mesh_dev : nullptr, b->bases, b->total,
-                       b->overflow, b->emit_order, b->ctx->stream);
+                       b->overflow, b->emit_order, s);
 }
-hipError_t enqueue_emit(vx_batch *b) {
+hipError_t enqueue_emit(vx_batch *b, hipStream_t s) {
     const bool self = self_scan(b);
     return launch_emit(b->mesh_dev, self ? nullptr : b->emit_order, b->n, b->n_items, b->max_edge,
                        b->bases, b->counts, b->slabs, b->out, b->ctx->tables_dev, b->overflow,
-                       emit_split_of(b), self ? b->total : nullptr, b->ctx->stream);
+                       emit_split_of(b), self ? b->total : nullptr, s);
 }
 
 // The form a run takes.  VX_BATCH_AUTO runs the staged form unless the
@@ -217,33 +217,32 @@ int32_t pipe_ratio_of(const vx_batch *b) {
     return b->mode == VX_BATCH_AUTO && b->tuned ? b->tuned_ratio : b->pipe_ratio;
 }
 
-hipError_t enqueue_fused(vx_batch *b) {
+hipError_t enqueue_fused(vx_batch *b, hipStream_t s) {
     vx_ctx *ctx = b->ctx;
     if (form_of(b) == VX_BATCH_PIPELINED)
         return launch_pipe(b->fused_dev, b->n, b->max_edge, b->pipe_lag, ctx->terrains_dev,
                            ctx->lut_dev,
                            ctx->tables_dev, b->fctl_ptrs, b->out, b->cull, fused_grid_of(b),
-                           pipe_ratio_of(b), ctx->stream);
+                           pipe_ratio_of(b), s);
     return launch_fused(b->fused_dev, b->n, b->max_edge, ctx->terrains_dev, ctx->lut_dev,
-                        ctx->tables_dev, b->fctl_ptrs, b->out, b->cull, fused_grid_of(b),
-                        ctx->stream);
+                        ctx->tables_dev, b->fctl_ptrs, b->out, b->cull, fused_grid_of(b), s);
 }
 
-// The split form: the staged kernels over two halves on two streams.  The
-// context stream fills chunks [0, m2) (the first half [0, m) and the later
-// chunks its counts read planes of) and then [m2, n) back to back, so the
-// fills stay on one queue; the second stream counts, scans and emits the
-// first half as soon as its fill is out, beside the second fill.  The
-// context stream then counts [m, n), scans it from the first half's total
-// and emits it, and waits for the second stream before the run ends.  Each
-// half's emission order holds indices relative to the half.
-hipError_t enqueue_split(vx_batch *b) {
+// The split form: the staged kernels over two halves on two streams.  Stream
+// s0 fills chunks [0, m2) (the first half [0, m) and the later chunks its
+// counts read planes of) and then [m2, n) back to back, so the fills stay on
+// one queue; the second stream counts, scans and emits the first half as soon
+// as its fill is out, beside the second fill.  Stream s0 then counts [m, n),
+// scans it from the first half's total and emits it, and waits for the second
+// stream before the run ends.  Each half's emission order holds indices
+// relative to the half.
+hipError_t enqueue_split(vx_batch *b, hipStream_t s0) {
     b->order_halves = true;
     vx_ctx *ctx = b->ctx;
     hipError_t e = hipSuccess;
     if (!ctx->stream2) e = hipStreamCreateWithFlags(&ctx->stream2, hipStreamNonBlocking);
     if (e != hipSuccess) return e;
-    hipStream_t s0 = ctx->stream, s1 = ctx->stream2;
+    hipStream_t s1 = ctx->stream2;
     const int32_t n = b->n, m = b->split_m, m2 = b->split_m2;
     const int32_t fs = fill_split_of(b), es = emit_split_of(b);
     e = launch_cull(b->cull, s0);
@@ -263,7 +262,7 @@ hipError_t enqueue_split(vx_batch *b) {
         e = launch_emit(b->mesh_dev, b->emit_order, m, m, b->max_edge, b->bases, b->counts,
                         nullptr, b->out, ctx->tables_dev, b->overflow, es, nullptr, s1);
     if (e == hipSuccess) e = hipEventRecord(b->split_ev[2], s1);
-    // second half on the context stream
+    // second half on s0
     if (e == hipSuccess)
         e = launch_fill(b->fill_dev + m2, nullptr, n - m2, b->max_edge, ctx->terrains_dev,
                         ctx->lut_dev, b->overflow + 1, fs, b->fill_kinds, s0);
@@ -283,15 +282,15 @@ hipError_t enqueue_split(vx_batch *b) {
     return e;
 }
 
-hipError_t enqueue_all(vx_batch *b) {
-    if (use_fused(b)) return enqueue_fused(b);
-    if (form_of(b) == VX_BATCH_SPLIT) return enqueue_split(b);
+hipError_t enqueue_all(vx_batch *b, hipStream_t s) {
+    if (use_fused(b)) return enqueue_fused(b, s);
+    if (form_of(b) == VX_BATCH_SPLIT) return enqueue_split(b, s);
     // the cull runs beside the count, or alone when the fill counts
-    hipError_t e = b->fill_counts ? launch_cull(b->cull, b->ctx->stream) : hipSuccess;
-    if (e == hipSuccess) e = enqueue_fill(b);
-    if (e == hipSuccess && !b->fill_counts) e = enqueue_count(b, b->cull);
-    if (e == hipSuccess && !self_scan(b)) e = enqueue_scan(b);
-    if (e == hipSuccess) e = enqueue_emit(b);
+    hipError_t e = b->fill_counts ? launch_cull(b->cull, s) : hipSuccess;
+    if (e == hipSuccess) e = enqueue_fill(b, s);
+    if (e == hipSuccess && !b->fill_counts) e = enqueue_count(b, b->cull, s);
+    if (e == hipSuccess && !self_scan(b)) e = enqueue_scan(b, s);
+    if (e == hipSuccess) e = enqueue_emit(b, s);
     return e;
 }
 
@@ -304,16 +303,20 @@ hipError_t launch_graph(vx_batch *b) {
 
 int ready_form(vx_batch *b);
 
+// Captures a run on a stream of its own: the context's is the caller's too
+// (vx_ctx_stream), whose work would land in the graph.
 int capture_graph(vx_batch *b) {
     vx_ctx *ctx = b->ctx;
     drop_graph(b);
     if (int st = ready_form(b)) return st;
-    VX_HIP(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
+    if (!ctx->capture_stream)
+        VX_HIP(ctx, hipStreamCreateWithFlags(&ctx->capture_stream, hipStreamNonBlocking));
+    VX_HIP(ctx, hipStreamBeginCapture(ctx->capture_stream, hipStreamCaptureModeThreadLocal));
     const bool halves = b->order_halves;
-    hipError_t e = enqueue_all(b);
+    hipError_t e = enqueue_all(b, ctx->capture_stream);
     b->order_halves = halves;  // nothing has run
     hipGraph_t g = nullptr;
-    hipError_t e2 = hipStreamEndCapture(ctx->stream, &g);
+    hipError_t e2 = hipStreamEndCapture(ctx->capture_stream, &g);
     if (e != hipSuccess || e2 != hipSuccess) {
         if (g) (void)hipGraphDestroy(g);
         ctx->set_error(e != hipSuccess ? e : e2, "batch graph capture");
@@ -779,7 +782,7 @@ extern "C" int vx_batch_run(vx_ctx *ctx, vx_batch *b) {
         // the first run launches the kernels themselves; the graph is captured
         // while the GPU works on them (vx_batch_wait), or by the second run
         if (int st = ready_form(b)) return st;
-        VX_HIP(ctx, enqueue_all(b));
+        VX_HIP(ctx, enqueue_all(b, ctx->stream));
     } else {
         if (!b->graph_exec)
             if (int st = capture_graph(b)) return st;
@@ -802,7 +805,7 @@ extern "C" int vx_batch_run_per_chunk(vx_ctx *ctx, vx_batch *b) {
     for (int i = 0; i < n; i++)
         VX_HIP(ctx, launch_count(b->mesh_dev + i, 1, b->reqs[i].edge, b->counts + i, slabs_of(i),
                                  nullptr, CullJob{}, ctx->stream));
-    VX_HIP(ctx, enqueue_scan(b));
+    VX_HIP(ctx, enqueue_scan(b, ctx->stream));
     for (int i = 0; i < n; i++)
         VX_HIP(ctx, launch_emit(b->mesh_dev + i, nullptr, 1, 0, b->reqs[i].edge, b->bases + i,
                                 b->counts + i, slabs_of(i), b->out, ctx->tables_dev, b->overflow,
@@ -859,9 +862,9 @@ extern "C" int vx_batch_wait(vx_ctx *ctx, vx_batch *b, uint64_t *total_faces) {
         }
         // a persistent form writes no slab counts: count again first; without
         // a scan it is the count that clears the overflow word
-        if (b->slabs || self_scan(b)) VX_HIP(ctx, enqueue_count(b));
-        if (!self_scan(b)) VX_HIP(ctx, enqueue_scan(b));
-        VX_HIP(ctx, enqueue_emit(b));
+        if (b->slabs || self_scan(b)) VX_HIP(ctx, enqueue_count(b, CullJob{}, ctx->stream));
+        if (!self_scan(b)) VX_HIP(ctx, enqueue_scan(b, ctx->stream));
+        VX_HIP(ctx, enqueue_emit(b, ctx->stream));
         VX_HIP(ctx, hipMemcpyAsync(ctx->pinned + 8, b->overflow, 8, hipMemcpyDeviceToHost,
                                    ctx->stream));
         VX_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -1156,7 +1159,7 @@ extern "C" int vx_batch_profile(vx_ctx *ctx, vx_batch *b, int32_t reps, float ms
     for (int r = 0; r < reps && !st && whole; r++) {
         if ((st = ready_form(b))) break;
         hipError_t e = hipEventRecord(ev[0], ctx->stream);
-        if (e == hipSuccess) e = enqueue_all(b);
+        if (e == hipSuccess) e = enqueue_all(b, ctx->stream);
         if (e == hipSuccess) e = hipEventRecord(ev[1], ctx->stream);
         if (e == hipSuccess) e = hipEventSynchronize(ev[1]);
         if (e != hipSuccess) {
@@ -1170,13 +1173,13 @@ extern "C" int vx_batch_profile(vx_ctx *ctx, vx_batch *b, int32_t reps, float ms
     }
     for (int r = 0; r < reps && !st && !whole; r++) {
         hipError_t e = hipEventRecord(ev[0], ctx->stream);
-        if (e == hipSuccess) e = enqueue_fill(b);
+        if (e == hipSuccess) e = enqueue_fill(b, ctx->stream);
         if (e == hipSuccess) e = hipEventRecord(ev[1], ctx->stream);
-        if (e == hipSuccess && !b->fill_counts) e = enqueue_count(b);
+        if (e == hipSuccess && !b->fill_counts) e = enqueue_count(b, CullJob{}, ctx->stream);
         if (e == hipSuccess) e = hipEventRecord(ev[2], ctx->stream);
-        if (e == hipSuccess && !self_scan(b)) e = enqueue_scan(b);
+        if (e == hipSuccess && !self_scan(b)) e = enqueue_scan(b, ctx->stream);
         if (e == hipSuccess) e = hipEventRecord(ev[3], ctx->stream);
-        if (e == hipSuccess) e = enqueue_emit(b);
+        if (e == hipSuccess) e = enqueue_emit(b, ctx->stream);
         if (e == hipSuccess) e = hipEventRecord(ev[4], ctx->stream);
         if (e == hipSuccess) e = hipEventSynchronize(ev[4]);
         if (e != hipSuccess) {

@@ -69,6 +69,7 @@ inline bool coord_in_range(vx_coord c, int32_t edge) {
 struct vx_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
+    hipStream_t capture_stream = nullptr;  // captures batch graphs, runs nothing (made on first use)
     hipStream_t stream2 = nullptr;  // second branch of split-batch runs (made on first use)
     std::recursive_mutex mu;
     uint64_t budget = 0;
