@@ -20,6 +20,7 @@ std::string g_log, g_fail;
 std::map<const void *, std::string> g_kernels;
 void *g_capturing = nullptr;  // the capturing stream
 void *g_captured = nullptr;   // the last that was
+void *g_synced = nullptr;     // the last stream waited for
 int g_capture_mode = 0;
 Dim3 g_grid, g_block;
 size_t g_shared;
@@ -46,6 +47,7 @@ const char *calls_log() { return g_log.c_str(); }
 void calls_clear() { g_log.clear(); }
 void calls_fail(const char *name) { g_fail = name; }  // the next call of that name fails
 void *calls_capture_stream() { return g_captured; }
+void *calls_synced_stream() { return g_synced; }
 
 // ---- HIP
 int hipGetDeviceCount(int *n) { return *n = 1, kOk; }
@@ -77,6 +79,7 @@ int hipMemsetAsync(void *d, int v, size_t n, void *st) {
 int hipStreamCreateWithFlags(void **s, unsigned) { return make(s); }
 int hipStreamDestroy(void *) { return kOk; }
 int hipStreamSynchronize(void *s) {
+    g_synced = s;
     if (call("hipStreamSynchronize", s)) return kFailed;
     return captured(s) ? kUnsupported : kOk;
 }

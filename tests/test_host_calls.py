@@ -143,3 +143,38 @@ for runs in (0, 1, 2):
     got = calls()[1:-1]
     assert got and all(c.startswith("captured:") for c in got), (runs, got)
 """)
+
+
+@pytest.mark.parametrize("use", ["create_mesh", "neighbour", "ids", "occupancy"])
+def test_chunk_of_another_context_is_waited_for(scenario, use):
+    """A chunk made in one context and used through another: its pack or fill
+    runs on the first one's stream, so the call waits for that first; within a
+    context the stream orders them."""
+    scenario(f"""
+other = V.Context(0)
+hip.calls_synced_stream.restype = C.c_void_p
+chunk = V.Chunk.from_ids(ctx, (0, 0, 0), 32, np.ones(32 ** 3, np.uint8))
+mine = V.Chunk.from_ids(other, (1, 0, 0), 32, np.ones(32 ** 3, np.uint8))
+def use(c):
+    if "{use}" == "create_mesh":
+        c.create_mesh()
+    elif "{use}" == "neighbour":
+        mine.create_mesh((c, None, None, None))
+    else:
+        getattr(c, "{use}")()
+seen = []
+def sync_first(c):
+    calls()
+    hip.calls_fail(b"hipStreamSynchronize")  # ends the call at its first wait
+    try:
+        use(c)
+        assert False
+    except V.VoxelError:
+        pass
+    return calls()[0] == "hipStreamSynchronize" and hip.calls_synced_stream() == stream.value
+foreign = V.Chunk(other, chunk.h)  # the same chunk through the other context
+assert sync_first(foreign)
+foreign.h = None
+if "{use}" != "neighbour":
+    assert not sync_first(chunk)
+""")

@@ -683,11 +683,18 @@ extern "C" int vx_chunk_info(const vx_chunk *c, vx_coord *coord, int32_t *edge) 
     return VX_OK;
 }
 
+// A chunk of another context may still be filled or packed on that context's
+// stream, which this one's does not follow.
+static hipError_t chunk_ready(const vx_ctx *ctx, const vx_chunk *c) {
+    return !c || c->ctx == ctx ? hipSuccess : hipStreamSynchronize(c->ctx->stream);
+}
+
 extern "C" int vx_chunk_read_ids(vx_ctx *ctx, const vx_chunk *c, uint8_t *dst, uint64_t cap) {
     if (!ctx || !c || !dst) return VX_ERR_INVALID;
     const uint64_t n = (uint64_t)c->edge * c->edge * c->edge;
     if (cap < n) return VX_ERR_CAPACITY;
     std::lock_guard<std::recursive_mutex> g(ctx->mu);
+    VX_HIP(ctx, chunk_ready(ctx, c));
     VX_HIP(ctx, hipMemcpyAsync(dst, c->ids, n, hipMemcpyDeviceToHost, ctx->stream));
     VX_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return VX_OK;
@@ -699,6 +706,7 @@ extern "C" int vx_chunk_read_occupancy(vx_ctx *ctx, const vx_chunk *c, uint32_t 
     const uint64_t n = (uint64_t)c->edge * c->edge * words_per_row(c->edge);
     if (cap_words < n) return VX_ERR_CAPACITY;
     std::lock_guard<std::recursive_mutex> g(ctx->mu);
+    VX_HIP(ctx, chunk_ready(ctx, c));
     VX_HIP(ctx, hipMemcpyAsync(dst, c->occ, n * 4, hipMemcpyDeviceToHost, ctx->stream));
     VX_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return VX_OK;
@@ -787,6 +795,8 @@ extern "C" int vx_chunk_create_mesh(vx_ctx *ctx, vx_chunk *chunk, vx_chunk *cons
         for (int k = 0; k < 4; k++)
             if (adj[k] && adj[k]->edge != chunk->edge) return VX_ERR_INVALID;
     std::lock_guard<std::recursive_mutex> g(ctx->mu);
+    VX_HIP(ctx, chunk_ready(ctx, chunk));
+    for (int k = 0; adj && k < 4; k++) VX_HIP(ctx, chunk_ready(ctx, adj[k]));
     const MeshWork w = mesh_work_of(chunk, adj);
     uint32_t *count_dev = (uint32_t *)ctx->small_dev;
     uint32_t *slabs_dev = count_dev + 4;
