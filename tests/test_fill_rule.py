@@ -164,3 +164,51 @@ def test_error_bound(octaves):
         eps = (48 + 8 * octaves) * 2.0 ** -24 * float(mag)
         err = np.abs(acc.astype(np.float64) - exact).max()
         assert err <= eps, (gain, err, eps)
+
+
+PAYS = r"""
+#include <cstdio>
+#include "vx_fill_rule.h"
+int main() {
+    int o, z, e, m, n;
+    float f, l;
+    while (scanf("%d %f %f %d %d %d %d", &o, &f, &l, &z, &e, &m, &n) == 7)
+        printf("%d\n", vx::fast_pays(o, f, l, z != 0, e, m, n));
+}
+"""
+
+
+def test_batches_that_gain(tmp_path):
+    """Where a batch's chunks leave the fast fill because the general kernels
+    are faster: fine octaves, a zero threshold on lattice planes, small batches
+    of 16^3; and the tuned terrains, which stay."""
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        pytest.skip("no host C++ compiler")
+    (tmp_path / "p.cpp").write_text(PAYS)
+    subprocess.run([cxx, "-std=c++17", "-O1", "-ffp-contract=off", "-I", CSRC, str(tmp_path / "p.cpp"),
+                    "-o", str(tmp_path / "p")], check=True)
+    cases = [  # octaves, frequency, lacunarity, zero threshold, edge, largest edge, chunks -> gains
+        (4, 1 / 64, 2.0, 0, 32, 32, 4096, 1), (3, 0.09, 0.5, 1, 32, 32, 1640, 1), (4, 1 / 64, 2.0, 0, 64, 64, 323, 1),
+        (6, 0.01, 2.0, 0, 32, 32, 1023, 1), (6, 1 / 64, 2.0, 1, 16, 16, 4, 1), (1, 0.09, 2.0, 1, 32, 32, 256, 1),
+        # the finest octave
+        (1, 0.32, 2.0, 0, 32, 32, 256, 1), (1, 0.33, 2.0, 0, 32, 32, 256, 0), (3, 0.125, 2.0, 0, 32, 32, 256, 0),
+        (3, 0.09, 2.0, 0, 32, 32, 511, 0), (3, 0.09, 2.0, 0, 32, 32, 512, 1),
+        (4, 0.055, 2.0, 0, 32, 32, 1023, 1), (4, 0.055, 2.0, 0, 32, 32, 1024, 0), (4, 0.0625, 2.0, 0, 32, 32, 256, 0),
+        (4, 0.0625, 2.0, 0, 64, 64, 64, 0), (1, 0.45, 2.0, 0, 64, 64, 16, 1), (1, 0.45, 2.0, 0, 64, 64, 17, 0),
+        (2, 0.225, 2.0, 0, 64, 64, 323, 1), (2, 0.25, 2.0, 0, 64, 64, 8, 0),
+        (2, 0.2, 2.0, 0, 64, 64, 64, 1), (3, 0.6, 0.5, 0, 64, 64, 64, 0), (5, 1 / 32, 2.0, 0, 64, 64, 64, 1),
+        # zero thresholds
+        (1, 0.125, 2.0, 1, 32, 32, 1024, 0), (1, 1 / 64, 2.0, 1, 64, 64, 64, 0), (1, 1e-5, 2.0, 1, 32, 32, 256, 0),
+        (2, 0.05, 2.0, 1, 32, 32, 256, 1), (2, 0.0625, 2.0, 1, 32, 32, 1023, 0), (2, 0.0625, 2.0, 1, 32, 32, 1024, 1),
+        (2, 0.0625, 2.0, 1, 64, 64, 256, 1), (1, 0.35, 2.0, 1, 64, 64, 64, 0), (1, 0.3217, 2.0, 1, 64, 64, 64, 1),
+        (6, 3e-7, 2.0, 1, 32, 32, 64, 0),
+        (2, 0.0625, 1.9, 1, 32, 32, 256, 1), (3, 0.0625, 2.0, 1, 32, 32, 256, 1),
+        # 16^3 chunks, alone and beside larger ones
+        (3, 1 / 64, 2.0, 0, 16, 16, 383, 0), (3, 1 / 64, 2.0, 0, 16, 16, 384, 1), (3, 1 / 64, 2.0, 0, 16, 32, 64, 1),
+        (1, 1 / 64, 2.0, 0, 16, 16, 4000, 0), (3, 1 / 64, 2.0, 1, 16, 16, 4000, 0), (3, 0.013, 1.9, 1, 16, 16, 512, 1),
+        (4, 1 / 64, 2.0, 1, 16, 16, 1023, 0), (4, 1 / 64, 2.0, 1, 16, 16, 1024, 1),
+    ]
+    text = "\n".join(" ".join(repr(float(v)) if isinstance(v, float) else str(v) for v in c[:-1]) for c in cases)
+    out = subprocess.run([str(tmp_path / "p")], input=text, capture_output=True, text=True, check=True)
+    assert [int(v) for v in out.stdout.split()] == [c[-1] for c in cases]

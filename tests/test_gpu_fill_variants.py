@@ -123,3 +123,26 @@ def test_tiles_beside_64(ctx, oracle_mod, kind, n):
         ch.release()
         assert b.chunk_faces(i)[1] == len(oracle_mod.mesh_buffers(ref, edges[i], (0, 0, 0), [None] * 4)[0]), i
     b.close()
+
+
+@pytest.mark.parametrize("n", [383, 384])
+@pytest.mark.parametrize("name", ["16^3", "beside larger"])
+def test_batch_rule(ctx, oracle_mod, name, n):
+    """Batches on both sides of the rule that sends chunks to the general
+    kernels: 16^3 chunks by their number, in larger batches each terrain by its
+    finest octave, both kernels on one batch."""
+    ts = [dens(octaves=3, frequency=1 / 60), dens(octaves=3, frequency=1 / 6), dens(octaves=1, frequency=0.25, y_scale=0.0),
+          dens(octaves=6, frequency=1 / 80)]
+    ots = [oracle_terrain(oracle_mod, t) for t in ts]
+    edges = [16 if name == "16^3" else (16, 32)[i % 2] for i in range(n)]
+    coords = [(i % 23 - 11, 0, i // 23) for i in range(n)]
+    b = V.Batch(ctx, coords, edges, [ctx.terrain(ts[i % 4]) for i in range(n)])
+    for splits in ((0, 0), (2, 1)):
+        b.set_splits(*splits)
+        b.run()
+        b.wait()
+        for i in list(range(8)) + [n // 2, n // 2 + 1, n - 2, n - 1]:
+            ref = oracle_mod.chunk_fill(ots[i % 4], *coords[i], edges[i])
+            assert (b.ids(i) == ref).all(), (i, splits)
+            assert b.chunk_faces(i)[1] == len(oracle_mod.mesh_buffers(ref, edges[i], (0, 0, 0), [None] * 4)[0]), i
+    b.close()

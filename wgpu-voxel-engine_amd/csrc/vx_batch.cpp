@@ -331,6 +331,7 @@ int capture_graph(vx_batch *b) {
 // and the neighbours' planes).
 void describe(const vx_batch *b, FillWork *fw, MeshWork *mw) {
     char *store = (char *)b->store;
+    BatchVariants variants(b->max_edge, b->n);
     for (int i = 0; i < b->n; i++) {
         const vx_batch_req &r = b->reqs[i];
         const Layout L = layout_of(r.edge);
@@ -342,7 +343,7 @@ void describe(const vx_batch *b, FillWork *fw, MeshWork *mw) {
         f.cz = r.coord.z;
         f.edge = r.edge;
         f.terrain = r.terrain_id;
-        f.variant = fill_variant(b->ctx->terrains[r.terrain_id], f.cx, f.cy, f.cz, f.edge);
+        f.variant = variants.of(b->ctx->terrains[r.terrain_id], r.terrain_id, f.cx, f.cy, f.cz, f.edge);
         f.ids = (uint8_t *)base;
         f.occ = (uint32_t *)(base + L.occ);
         f.planes = (uint32_t *)(base + L.planes);

@@ -77,4 +77,62 @@ inline int32_t fast_variant(int32_t octaves, float frequency, float lacunarity, 
     return 0;
 }
 
+// True if every voxel coordinate of the frequency lies on one of at most 64
+// positions in a cell (f is a multiple of 1/q), or cells are larger than 64 voxels.
+inline bool on_lattice(float f) {
+    if (f < 1.0f / 64) return true;
+    for (int q = 1; q <= 64; q++) {
+        const float p = f * (float)q, d = p - (float)(int)(p + 0.5f);
+        if (d < 1e-5f && d > -1e-5f) return true;
+    }
+    return false;
+}
+
+// Whether a chunk that fast_variant accepts gains from it in a batch of n
+// chunks of edges up to max_edge (one chunk alone always does: the general
+// kernel has one workgroup for it).  zero: the threshold is zero at every
+// layer (reference rule, y_scale 0).  From the fill times of 1 to 2,000 chunks
+// of each edge, general / fast:
+//   - above 4 octaves the general kernels evaluate octave by octave: 1.1 to 30.
+//   - Up to 4, their rows share a column's terms while its cell lasts, and
+//     tables gain less the more cells a chunk has.  At a finest frequency of
+//     0.32 / 0.35 / 0.41 / 0.45 / 0.5: 32^3 of 1 and 2 octaves 1.05 / 1.0 / 0.9 / 0.75 /
+//     0.8; of 3 0.95 / 1.0 / 1.0 / 1.0 / 0.8 (1.2 at 0.35 from 512 chunks on), of 4 1.15 /
+//     1.2 / 1.1 / 1.15 / 0.85 (0.9 at 0.45 from 1,024 on); 64^3 of 1, 3 and 4 1.3 to 2 /
+//     1.0 to 2 / 1.0 to 1.9 / 0.75 to 1.3 / 0.6 to 1.2, of 2 1.5 / 1.4 / 1.1 / 1.25 / 0.6.
+//   - A zero threshold meets noise that is exactly zero wherever a voxel lies
+//     on a lattice plane of every octave, and those rows are evaluated twice:
+//     one octave 0.4 to 1.05 (off the lattice 1.0 to 1.8 up to 0.25, at 64^3 up to
+//     0.35), two 0.95 to 1.25 up to 0.1, at 0.125 0.85 to 0.95 (1.2 from 1,024 chunks
+//     on) and 0.4 to 0.75 from 0.25 on (64^3 1.0 to 1.3), three and four as other
+//     terrains.  Where all cells are larger than 50,000 voxels it is zero nearly
+//     everywhere: 0.85.
+//   - 16^3 chunks pay for a chunk's tables over a quarter of the lines: 0.6 to
+//     1.05 below 384 chunks (one octave 0.8 to 1.0 at any number), then 0.95 to 1.3,
+//     on a lattice at threshold zero 0.5 to 1.0 below 1,024.
+inline bool fast_pays(int32_t octaves, float frequency, float lacunarity, bool zero, int32_t edge,
+                      int32_t max_edge, int32_t n) {
+    float f = frequency, fine = 0.0f;
+    bool lattice = zero && octaves <= 4;
+    for (int o = 0; o < octaves; o++) {
+        fine = f > fine ? f : fine;
+        lattice = lattice && on_lattice(f);
+        f = f * lacunarity;
+    }
+    if (zero && fine < 2e-5f) return false;
+    if (octaves > 4) return true;
+    if (max_edge <= 16) {
+        if (octaves == 1) return false;
+        return lattice ? octaves == 4 && n >= 1024 : n >= 384;
+    }
+    if (edge == 64) {
+        if (zero && octaves == 1) return !lattice && fine <= 0.36f;
+        return fine <= (octaves == 2 || n <= 16 ? 0.47f : 0.42f);
+    }
+    if (zero && octaves == 1) return !lattice && fine <= 0.25f;
+    if (lattice && octaves == 2) return fine <= (n >= 1024 ? 0.125f : 0.1f);
+    if (octaves == 4) return fine <= (n >= 1024 ? 0.42f : 0.46f);
+    return fine <= (octaves == 3 && n >= 512 ? 0.38f : 0.325f);
+}
+
 }  // namespace vx

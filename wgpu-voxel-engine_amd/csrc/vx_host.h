@@ -17,6 +17,26 @@ namespace vx {
 
 constexpr int kMaxTerrains = 64;
 
+// fill_variant of the chunks of a batch of n with edges up to max_edge
+// (fast_pays).
+class BatchVariants {
+    int32_t max_edge, n;
+    int8_t pays[kMaxTerrains][3] = {};  // by terrain and edge: 0 = not asked yet, 1 = yes, -1 = no
+
+  public:
+    BatchVariants(int32_t max_edge_, int32_t n_) : max_edge(max_edge_), n(n_) {}
+    int32_t of(const TerrainDev &T, int32_t terrain, int32_t cx, int32_t cy, int32_t cz, int32_t edge) {
+        const int32_t v = fill_variant(T, cx, cy, cz, edge);
+        if (!v || (T.kind != kDensity && T.kind != kReference)) return v;
+        int8_t &p = pays[terrain][edge >> 5];
+        if (!p) {
+            const bool zero = T.kind == kReference || (T.y_scale < 1e-6f && T.y_scale > -1e-6f);
+            p = fast_pays(T.octaves, T.frequency, T.lacunarity, zero, edge, max_edge, n) ? 1 : -1;
+        }
+        return p > 0 ? v : 0;
+    }
+};
+
 // Caching device allocator: blocks are rounded to size classes (4 per power
 // of two, >= 256 B) and recycled through per-class free lists, so the chunk
 // and mesh churn of a streaming world never reaches hipMalloc/hipFree after

@@ -354,6 +354,7 @@ int admit(vx_server *S) {
     int32_t *ord = (int32_t *)((char *)mw + up256((size_t)S->max_batch * sizeof(MeshWork)));
     F->nb_present.resize(n);
     uint32_t kinds = 0;
+    BatchVariants variants(F->max_edge, n);
     for (int i = 0; i < n; i++) {
         const vx_request &r = F->reqs[i];
         const ChunkLayoutS L = layout_s(r.edge);
@@ -365,7 +366,7 @@ int admit(vx_server *S) {
         f.cz = r.coord.z;
         f.edge = r.edge;
         f.terrain = r.terrain_id;
-        f.variant = fill_variant(ctx->terrains[r.terrain_id], f.cx, f.cy, f.cz, f.edge);
+        f.variant = variants.of(ctx->terrains[r.terrain_id], f.terrain, f.cx, f.cy, f.cz, f.edge);
         kinds |= f.variant ? kFillFast : kFillGeneral;
         f.ids = (uint8_t *)c;
         f.occ = (uint32_t *)(c + L.occ);
