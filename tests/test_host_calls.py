@@ -178,3 +178,28 @@ foreign.h = None
 if "{use}" != "neighbour":
     assert not sync_first(chunk)
 """)
+
+
+def test_mixed_batch_fills_side_by_side(scenario):
+    """A batch whose chunks take both fill kernels: the general ones on the
+    second stream, with as many workgroups as a batch of them alone, joined
+    before the count; a batch of one kind launches one fill."""
+    scenario("""
+fine = terrain(frequency=0.5, octaves=2)  # past the fast fill's frequencies
+tids = [ctx.terrain(fine if i % 8 == 0 else terrain()) for i in range(512)]
+b = V.Batch(ctx, [(i, 0, 0) for i in range(512)], 32, tids)
+calls()
+b.run()
+got = calls()
+at = [i for i, c in enumerate(got) if c == "hipStreamWaitEvent"]
+names = [c.split()[0] for c in got if "_kernel" in c]
+assert names[:3] == ["fill_split_kernel", "fill_fast_kernel", "count_kernel"], got
+assert len(at) == 2 and at[1] < got.index("count_kernel 512"), got
+assert "fill_split_kernel 2048" in got and "fill_fast_kernel 1024" in got, got
+b.wait()
+one = batch(64)
+calls()
+one.run()
+got = calls()
+assert [c.split()[0] for c in got if "fill" in c] == ["fill_fast_kernel"] and "hipStreamWaitEvent" not in got
+""")

@@ -163,11 +163,27 @@ int32_t emit_split_of(const vx_batch *b) {
     return tuned_auto(b) ? b->tuned_emit_split : b->emit_split;
 }
 
+// A batch of both kinds of chunks fills them side by side, the general ones on
+// the second stream: either kernel alone may leave most of the GPU idle (256
+// chunks, half of each kind, 189 us a pass one after the other, 169 so).  More
+// general chunks than fill the GPU lose 2% beside the others and run after them.
 hipError_t enqueue_fill(vx_batch *b, hipStream_t s) {
     vx_ctx *ctx = b->ctx;
-    return launch_fill(b->fill_dev, b->order_dev, b->n, b->max_edge, ctx->terrains_dev,
-                       ctx->lut_dev, b->overflow + 1, fill_split_of(b), b->fill_kinds, s);
+    auto fill = [&](FillMix mix, hipStream_t st) {
+        return launch_fill(b->fill_dev, b->order_dev, b->n, b->max_edge, ctx->terrains_dev,
+                           ctx->lut_dev, b->overflow + 1, fill_split_of(b), mix, st);
+    };
+    if (!b->fill_mix.fast || !b->fill_mix.general || b->fill_mix.general > kFillGrid)
+        return fill(b->fill_mix, s);
+    hipError_t e = hipEventRecord(b->mix_ev[0], s);
+    if (e == hipSuccess) e = hipStreamWaitEvent(ctx->stream2, b->mix_ev[0], 0);
+    if (e == hipSuccess) e = fill(FillMix{0, b->fill_mix.general}, ctx->stream2);
+    if (e == hipSuccess) e = hipEventRecord(b->mix_ev[1], ctx->stream2);
+    if (e == hipSuccess) e = fill(FillMix{b->fill_mix.fast, 0}, s);
+    if (e == hipSuccess) e = hipStreamWaitEvent(s, b->mix_ev[1], 0);
+    return e;
 }
+
 // Batches of few chunks have no scan: the emit sums the counts itself.
 bool self_scan(const vx_batch *b) { return b->n <= kSelfScan && !b->fill_counts; }
 
@@ -240,15 +256,13 @@ hipError_t enqueue_split(vx_batch *b, hipStream_t s0) {
     b->order_halves = true;
     vx_ctx *ctx = b->ctx;
     hipError_t e = hipSuccess;
-    if (!ctx->stream2) e = hipStreamCreateWithFlags(&ctx->stream2, hipStreamNonBlocking);
-    if (e != hipSuccess) return e;
     hipStream_t s1 = ctx->stream2;
     const int32_t n = b->n, m = b->split_m, m2 = b->split_m2;
     const int32_t fs = fill_split_of(b), es = emit_split_of(b);
     e = launch_cull(b->cull, s0);
     if (e == hipSuccess)
         e = launch_fill(b->fill_dev, nullptr, m2, b->max_edge, ctx->terrains_dev, ctx->lut_dev,
-                        b->overflow + 1, fs, b->fill_kinds, s0);
+                        b->overflow + 1, fs, b->fill_mix, s0);
     if (e == hipSuccess) e = hipEventRecord(b->split_ev[0], s0);
     // first half on the second stream
     if (e == hipSuccess) e = hipStreamWaitEvent(s1, b->split_ev[0], 0);
@@ -265,7 +279,7 @@ hipError_t enqueue_split(vx_batch *b, hipStream_t s0) {
     // second half on s0
     if (e == hipSuccess)
         e = launch_fill(b->fill_dev + m2, nullptr, n - m2, b->max_edge, ctx->terrains_dev,
-                        ctx->lut_dev, b->overflow + 1, fs, b->fill_kinds, s0);
+                        ctx->lut_dev, b->overflow + 1, fs, b->fill_mix, s0);
     if (e == hipSuccess && !b->fill_counts)
         e = launch_count(b->mesh_dev + m, n - m, b->max_edge, b->counts + m, nullptr, nullptr,
                          CullJob{}, s0);
@@ -327,9 +341,8 @@ int capture_graph(vx_batch *b) {
     return VX_OK;
 }
 
-// Fill and mesh work of every chunk (device pointers into the batch's store
-// and the neighbours' planes).
-void describe(const vx_batch *b, FillWork *fw, MeshWork *mw) {
+// Fill work of every chunk (device pointers into the batch's store).
+void describe_fill(const vx_batch *b, FillWork *fw) {
     char *store = (char *)b->store;
     BatchVariants variants(b->max_edge, b->n);
     for (int i = 0; i < b->n; i++) {
@@ -349,6 +362,11 @@ void describe(const vx_batch *b, FillWork *fw, MeshWork *mw) {
         f.planes = (uint32_t *)(base + L.planes);
         f.meta = (uint32_t *)(base + L.meta);
     }
+}
+
+// Mesh work of every chunk (the neighbours' planes from their fill work), and
+// where the fill counts, the fill work's share of it.
+void describe_mesh(const vx_batch *b, FillWork *fw, MeshWork *mw) {
     for (int i = 0; i < b->n; i++) {
         const vx_batch_req &r = b->reqs[i];
         MeshWork &m = mw[i];
@@ -377,18 +395,24 @@ void describe(const vx_batch *b, FillWork *fw, MeshWork *mw) {
 }
 
 // What the form a run takes needs beside the descriptors, made when that form
-// first runs: the persistent forms' work list, the split form's events.
+// first runs: the persistent forms' work list, the second stream and its events
+// of the split form and of a staged batch of both kinds of chunks.
 int ready_form(vx_batch *b) {
     vx_ctx *ctx = b->ctx;
-    const int form = form_of(b);
-    if (form == VX_BATCH_SPLIT)
-        for (hipEvent_t &ev : b->split_ev)
-            if (!ev) VX_HIP(ctx, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    const bool split = form_of(b) == VX_BATCH_SPLIT;
+    const bool mixed = !split && !use_fused(b) && b->fill_mix.fast && b->fill_mix.general;
+    if ((split || mixed) && !ctx->stream2)
+        VX_HIP(ctx, hipStreamCreateWithFlags(&ctx->stream2, hipStreamNonBlocking));
+    for (hipEvent_t &ev : b->split_ev)
+        if (split && !ev) VX_HIP(ctx, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    for (hipEvent_t &ev : b->mix_ev)
+        if (mixed && !ev) VX_HIP(ctx, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     if (!use_fused(b) || b->fused_made) return VX_OK;
     std::vector<FillWork> fw(b->n);
     std::vector<MeshWork> mw(b->n);
     std::vector<FusedWork> fu(b->n);
-    describe(b, fw.data(), mw.data());
+    describe_fill(b, fw.data());
+    describe_mesh(b, fw.data(), mw.data());
     for (int i = 0; i < b->n; i++) {
         fu[i].f = fw[i];
         fu[i].m = mw[i];
@@ -419,6 +443,8 @@ void free_batch(vx_batch *b) {
     ctx->dev_free(b->fused_dev);
     ctx->dev_free(b->fctl);
     for (hipEvent_t &ev : b->split_ev)
+        if (ev) (void)hipEventDestroy(ev);
+    for (hipEvent_t &ev : b->mix_ev)
         if (ev) (void)hipEventDestroy(ev);
     delete b;
 }
@@ -592,14 +618,9 @@ extern "C" int vx_batch_create_ext(vx_ctx *ctx, const vx_batch_req *reqs, int32_
     b->overflow = (uint32_t *)(b->total + 1);  // [0] arena overflow, [1] schedule error
     b->emit_order = (int32_t *)(desc + off_emit);
     if (slabbed) b->slabs = (uint32_t *)(desc + off_slabs);
-    // The fill counts the faces itself when every chunk has its own
-    // workgroup and no neighbour inside the batch (each neighbour plane is
-    // absent or resident before the run): the staged form then has no
-    // count kernel.
-    b->fill_counts = b->max_edge <= 32 && fill_whole_chunks(n);
-    for (int i = 0; i < n && b->fill_counts; i++)
-        for (int k = 0; k < 4; k++)
-            if (reqs[i].nb[k] >= 0) b->fill_counts = false;
+    bool alone = true;  // no neighbour inside the batch
+    for (int i = 0; i < n && alone; i++)
+        for (int k = 0; k < 4; k++) alone &= reqs[i].nb[k] < 0;
     {
         // assembled in the context's pinned staging where it fits (the copy is
         // then asynchronous), else in pageable memory
@@ -609,9 +630,15 @@ extern "C" int vx_batch_create_ext(vx_ctx *ctx, const vx_batch_req *reqs, int32_
             pageable.resize(desc_bytes);
             up = pageable.data();
         }
-        describe(b, (FillWork *)up, (MeshWork *)(up + off_mesh));
-        for (int i = 0; i < n; i++)
-            b->fill_kinds |= ((FillWork *)up)[i].variant ? kFillFast : kFillGeneral;
+        FillWork *const fw = (FillWork *)up;
+        describe_fill(b, fw);
+        for (int i = 0; i < n; i++) b->fill_mix.add(fw[i]);
+        // The fill counts the faces itself when every chunk has its own
+        // workgroup and no neighbour inside the batch (each neighbour plane is
+        // absent or resident before the run): the staged form then has no
+        // count kernel.
+        b->fill_counts = alone && b->max_edge <= 32 && fill_whole_chunks(n, b->fill_mix);
+        describe_mesh(b, fw, (MeshWork *)(up + off_mesh));
         if (!b->uniform) {
             int32_t *order = (int32_t *)(up + off_order);
             std::iota(order, order + n, 0);
@@ -649,7 +676,7 @@ extern "C" int vx_batch_create_ext(vx_ctx *ctx, const vx_batch_req *reqs, int32_
             for (int k = 0; k < 4; k++) m2 = std::max(m2, reqs[i].nb[k] + 1);
         b->split_m = m;
         b->split_m2 = m2;
-        b->split_ok = !b->fill_counts || (m2 >= kFillGrid && n - m2 >= kFillGrid);
+        b->split_ok = !alone || n < kFillGrid || (m2 >= kFillGrid && n - m2 >= kFillGrid);
         b->split_total = (uint64_t *)((char *)b->total + 16);  // in the control block's spare words
     }
     // fused form: every in-batch neighbour must be the adjacent chunk with the
@@ -801,7 +828,7 @@ extern "C" int vx_batch_run_per_chunk(vx_ctx *ctx, vx_batch *b) {
     const int n = b->n;
     for (int i = 0; i < n; i++)
         VX_HIP(ctx, launch_fill(b->fill_dev + i, nullptr, 1, b->reqs[i].edge, ctx->terrains_dev,
-                                ctx->lut_dev, b->overflow + 1, 0, b->fill_kinds, ctx->stream));
+                                ctx->lut_dev, b->overflow + 1, 0, b->fill_mix, ctx->stream));
     auto slabs_of = [&](int i) { return b->slabs ? b->slabs + (size_t)kSlabs * i : nullptr; };
     for (int i = 0; i < n; i++)
         VX_HIP(ctx, launch_count(b->mesh_dev + i, 1, b->reqs[i].edge, b->counts + i, slabs_of(i),
@@ -1173,6 +1200,7 @@ extern "C" int vx_batch_profile(vx_ctx *ctx, vx_batch *b, int32_t reps, float ms
         acc[0] += t;
     }
     for (int r = 0; r < reps && !st && !whole; r++) {
+        if ((st = ready_form(b))) break;
         hipError_t e = hipEventRecord(ev[0], ctx->stream);
         if (e == hipSuccess) e = enqueue_fill(b, ctx->stream);
         if (e == hipSuccess) e = hipEventRecord(ev[1], ctx->stream);

@@ -170,7 +170,7 @@ struct vx_batch {
     float *planes_dev = nullptr;    // device copy of the cull planes
     vx::FillWork *fill_dev = nullptr;
     vx::MeshWork *mesh_dev = nullptr;
-    uint32_t fill_kinds = 0;        // kFillFast / kFillGeneral: the chunks' fill kernels
+    vx::FillMix fill_mix;           // chunks by fill kernel
     int32_t *order_dev = nullptr;   // longest-first schedule (null when uniform)
     void *desc = nullptr;           // block of the descriptors, the schedules and the control words
     int32_t *coords_dev = nullptr;  // chunk coordinates (draw lists), made on first use
@@ -202,6 +202,7 @@ struct vx_batch {
                                     // later chunks it borders)
     uint64_t *split_total = nullptr;   // faces of the first half (device)
     hipEvent_t split_ev[3] = {};    // fill, scan of the first half; the second half's end
+    hipEvent_t mix_ev[2] = {};      // the general fill's start and end beside the fast one
     int32_t pipe_lag = 0;           // farthest in-batch neighbour index ahead of a chunk
     vx::FusedWork *fused_dev = nullptr;
     bool fused_made = false;        // fused_dev has been written

@@ -216,16 +216,23 @@ inline int emit_parts_for(int32_t items, int32_t max_edge, int32_t hint = 0) {
     const int p = ((max_edge > 32 ? kEmitGrid64 : kEmitGrid) + items - 1) / items;
     return p < 16 ? (p - 1) | 1 : 15;
 }
-// parts_hint: fill_parts_for's hint.  kinds: which chunks the work holds
-// (kFillFast: a FillWork.variant set, kFillGeneral: 0): a kernel for each.
-enum : uint32_t { kFillFast = 1u, kFillGeneral = 2u };
+// Chunks of a launch by kernel: fast ones (a FillWork.variant set), general ones (0).
+struct FillMix {
+    int32_t fast = 0, general = 0;
+    void add(const FillWork &w) { (w.variant ? fast : general)++; }
+};
+// parts_hint: fill_parts_for's hint.  mix (of the batch that the launch is of):
+// a kernel for each kind there is.  The general one takes as many workgroups a
+// chunk as a batch of its chunks alone would: 64 of them among 512 filled in
+// 70 us with the batch's two, 41 with their four.
 hipError_t launch_fill(const FillWork *work, const int32_t *order, int32_t n, int32_t max_edge,
                        const TerrainDev *terrains, const GradLut *lut, uint32_t *error,
-                       int32_t parts_hint, uint32_t kinds, hipStream_t s);
-// True iff launch_fill gives each chunk one workgroup (fill_kernel), so that
-// FillWork.count_out is honoured for every chunk of the batch (whatever the
-// hint).
-inline bool fill_whole_chunks(int32_t n) { return n >= kFillGrid; }
+                       int32_t parts_hint, FillMix mix, hipStream_t s);
+// True iff launch_fill gives each chunk of a batch of n one workgroup, so that
+// FillWork.count_out is honoured for every chunk (whatever the hint).
+inline bool fill_whole_chunks(int32_t n, FillMix mix) {
+    return n >= kFillGrid && (mix.general == 0 || mix.general >= kFillGrid);
+}
 // Batches that hold 64^3 chunks emit by items: each 64^3 chunk is kSlabs
 // y-slabs of kSlabLayers layers (face counts per slab in slabs[kSlabs * i
 // ..], written by the count kernel), any other chunk one item.  With `items`

@@ -3009,24 +3009,25 @@ __global__ void __launch_bounds__(kDrawOneBlock) draw_one_kernel(Planes planes,
 // --------------------------------------------------------------- launchers
 hipError_t launch_fill(const FillWork *work, const int32_t *order, int32_t n, int32_t max_edge,
                        const TerrainDev *terrains, const GradLut *lut, uint32_t *error,
-                       int32_t parts_hint, uint32_t kinds, hipStream_t s) {
+                       int32_t parts_hint, FillMix mix, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     if (parts_hint != 0 && parts_hint != 1 && parts_hint != 2 && parts_hint != 4 && parts_hint != 8)
         return hipErrorInvalidValue;
+    const int32_t hint = n < kFillGrid ? parts_hint : 0;
     // small batches: several workgroups per chunk, each on a band of rows
-    const int parts = fill_parts_for(n, max_edge, parts_hint);
-    const int grid = n * parts;
-    if (kinds & kFillFast) {
+    if (mix.fast > 0) {
+        const int parts = fill_parts_for(n, max_edge, hint);
         if (max_edge <= 16)
-            fill_fast_kernel<16><<<grid, kBlock, 0, s>>>(work, order, n, terrains, lut, parts, error);
+            fill_fast_kernel<16><<<n * parts, kBlock, 0, s>>>(work, order, n, terrains, lut, parts, error);
         else if (max_edge <= 32)
-            fill_fast_kernel<32><<<grid, kBlock, 0, s>>>(work, order, n, terrains, lut, parts, error);
+            fill_fast_kernel<32><<<n * parts, kBlock, 0, s>>>(work, order, n, terrains, lut, parts, error);
         else {
-            const int p = parts_hint ? max(parts, 4) : fill64_parts_for(n);
+            const int p = hint ? max(parts, 4) : fill64_parts_for(n);
             fill_fast_kernel<64><<<n * p, kBlock, 0, s>>>(work, order, n, terrains, lut, p, error);
         }
     }
-    if (!(kinds & kFillGeneral)) return hipGetLastError();
+    if (mix.general <= 0) return hipGetLastError();
+    const int parts = fill_parts_for(min(mix.general, n), max_edge, hint), grid = n * parts;
     if (parts == 1) {
         if (max_edge <= 16) fill_kernel<16><<<n, kBlock, 0, s>>>(work, order, n, terrains, lut, error);
         else if (max_edge <= 32) fill_kernel<32><<<n, kBlock, 0, s>>>(work, order, n, terrains, lut, error);

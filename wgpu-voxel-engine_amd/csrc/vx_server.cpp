@@ -353,7 +353,7 @@ int admit(vx_server *S) {
     MeshWork *mw = (MeshWork *)(sl.pinned + up256((size_t)S->max_batch * sizeof(FillWork)));
     int32_t *ord = (int32_t *)((char *)mw + up256((size_t)S->max_batch * sizeof(MeshWork)));
     F->nb_present.resize(n);
-    uint32_t kinds = 0;
+    FillMix mix;
     BatchVariants variants(F->max_edge, n);
     for (int i = 0; i < n; i++) {
         const vx_request &r = F->reqs[i];
@@ -367,7 +367,7 @@ int admit(vx_server *S) {
         f.edge = r.edge;
         f.terrain = r.terrain_id;
         f.variant = variants.of(ctx->terrains[r.terrain_id], f.terrain, f.cx, f.cy, f.cz, f.edge);
-        kinds |= f.variant ? kFillFast : kFillGeneral;
+        mix.add(f);
         f.ids = (uint8_t *)c;
         f.occ = (uint32_t *)(c + L.occ);
         f.planes = (uint32_t *)(c + L.planes);
@@ -419,7 +419,7 @@ int admit(vx_server *S) {
     }
     if (e == hipSuccess)
         e = launch_fill(F->fill_dev, F->order_dev, n, F->max_edge, ctx->terrains_dev, ctx->lut_dev,
-                        F->overflow + 1, 0, kinds, s);
+                        F->overflow + 1, 0, mix, s);
     if (e == hipSuccess) e = launch_count(F->mesh_dev, n, F->max_edge, F->counts, F->slabs, nullptr,
                                           CullJob{}, s);
     // the scan rewrites the order array (the fill has consumed it) as the
