@@ -82,3 +82,42 @@ def test_batch_parts(ctx, oracle_mod, edge, n):
         assert (got["m"].view(np.uint32) == ei["m"].view(np.uint32)).all(), i
         assert (got["tex"] == ei["tex"]).all(), i
     b.close()
+
+
+@pytest.mark.parametrize("formats", [V.FMT_VERTICES, V.FMT_INSTANCES, V.FMT_VERTICES | V.FMT_INSTANCES])
+@pytest.mark.parametrize("n", [1279, 1280])
+def test_batch_parts_by_faces(ctx, oracle_mod, n, formats):
+    """Three workgroups an item, but one for an item of 8,192 faces and more
+    that writes vertices: items on both sides of it, empty ones among them."""
+    print("[case]", n, formats, flush=True)
+    kw = dict(seed=7, lacunarity=2.0, gain=0.5)
+    ts = [V.Terrain(kind=V.TERRAIN_REFERENCE, octaves=2, frequency=0.3, **kw),   # 28,000 faces
+          V.Terrain(kind=V.TERRAIN_REFERENCE, octaves=3, frequency=0.057, **kw),  # about 8,000
+          V.Terrain(kind=V.TERRAIN_DENSITY, octaves=4, frequency=1 / 64, y_scale=1 / 128, **kw),
+          V.Terrain(kind=V.TERRAIN_AIR)]
+    ots = [oracle_mod.terrain(kind=t.kind, seed=t.seed, octaves=t.octaves, frequency=t.frequency,
+                              lacunarity=t.lacunarity, gain=t.gain, height_scale=t.height_scale,
+                              height_max=t.height_max, y_scale=t.y_scale) for t in ts]
+    pick = [(i // 32 if i % 32 == 5 else 3) % 4 for i in range(n)]
+    coords = [(i % 31 - 15, 0, i // 31) for i in range(n)]
+    b = V.Batch(ctx, coords, 32, [ctx.terrain(ts[k]) for k in pick], None, formats=formats)
+    b.run()
+    b.wait()
+    inst = b.mesh(V.FMT_INSTANCES) if formats & V.FMT_INSTANCES else None
+    vert, idx = (b.mesh(V.FMT_VERTICES), b.mesh(V.FMT_INDICES)) if formats & V.FMT_VERTICES else (None, None)
+    counts = []
+    for i in [k for k in range(n) if pick[k] != 3] + [0, n - 1]:
+        ids = oracle_mod.chunk_fill(ots[pick[i]], *coords[i], 32)
+        faces, ei, ev, ex = oracle_mod.mesh_buffers(ids, 32, tuple(v * 32 for v in coords[i]), [None] * 4)
+        first, cnt = b.chunk_faces(i)
+        assert cnt == len(faces), i
+        counts.append(cnt)
+        if inst is not None:
+            got = inst[first:first + cnt]
+            assert (got["m"].view(np.uint32) == ei["m"].view(np.uint32)).all(), i
+            assert (got["tex"] == ei["tex"]).all(), i
+        if vert is not None:
+            assert (vert[4 * first:4 * (first + cnt)].view(np.uint32) == ev.view(np.uint32)).all(), i
+            assert (idx[6 * first:6 * (first + cnt)] == ex).all(), i
+    assert min(c for c in counts if c) < 8192 < max(counts)
+    b.close()

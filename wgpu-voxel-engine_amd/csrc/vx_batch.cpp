@@ -1073,7 +1073,7 @@ extern "C" int vx_batch_autotune(vx_ctx *ctx, vx_batch *b, int32_t reps, vx_tune
     // per item, each beside the other stage's rule
     {
         const int32_t items = emit_items_of(b->n, b->n_items, b->max_edge);
-        const int hf = fill_parts_for(b->n, b->max_edge), he = emit_parts_for(items, b->max_edge);
+        const int hf = fill_parts_for(b->n, b->max_edge), he = emit_parts_for(items, b->max_edge, b->formats & kFmtVertices);
         if (b->n < kFillGrid) {
             cands.push_back({VX_BATCH_STAGED, 0, 0, hf / 2, 0});
             if (hf * 2 <= (b->max_edge > 32 ? 8 : 4)) cands.push_back({VX_BATCH_STAGED, 0, 0, hf * 2, 0});

@@ -196,16 +196,18 @@ inline int fill_parts_for(int32_t n, int32_t max_edge, int32_t hint = 0) {
 // take 15 / 17 / 18 / 19 / 23 us at 4 / 4 / 3 / 2 / 1 parts, against 22 / 21 / 24 /
 // 25 / 31 at the rule of edge 32.  Edge 32: kEmitGrid workgroups, at most 15
 // parts (512 chunks at 1 / 3 / 5 / 8 parts 127 / 95 / 94 / 101 us a pass), three up
-// to kEmitThree (1,640 chunks whose faces differ much at 1 / 2 / 3 / 4 parts
-// 184 / 169 / 172 / 177, alike ones 308 / 319 / 307), one beyond (1,980 alike ones
-// 353 / 374 / 353, 2,450 424 / 463 / 429).  Slabs of 64^3 chunks hold more faces:
-// kEmitGrid64 (1,292 slabs at 1 / 3 / 5 / 8 parts 430 / 386 / 364 / 416); one at
-// kEmitGrid items or more (two at 4,100 mixed items lose 15%).  Odd numbers:
-// workgroups go round the 8 XCDs, and an even number puts the same parts and
-// slabs, which are not alike, on the same ones (1,600 slabs at 2 / 3 / 4 parts
-// 347 / 304 / 346).  `hint` (1..4; 0 = this rule) replaces the rule below
-// kEmitGrid items.
-inline int emit_parts_for(int32_t items, int32_t max_edge, int32_t hint = 0) {
+// to kEmitThree, but for chunks of many faces (emit_shares; 1,640 chunks of
+// instances at 1 / 3 parts 171 / 170 us density, 184 / 174 reference rule, 139 / 133
+// heightmap), one beyond (1,980 alike ones 353 / 374 / 353, 2,450 424 / 463 / 429 at
+// 1 / 2 / 3).  Slabs of 64^3 chunks hold more faces: kEmitGrid64 (1,292 slabs at 1 / 3 /
+// 5 / 8 parts 430 / 386 / 364 / 416); without vertices seven at most from 256 slabs
+// on (600 slabs at 3 / 7 / 11 parts 156 / 146 / 159 us density, 490 / 496 / 523 with
+// 22,000 faces each; with vertices the latter prefer 11, 582 / 552); one at
+// kEmitGrid items or more (two at 4,100 mixed items lose 15%).  Odd numbers above two: workgroups go round the 8
+// XCDs, and an even number puts the same parts and slabs, which are not alike,
+// on the same ones (1,600 slabs at 2 / 3 / 4 parts 347 / 304 / 346).  `hint` (1..4;
+// 0 = this rule) replaces the rule below kEmitGrid items.
+inline int emit_parts_for(int32_t items, int32_t max_edge, bool vertices, int32_t hint = 0) {
     if (items >= kEmitGrid) return 1;
     if (hint > 0) return hint;
     if (max_edge <= 16) {
@@ -214,7 +216,18 @@ inline int emit_parts_for(int32_t items, int32_t max_edge, int32_t hint = 0) {
     }
     if (max_edge <= 32 && 2 * items >= kEmitGrid) return items < kEmitThree ? 3 : 1;
     const int p = ((max_edge > 32 ? kEmitGrid64 : kEmitGrid) + items - 1) / items;
-    return p < 16 ? (p - 1) | 1 : 15;
+    const int most = max_edge > 32 && items >= 256 && !vertices ? 7 : 15;
+    return p <= most ? (p - 1) | 1 : most;
+}
+// Whether the parts of a batch of n items share an item of F faces.  Where the
+// items alone fill the GPU, several parts even out a last round of unequal
+// items, but writing vertices and indices of many faces (104 B each) from
+// three workgroups at once loses more: 1,640 chunks of 32^3 at 1 / 3 parts, 2,700
+// faces each 163 / 155 us, 11,500 663 / 689, 28,000 1,424 / 1,481 (instances, 68 B, gain:
+// 555 / 501 and 1,078 / 980).
+constexpr uint32_t kEmitDense = 8192;
+constexpr bool emit_shares(int32_t n, uint32_t F, bool vertices) {
+    return !vertices || F < kEmitDense || 2 * n < kEmitGrid;
 }
 // Chunks of a launch by kernel: fast ones (a FillWork.variant set), general ones (0).
 struct FillMix {

@@ -2366,7 +2366,12 @@ emit_kernel(const MeshWork *__restrict__ work, const int32_t *__restrict__ order
     if (!order_entry_ok(item, n, overflow + 1)) return;
     const uint64_t base =
         total ? self_base(counts, item, n, bases, total, S.red, part == 0) : bases[item];
-    emit_item<MAXN, BLOCK>(work[item], base, counts[item], out, tables, overflow, S, part, parts);
+    const uint32_t F = counts[item];
+    if (!emit_shares(n, F, out.formats & kFmtVertices)) {
+        if (part > 0) return;
+        parts = 1;
+    }
+    emit_item<MAXN, BLOCK>(work[item], base, F, out, tables, overflow, S, part, parts);
 }
 
 // One slab of a 64^3 chunk: its faces start `off` faces into the chunk,
@@ -3125,7 +3130,8 @@ hipError_t launch_emit(const MeshWork *work, const int32_t *order, int32_t n, in
     // small batches: several workgroups per item, so the grid still covers
     // about a full GPU of workgroups and an item's tiles are emitted side by
     // side
-    const int parts = emit_parts_for(max_edge <= 32 ? n : n_items > 0 ? n_items : items, max_edge, parts_hint);
+    const int parts = emit_parts_for(max_edge <= 32 ? n : n_items > 0 ? n_items : items, max_edge,
+                                     out.formats & kFmtVertices, parts_hint);
     const int grid = items * parts;
     if (max_edge <= 16)
         emit_kernel<16, kBlock><<<grid, kBlock, 0, s>>>(work, order, bases, counts, out, tables,
