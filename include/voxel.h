@@ -326,10 +326,12 @@ int vx_batch_set_grid(vx_batch *batch, int32_t grid);
  * autotuner has chosen a split for the batch. */
 int vx_batch_set_roles(vx_batch *batch, int32_t ratio);
 /* Tile shape of the VX_BATCH_STAGED form for small batches: workgroups per
- * chunk of the fill (1, 2, 4 or 8; used below 1,024 chunks, where the rule
- * is 2, 4 or 8, and 8 only for 64^3 chunks, which take at least 4) and per item of the emit (1..4;
- * used below 2,560 items, where the rule is 2 to 16); 0 = the rule.
- * Larger batches take one workgroup per chunk and per item whatever is set.
+ * chunk of the fill (1, 2, 4 or 8; used below 1,024 chunks, where the rule is
+ * 2, 4 or 8; chunks of batches that hold 64^3 ones and take the bounded fill
+ * get 4 at least, 4 to 16 by the rule) and per item of the emit (1..4; used below
+ * 2,560 items, where the rule gives an odd number up to 15, and 16^3 batches one
+ * round of 1,280 workgroups); 0 = the rule.  Larger batches take the rule
+ * whatever is set: one, but four for the bounded fill beside 64^3 chunks.
  * Other forms ignore it, and so does VX_BATCH_AUTO once the autotuner has
  * chosen a shape for the batch. */
 int vx_batch_set_splits(vx_batch *batch, int32_t fill_parts, int32_t emit_parts);

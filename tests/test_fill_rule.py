@@ -212,3 +212,54 @@ def test_batches_that_gain(tmp_path):
     text = "\n".join(" ".join(repr(float(v)) if isinstance(v, float) else str(v) for v in c[:-1]) for c in cases)
     out = subprocess.run([str(tmp_path / "p")], input=text, capture_output=True, text=True, check=True)
     assert [int(v) for v in out.stdout.split()] == [c[-1] for c in cases]
+
+
+TUNE = r"""
+#include <cstdio>
+#include "vx_fill_rule.h"
+int main() {
+    int n, m, general;
+    while (scanf("%d %d %d", &n, &m, &general) == 3) {
+        vx::FillMix mix;
+        mix.fast = n - general;
+        mix.general = general;
+        int32_t hints[4];
+        const int k = vx::tune_fill_hints(n, m, mix, hints);
+        const vx::FillShape r = vx::fill_shape(n, m, mix, 0);
+        printf("%d %d", r.fast, r.general);
+        for (int i = 0; i < k; i++) {
+            const vx::FillShape s = vx::fill_shape(n, m, mix, hints[i]);
+            printf(" %d %d %d", hints[i], s.fast, s.general);
+        }
+        printf("\n");
+    }
+}
+"""
+
+
+def test_tuner_hints(tmp_path):
+    """The fill shapes that the autotuner times: each another than the rule's
+    and than each other's, half and twice what the kernels do take."""
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        pytest.skip("no host C++ compiler")
+    (tmp_path / "t.cpp").write_text(TUNE)
+    subprocess.run([cxx, "-std=c++17", "-O1", "-I", CSRC, str(tmp_path / "t.cpp"), "-o", str(tmp_path / "t")],
+                   check=True)
+    cases = [(n, m, g) for n in (1, 64, 127, 128, 300, 511, 512, 700, 1023, 1024, 4000) for m in (16, 32, 64)
+             for g in sorted({0, 1, n // 2, n})]
+    out = subprocess.run([str(tmp_path / "t")], input="\n".join("%d %d %d" % c for c in cases),
+                         capture_output=True, text=True, check=True).stdout.splitlines()
+    got = {}
+    for case, line in zip(cases, out):
+        v = list(map(int, line.split()))
+        shapes = [tuple(v[:2])] + [tuple(v[i + 1:i + 3]) for i in range(2, len(v), 3)]
+        hints = v[2::3]
+        assert len(set(shapes)) == len(shapes), (case, v)
+        assert set(hints) <= {1, 2, 4, 8} and (case[0] < 1024 or not hints), (case, v)
+        assert (shapes[0][0] > 0) == (case[0] > case[2]) and (shapes[0][1] > 0) == (case[2] > 0), (case, v)
+        got[case] = hints
+    # 64^3 by the bounded fill: 16, 8 and 4 workgroups by the rule
+    assert (got[64, 64, 0], got[300, 64, 0], got[700, 64, 0]) == ([8], [4], [4])
+    assert got[300, 32, 0] == [2] and got[700, 32, 0] == [1, 4]   # as the general kernels
+    assert got[300, 64, 300] == [2, 8] and got[64, 64, 64] == [4]

@@ -203,3 +203,17 @@ one.run()
 got = calls()
 assert [c.split()[0] for c in got if "fill" in c] == ["fill_fast_kernel"] and "hipStreamWaitEvent" not in got
 """)
+
+
+def test_autotuner_times_each_fill_shape_once(scenario):
+    """64^3 chunks of the bounded fill: eight workgroups by the rule, four and
+    not eight again among the candidates, and each launched as named."""
+    scenario("""
+b = batch(130, 64, face_capacity=64)
+calls()
+r = b.autotune(1)
+fills = [c["splits"][0] for c in r["candidates"] if c["mode"] == "staged" and c["splits"][1] == 0]
+assert fills == [0, 4], r
+seen = {int(c.split()[1]) // 130 for c in calls() if c.startswith(("fill_fast", "captured:fill_fast"))}
+assert seen == {4, 8}, seen
+""")

@@ -632,7 +632,7 @@ extern "C" int vx_batch_create_ext(vx_ctx *ctx, const vx_batch_req *reqs, int32_
         }
         FillWork *const fw = (FillWork *)up;
         describe_fill(b, fw);
-        for (int i = 0; i < n; i++) b->fill_mix.add(fw[i]);
+        for (int i = 0; i < n; i++) b->fill_mix.add(fw[i].variant);
         // The fill counts the faces itself when every chunk has its own
         // workgroup and no neighbour inside the batch (each neighbour plane is
         // absent or resident before the run): the staged form then has no
@@ -1068,16 +1068,15 @@ extern "C" int vx_batch_autotune(vx_ctx *ctx, vx_batch *b, int32_t reps, vx_tune
     cands.push_back({VX_BATCH_STAGED, 0, 0});
     // staged tile shapes for batches small enough that the launchers split
     // chunks (the fill, under kFillGrid chunks) or items (the emit, under
-    // kEmitGrid items) over several workgroups: half and twice the fill's
-    // rule, and one or four (two when the rule gives four or more) emit workgroups
-    // per item, each beside the other stage's rule
+    // kEmitGrid items) over several workgroups: half and twice the fill's rule
+    // (tune_fill_hints), and one or four (two when the rule gives four or more)
+    // emit workgroups per item, each beside the other stage's rule
     {
         const int32_t items = emit_items_of(b->n, b->n_items, b->max_edge);
-        const int hf = fill_parts_for(b->n, b->max_edge), he = emit_parts_for(items, b->max_edge, b->formats & kFmtVertices);
-        if (b->n < kFillGrid) {
-            cands.push_back({VX_BATCH_STAGED, 0, 0, hf / 2, 0});
-            if (hf * 2 <= (b->max_edge > 32 ? 8 : 4)) cands.push_back({VX_BATCH_STAGED, 0, 0, hf * 2, 0});
-        }
+        const int he = emit_parts_for(items, b->max_edge, b->formats & kFmtVertices);
+        int32_t hints[4];
+        const int k = tune_fill_hints(b->n, b->max_edge, b->fill_mix, hints);
+        for (int i = 0; i < k; i++) cands.push_back({VX_BATCH_STAGED, 0, 0, hints[i], 0});
         if (items < kEmitGrid) {
             if (he != 1) cands.push_back({VX_BATCH_STAGED, 0, 0, 0, 1});
             cands.push_back({VX_BATCH_STAGED, 0, 0, 0, he >= 4 ? 2 : 4});

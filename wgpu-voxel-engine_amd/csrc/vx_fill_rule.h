@@ -1,9 +1,11 @@
-// vx_fill_rule.h -- which chunks the fast density fill takes, and with which
-// compiled variant.  Plain C++ (no HIP), shared by the host runtime and the
-// kernels and checked on the CPU.
+// vx_fill_rule.h -- which chunks the fast density fill takes, with which
+// compiled variant, and how many workgroups fill a chunk.  Plain C++ (no HIP),
+// shared by the host runtime and the kernels and checked on the CPU.
 #pragma once
 
 #include <stdint.h>
+
+#include <initializer_list>
 
 namespace vx {
 
@@ -133,6 +135,67 @@ inline bool fast_pays(int32_t octaves, float frequency, float lacunarity, bool z
     if (lattice && octaves == 2) return fine <= (n >= 1024 ? 0.125f : 0.1f);
     if (octaves == 4) return fine <= (n >= 1024 ? 0.42f : 0.46f);
     return fine <= (octaves == 3 && n >= 512 ? 0.38f : 0.325f);
+}
+
+// ---- workgroups per chunk
+constexpr int kFillGrid = 1024;  // fill workgroups that fill the GPU (4 per CU)
+
+// Chunks of a batch by kernel: fast ones (a variant set), general ones.
+struct FillMix {
+    int32_t fast = 0, general = 0;
+    void add(int32_t variant) { (variant ? fast : general)++; }
+};
+
+// Workgroups per chunk of n chunks: one for kFillGrid or more; below that 2, 4
+// or 8 so that the grid still covers about kFillGrid workgroups (8 only for at
+// most kFillGrid / 8 chunks that hold 64^3 ones).  `hint` (1, 2, 4 or 8; 0 =
+// this rule) replaces the rule where it would split.
+constexpr int fill_parts_for(int32_t n, int32_t max_edge, int32_t hint = 0) {
+    if (n >= kFillGrid) return 1;
+    if (hint > 0) return hint;
+    return 2 * n >= kFillGrid ? 2 : (max_edge > 32 && 8 * n <= kFillGrid) ? 8 : 4;
+}
+
+// Workgroups per chunk that each fill kernel takes on a batch of n chunks (0 =
+// it has none): the fast one by all n, with 64^3 chunks fill64_parts_for or a
+// hint of 4 at least; the general one as a batch of its chunks alone would (64
+// of them among 512 filled in 70 us with the batch's two, in 41 with their four).
+// Batches of kFillGrid chunks and more ignore the hint.
+struct FillShape {
+    int fast, general;
+};
+constexpr FillShape fill_shape(int32_t n, int32_t max_edge, FillMix mix, int32_t hint) {
+    const int32_t h = n < kFillGrid ? hint : 0, general = mix.general < n ? mix.general : n;
+    const int fast = max_edge <= 32 ? fill_parts_for(n, max_edge, h)
+                     : h            ? (h > 4 ? h : 4)
+                                    : fill64_parts_for(n);
+    return FillShape{mix.fast > 0 ? fast : 0, general > 0 ? fill_parts_for(general, max_edge, h) : 0};
+}
+
+// True iff each chunk of a batch of edges up to 32 gets one workgroup, so that
+// FillWork.count_out is honoured for every chunk (whatever the hint).
+constexpr bool fill_whole_chunks(int32_t n, FillMix mix) {
+    return n >= kFillGrid && (mix.general == 0 || mix.general >= kFillGrid);
+}
+
+// Hints worth timing on a batch: half and twice what the rule gives each of its
+// kernels (four at most up to edge 32, eight beyond), without those that come
+// to a shape that another, or the rule, has already.  At most 4; their number.
+constexpr int tune_fill_hints(int32_t n, int32_t max_edge, FillMix mix, int32_t hints[4]) {
+    if (n >= kFillGrid) return 0;
+    FillShape seen[5] = {fill_shape(n, max_edge, mix, 0)};
+    int k = 0;
+    for (const int parts : {seen[0].general, seen[0].fast})
+        for (const int h : {parts / 2, parts * 2}) {
+            if (h < 1 || h > (max_edge > 32 ? 8 : 4)) continue;
+            const FillShape s = fill_shape(n, max_edge, mix, h);
+            bool known = false;
+            for (int i = 0; i <= k; i++) known |= seen[i].fast == s.fast && seen[i].general == s.general;
+            if (known) continue;
+            hints[k++] = h;
+            seen[k] = s;
+        }
+    return k;
 }
 
 }  // namespace vx

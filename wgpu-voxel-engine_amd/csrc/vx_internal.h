@@ -16,7 +16,6 @@ constexpr int kDescTile = 4096;    // face descriptors staged in LDS per emit ti
 constexpr int kEmitGrid = 2560;    // emit workgroups that fill the GPU twice (5 per CU at once)
 constexpr int kEmitThree = 1792;   // chunks of edge 32 up to which three workgroups each pay
 constexpr int kEmitGrid64 = 6144;  // the same over slabs of 64^3 chunks (4 per CU at once)
-constexpr int kFillGrid = 1024;    // fill workgroups that fill the GPU (4 per CU)
 
 // Terrain kinds (mirror of vx_terrain.kind in include/voxel.h).
 enum : int32_t { kAir = 0, kSolid = 1, kHeightmap = 2, kDensity = 3, kReference = 4 };
@@ -178,17 +177,6 @@ inline int words_per_row(int edge) { return (edge + 31) / 32; }
 // null for 0..n-1.  An entry outside [0, n) makes its workgroup do nothing
 // and sets a sticky error word: `error` for the fill, overflow[1] for the
 // emit, whose overflow[0] is the arena-overflow flag the scan clears.
-// Workgroups per chunk of the fill: one for batches of kFillGrid chunks or
-// more; below that 2, 4 or 8 so that the grid still covers about kFillGrid
-// workgroups (8 only for batches of at most kFillGrid / 8 chunks that hold
-// 64^3 chunks).  `hint` (1, 2, 4 or 8; 0 = this rule) replaces the rule
-// for the batches it would split.  (64^3 chunks on the fast path:
-// fill64_parts_for.)
-inline int fill_parts_for(int32_t n, int32_t max_edge, int32_t hint = 0) {
-    if (n >= kFillGrid) return 1;
-    if (hint > 0) return hint;
-    return 2 * n >= kFillGrid ? 2 : (max_edge > 32 && 8 * n <= kFillGrid) ? 8 : 4;
-}
 // Workgroups per emit item, so that the last round of the 1,280 workgroups
 // that run at once is short without many that only repeat an item's set-up.
 // Edge 16 (700 faces an item, the set-up is most of it): one round, and at
@@ -229,23 +217,10 @@ constexpr uint32_t kEmitDense = 8192;
 constexpr bool emit_shares(int32_t n, uint32_t F, bool vertices) {
     return !vertices || F < kEmitDense || 2 * n < kEmitGrid;
 }
-// Chunks of a launch by kernel: fast ones (a FillWork.variant set), general ones (0).
-struct FillMix {
-    int32_t fast = 0, general = 0;
-    void add(const FillWork &w) { (w.variant ? fast : general)++; }
-};
-// parts_hint: fill_parts_for's hint.  mix (of the batch that the launch is of):
-// a kernel for each kind there is.  The general one takes as many workgroups a
-// chunk as a batch of its chunks alone would: 64 of them among 512 filled in
-// 70 us with the batch's two, 41 with their four.
+// parts_hint, mix (of the batch that the launch is of): fill_shape.
 hipError_t launch_fill(const FillWork *work, const int32_t *order, int32_t n, int32_t max_edge,
                        const TerrainDev *terrains, const GradLut *lut, uint32_t *error,
                        int32_t parts_hint, FillMix mix, hipStream_t s);
-// True iff launch_fill gives each chunk of a batch of n one workgroup, so that
-// FillWork.count_out is honoured for every chunk (whatever the hint).
-inline bool fill_whole_chunks(int32_t n, FillMix mix) {
-    return n >= kFillGrid && (mix.general == 0 || mix.general >= kFillGrid);
-}
 // Batches that hold 64^3 chunks emit by items: each 64^3 chunk is kSlabs
 // y-slabs of kSlabLayers layers (face counts per slab in slabs[kSlabs * i
 // ..], written by the count kernel), any other chunk one item.  With `items`

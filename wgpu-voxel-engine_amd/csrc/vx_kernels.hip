@@ -3018,21 +3018,18 @@ hipError_t launch_fill(const FillWork *work, const int32_t *order, int32_t n, in
     if (n <= 0) return hipSuccess;
     if (parts_hint != 0 && parts_hint != 1 && parts_hint != 2 && parts_hint != 4 && parts_hint != 8)
         return hipErrorInvalidValue;
-    const int32_t hint = n < kFillGrid ? parts_hint : 0;
     // small batches: several workgroups per chunk, each on a band of rows
-    if (mix.fast > 0) {
-        const int parts = fill_parts_for(n, max_edge, hint);
+    const FillShape shape = fill_shape(n, max_edge, mix, parts_hint);
+    if (const int p = shape.fast) {
         if (max_edge <= 16)
-            fill_fast_kernel<16><<<n * parts, kBlock, 0, s>>>(work, order, n, terrains, lut, parts, error);
+            fill_fast_kernel<16><<<n * p, kBlock, 0, s>>>(work, order, n, terrains, lut, p, error);
         else if (max_edge <= 32)
-            fill_fast_kernel<32><<<n * parts, kBlock, 0, s>>>(work, order, n, terrains, lut, parts, error);
-        else {
-            const int p = hint ? max(parts, 4) : fill64_parts_for(n);
+            fill_fast_kernel<32><<<n * p, kBlock, 0, s>>>(work, order, n, terrains, lut, p, error);
+        else
             fill_fast_kernel<64><<<n * p, kBlock, 0, s>>>(work, order, n, terrains, lut, p, error);
-        }
     }
-    if (mix.general <= 0) return hipGetLastError();
-    const int parts = fill_parts_for(min(mix.general, n), max_edge, hint), grid = n * parts;
+    const int parts = shape.general, grid = n * parts;
+    if (!parts) return hipGetLastError();
     if (parts == 1) {
         if (max_edge <= 16) fill_kernel<16><<<n, kBlock, 0, s>>>(work, order, n, terrains, lut, error);
         else if (max_edge <= 32) fill_kernel<32><<<n, kBlock, 0, s>>>(work, order, n, terrains, lut, error);

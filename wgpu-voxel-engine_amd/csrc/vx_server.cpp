@@ -367,7 +367,7 @@ int admit(vx_server *S) {
         f.edge = r.edge;
         f.terrain = r.terrain_id;
         f.variant = variants.of(ctx->terrains[r.terrain_id], f.terrain, f.cx, f.cy, f.cz, f.edge);
-        mix.add(f);
+        mix.add(f.variant);
         f.ids = (uint8_t *)c;
         f.occ = (uint32_t *)(c + L.occ);
         f.planes = (uint32_t *)(c + L.planes);
