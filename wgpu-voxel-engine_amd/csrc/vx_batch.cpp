@@ -389,7 +389,6 @@ void describe_mesh(const vx_batch *b, FillWork *fw, MeshWork *mw) {
         if (b->fill_counts) {
             for (int k = 0; k < 4; k++) fw[i].cnb[k] = m.nb[k];
             fw[i].count_out = b->counts + i;
-            fw[i].slab_out = b->slabs ? b->slabs + (size_t)kSlabs * i : nullptr;
         }
     }
 }

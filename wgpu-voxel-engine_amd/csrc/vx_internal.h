@@ -77,14 +77,13 @@ struct FillWork {
     uint32_t *planes;      // 4 planes * edge * W words: x=0, x=N-1, z=0, z=N-1
     uint32_t *meta;        // [0] solid block id (or kBlockMixed)
     float *noise_out;      // optional raw noise (density: edge^3, heightmap: edge^2)
-    // Optional (fill_kernel, one workgroup per chunk): the fill also counts
+    // Optional (one workgroup per chunk, edges up to 32): the fill also counts
     // the chunk's visible faces, for chunks whose every neighbour is absent
     // or was written before the launch.  cnb[k] = the plane of neighbour k
     // (-x, +x, -z, +z) facing this chunk, null = absent; count_out[0] = the
-    // face count; slab_out[0..kSlabs) = a 64^3 chunk's per-slab counts.
+    // face count.
     const uint32_t *cnb[4];
     uint32_t *count_out;   // null: the count kernel counts
-    uint32_t *slab_out;
 };
 
 // One chunk to mesh.  nb[k] points at the neighbour's plane facing this

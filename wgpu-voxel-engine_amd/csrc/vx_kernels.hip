@@ -677,7 +677,7 @@ __device__ void fill_part(const FillWork &w, const TerrainDev &T, FillShared<MAX
 }
 
 template <int N, int MAXN, class SH>
-__device__ void count_loaded(SH &S, uint32_t *count_out, uint32_t *slabs);
+__device__ uint32_t count_rows(SH &S);
 
 // The four planes facing a chunk (null = absent neighbour) into S.nb.
 template <int N, int MAXN, int BLOCK = kBlock, class SH>
@@ -690,9 +690,17 @@ __device__ __forceinline__ void load_neighbours(const uint32_t *const (&planes)[
     }
 }
 
-// With w.count_out the fill also counts the chunk's faces from the rows it
-// holds in LDS and the neighbour planes w.cnb (all written before the
-// launch), which spares the batch its count kernel.
+// With w.count_out the fill also counts the faces of a chunk of edge up to 32
+// from the rows it holds in LDS and the neighbour planes w.cnb (all written
+// before the launch), which spares the batch its count kernel.
+template <int N, int MAXN, class SH>
+__device__ __forceinline__ void count_filled(const FillWork &w, SH &S) {
+    load_neighbours<N, MAXN>(w.cnb, S);  // S.nb: no halo lines here
+    __syncthreads();
+    const uint32_t total = count_rows<N, MAXN>(S);
+    if (threadIdx.x == 0) *w.count_out = total;
+}
+
 template <int N, int MAXN, bool DBG>
 __device__ __forceinline__ void fill_chunk(const FillWork &w, const TerrainDev &T, FillShared<MAXN> &S) {
     const Halo H{0, 0u};
@@ -700,11 +708,8 @@ __device__ __forceinline__ void fill_chunk(const FillWork &w, const TerrainDev &
                                                          w.noise_out);
     __syncthreads();
     write_chunk_outputs<N, MAXN>(w, S, true, kBlockGrass);
-    if (w.count_out) {
-        load_neighbours<N, MAXN>(w.cnb, S);  // S.nb: no halo lines here
-        __syncthreads();
-        count_loaded<N, MAXN>(S, w.count_out, w.slab_out);
-    }
+    if constexpr (MAXN <= 32)
+        if (w.count_out) count_filled<N, MAXN>(w, S);
 }
 
 template <int N, int MAXN, bool REF>
@@ -1488,13 +1493,8 @@ __device__ __forceinline__ void fast_part(const FillWork &w, const TerrainDev &T
     } else {
         fast_tile<N, MAXN, 0>(w, T, G, S, FillTile<LS>{y_lo, y_lo + rows, z_lo, ls});
     }
-    if constexpr (MAXN <= 32) {
-        if (w.count_out && parts == 1) {
-            load_neighbours<N, MAXN>(w.cnb, S);
-            __syncthreads();
-            count_loaded<N, MAXN>(S, w.count_out, w.slab_out);
-        }
-    }
+    if constexpr (MAXN <= 32)
+        if (w.count_out && parts == 1) count_filled<N, MAXN>(w, S);
 }
 
 template <int MAXN>
@@ -1744,50 +1744,6 @@ __device__ uint32_t count_rows(SH &S) {
         for (int d = 0; d < 6; d++) c += popc(m[d]);
     }
     return block_sum(c, S.red);
-}
-
-// Counts the faces of the chunk whose rows and neighbour planes are in
-// LDS (S.occ, S.nb).  A 64^3 chunk's count also goes out per slab
-// (slabs[0..kSlabs), when given): thread t's rows t + kBlock * i lie in
-// slab i / (kSlabLayers * 64 / kBlock).
-template <int N, int MAXN, class SH>
-__device__ void count_loaded(SH &S, uint32_t *count_out, uint32_t *slabs) {
-    if constexpr (N == 64) {
-        using R = typename RowType<MAXN>::T;
-        constexpr int PER = kSlabLayers * 64 / kBlock;  // a thread's rows per slab
-        // per-slab sums: wave reductions, then one barrier
-        __shared__ uint32_t s_part[kBlock / 64][kSlabs];
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll 1
-        for (int s = 0; s < kSlabs; s++) {
-            uint32_t c = 0;
-#pragma unroll
-            for (int i = 0; i < PER; i++) {
-                const int r = threadIdx.x + kBlock * (s * PER + i);
-                R m[6];
-                face_masks<N, MAXN>(S, r / N, r % N, m);
-#pragma unroll
-                for (int d = 0; d < 6; d++) c += popc(m[d]);
-            }
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-            if (lane == 0) s_part[wave][s] = c;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            uint32_t total = 0;
-            for (int s = 0; s < kSlabs; s++) {
-                uint32_t c = 0;
-                for (int k = 0; k < kBlock / 64; k++) c += s_part[k][s];
-                if (slabs) slabs[s] = c;
-                total += c;
-            }
-            *count_out = total;
-        }
-    } else {
-        const uint32_t total = count_rows<N, MAXN>(S);
-        if (threadIdx.x == 0) *count_out = total;
-    }
 }
 
 // Faces of a chunk that one wave of WAVES (wave `wave` of them) sees, counted
