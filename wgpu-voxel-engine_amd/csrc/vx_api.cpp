@@ -302,6 +302,7 @@ int vx_ctx::ensure_scratch(size_t bytes) {
 }
 
 constexpr size_t kStageBytes = 1 << 20;
+constexpr size_t kDrawStateAt = 64;  // in the context's small block, behind the per-chunk words
 
 char *vx_ctx::staging(size_t bytes) {
     if (bytes > kStageBytes) return nullptr;
@@ -380,13 +381,13 @@ extern "C" int vx_ctx_create(const vx_ctx_desc *desc, vx_ctx **out) {
     if ((st = c->dev_alloc(sizeof(GradLut), (void **)&c->lut_dev)) ||
         (st = c->dev_alloc(sizeof(MeshTables), (void **)&c->tables_dev)) ||
         (st = c->dev_alloc(kMaxTerrains * sizeof(TerrainDev), (void **)&c->terrains_dev)) ||
-        (st = c->dev_alloc(64, (void **)&c->small_dev)) ||
-        (st = c->dev_alloc(8 * (size_t)kDrawStateWords, (void **)&c->draw_state)) ||
-        (st = c->dev_alloc(4 * (size_t)draw_blocks(kDrawOne), (void **)&c->draw_counts))) {
+        (st = c->dev_alloc(kDrawStateAt + 8 * kDrawStateWords + 4 * (size_t)draw_blocks(kDrawOne),
+                           &c->small_dev))) {
         vx_ctx_destroy(c);
         return st;
     }
-    c->draw_counts_cap = draw_blocks(kDrawOne);
+    c->draw_state = (uint64_t *)((char *)c->small_dev + kDrawStateAt);
+    c->draw_small = (uint32_t *)(c->draw_state + kDrawStateWords);
     if (hipHostMalloc((void **)&c->pinned, 4096, hipHostMallocDefault) != hipSuccess) {
         c->pinned = nullptr;
         vx_ctx_destroy(c);
@@ -966,21 +967,20 @@ int vx_draw_list_locked(vx_ctx *ctx, const vx_frustum *f, const int32_t *coords_
                                     ctx->stream));
         return VX_OK;
     }
-    if (nb > ctx->draw_counts_cap) {
+    if (n > kDrawOne && nb > ctx->draw_counts_cap) {
         if (ctx->draw_counts) {
             VX_HIP(ctx, hipStreamSynchronize(ctx->stream));  // earlier lists may still read it
             ctx->dev_free(ctx->draw_counts);
             ctx->draw_counts = nullptr;
             ctx->draw_counts_cap = 0;
         }
-        const int32_t cap = std::max(nb, 256);
-        int st = ctx->dev_alloc((size_t)cap * 4, (void **)&ctx->draw_counts);
+        int st = ctx->dev_alloc((size_t)nb * 4, (void **)&ctx->draw_counts);
         if (st) return st;
-        ctx->draw_counts_cap = cap;
+        ctx->draw_counts_cap = nb;
     }
     VX_HIP(ctx, launch_draw_list(P, coords_dev, faces_dev, first_dev, n, edge, mode,
-                                 ctx->draw_counts, reinterpret_cast<DrawArgs *>(args_dev),
-                                 count_dev, ctx->stream));
+                                 n > kDrawOne ? ctx->draw_counts : ctx->draw_small,
+                                 reinterpret_cast<DrawArgs *>(args_dev), count_dev, ctx->stream));
     return VX_OK;
 }
 

@@ -99,12 +99,14 @@ struct vx_ctx {
     vx::TerrainDev *terrains_dev = nullptr;
     vx::GradLut *lut_dev = nullptr;
     vx::MeshTables *tables_dev = nullptr;
-    void *small_dev = nullptr;  // [0] face count, [1] overflow flag, [4..7] slab counts of the per-chunk path
+    void *small_dev = nullptr;  // [0] face count, [1] overflow flag, [4..7] slab counts of the
+                                // per-chunk path; then draw_state, draw_small
     void *scratch = nullptr;    // staging for host-array entry points
     size_t scratch_bytes = 0;
     unsigned char *pinned = nullptr;  // 4 KiB pinned host staging for readbacks
     hipEvent_t free_fence = nullptr;  // recorded on `stream` at every dev_free
-    uint32_t *draw_counts = nullptr;  // per-workgroup counts of draw-list passes
+    uint32_t *draw_small = nullptr;   // per-workgroup counts of two-pass lists of up to kDrawOne meshes
+    uint32_t *draw_counts = nullptr;  // the same of longer ones (made on first use)
     int32_t draw_counts_cap = 0;
     uint64_t *draw_state = nullptr;   // status words of one-launch draw lists
     uint64_t draw_tag = 0;            // one-launch draw lists queued
