@@ -217,3 +217,24 @@ assert fills == [0, 4], r
 seen = {int(c.split()[1]) // 130 for c in calls() if c.startswith(("fill_fast", "captured:fill_fast"))}
 assert seen == {4, 8}, seen
 """)
+
+
+def test_no_memory_for_a_form_is_an_error(scenario):
+    """Host memory that a run needs for its form and cannot have is a status,
+    not an exception through the C entry; the batch runs once there is some."""
+    scenario("""
+import resource
+b = batch(20000, 16, face_capacity=64)
+b.set_mode(V.BATCH_FUSED)
+used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+soft, hard = resource.getrlimit(resource.RLIMIT_AS)
+resource.setrlimit(resource.RLIMIT_AS, (used + (1 << 20), hard))
+try:
+    b.run()
+    status = V.OK
+except V.VoxelError as e:
+    status = e.status
+resource.setrlimit(resource.RLIMIT_AS, (soft, hard))
+assert status == -2, status  # VX_ERR_NOMEM
+b.run()
+""")

@@ -407,9 +407,16 @@ int ready_form(vx_batch *b) {
     for (hipEvent_t &ev : b->mix_ev)
         if (mixed && !ev) VX_HIP(ctx, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     if (!use_fused(b) || b->fused_made) return VX_OK;
-    std::vector<FillWork> fw(b->n);
-    std::vector<MeshWork> mw(b->n);
-    std::vector<FusedWork> fu(b->n);
+    std::vector<FillWork> fw;
+    std::vector<MeshWork> mw;
+    std::vector<FusedWork> fu;
+    try {
+        fw.resize(b->n);
+        mw.resize(b->n);
+        fu.resize(b->n);
+    } catch (const std::bad_alloc &) {
+        return VX_ERR_NOMEM;
+    }
     describe_fill(b, fw.data());
     describe_mesh(b, fw.data(), mw.data());
     for (int i = 0; i < b->n; i++) {
