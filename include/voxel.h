@@ -184,7 +184,8 @@ int vx_chunk_noise(vx_ctx *ctx, int32_t terrain_id, vx_coord coord, int32_t edge
 /* Chunk::create_mesh with the neighbour snapshot adj = {-x, +x, -z, +z}
  * (src/chunk_builder.rs:134-169); NULL = absent neighbour (its boundary
  * faces are emitted, src/chunk.rs:102-108).  Neighbours must have the same
- * edge.  Synchronises once to size the mesh. */
+ * edge.  Synchronises once to size the mesh, and first with the stream of
+ * another context whose chunks it is given. */
 int vx_chunk_create_mesh(vx_ctx *ctx, vx_chunk *chunk, vx_chunk *const adj[4], uint32_t formats,
                          vx_mesh **out);
 int vx_mesh_retain(vx_mesh *mesh);
@@ -225,7 +226,10 @@ int vx_frustum_mask_device(vx_ctx *ctx, const vx_frustum *f, const int32_t *coor
  * One entry per visible mesh (zero-face meshes give no-op draws, as in the
  * reference).  count_dev[0] = number of draws; count_dev[1] != 0 if some
  * offset did not fit the 32-bit fields.  Asynchronous on the context stream;
- * all pointers are device pointers; args_dev holds n entries. */
+ * all pointers are device pointers; args_dev holds n entries.  A call may be
+ * captured from the context stream; up to 65,536 meshes it allocates nothing,
+ * and its replays may run beside later uncaptured calls of the context, but
+ * not beside each other's. */
 typedef struct vx_draw_indexed {
     uint32_t index_count;
     uint32_t instance_count;
@@ -242,8 +246,8 @@ int vx_frustum_draw_list(vx_ctx *ctx, const vx_frustum *f, const int32_t *coords
 /* vx_frustum_draw_list that allocates nothing.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under
  * HIP graph capture, a per-frame render loop, harnesses that forbid
- * allocation).  Same arguments, kernels and results as vx_frustum_draw_list;
- * its per-workgroup partial counts live in a fixed 16 KiB device array per
+ * allocation).  Same arguments and results as vx_frustum_draw_list, in two
+ * passes whatever the length; its per-workgroup partial counts live in a fixed 16 KiB device array per
  * GPU, held until the process ends, instead of a context allocation, and it
  * queues no memset.  n may not exceed VX_DRAW_LIST_NOALLOC_MAX
  * (VX_ERR_INVALID).  Every call on one GPU uses that GPU's array: calls that
@@ -339,7 +343,8 @@ int vx_batch_set_splits(vx_batch *batch, int32_t fill_parts, int32_t emit_parts)
  * VX_BATCH_PIPELINED). */
 int vx_batch_get_mode(vx_batch *batch, int32_t *mode);
 /* Queues fill -> count -> scan -> emit on the context stream (replayed from a
- * captured hipGraph after the first run).  Asynchronous. */
+ * hipGraph after the first run, captured on a stream of the library's own).
+ * Asynchronous. */
 int vx_batch_run(vx_ctx *ctx, vx_batch *batch);
 /* Waits for the last run; if the mesh arena was too small it is grown and the
  * emit stage re-run.  Reports the batch's total face count. */
@@ -366,8 +371,8 @@ int vx_batch_profile(vx_ctx *ctx, vx_batch *batch, int32_t reps, float ms[5]);
 /* Autotuner: runs the batch once (sizing its mesh arena, so every candidate
  * is timed on the whole output), then times every candidate execution form
  * and launch shape of this batch (staged; for small batches also staged with other tile shapes,
- * vx_batch_set_splits: half and twice the fill's workgroups per chunk, one
- * and four (or two) emit workgroups per item; fused with one workgroup per
+ * vx_batch_set_splits: half and twice the fill's workgroups per chunk where
+ * they can be set, one and four (or two) emit workgroups per item; fused with one workgroup per
  * chunk and with 3 or 4 persistent workgroups per CU; pipelined with one
  * workgroup per chunk and one mesher in three, and with 8 workgroups per CU
  * and one mesher in two, three or four; split in two halves on two streams)
@@ -377,8 +382,10 @@ int vx_batch_profile(vx_ctx *ctx, vx_batch *batch, int32_t reps, float ms[5]);
  * (chunk-count bucket, largest edge, uniform or ragged, neighbours).  The
  * batch is left in VX_BATCH_AUTO running the choice; shapes set before with
  * vx_batch_set_grid / _roles / _splits are cleared.  With VX_TUNE_CACHE set
- * to a file path the cache persists across processes.  Batches created later
- * in VX_BATCH_AUTO use a cached choice. */
+ * to a file path the cache persists across processes (a choice is a launch
+ * shape, valid with any build; one made by another build of the library may
+ * no longer be the fastest: delete the file after an update).  Batches created
+ * later in VX_BATCH_AUTO use a cached choice. */
 #define VX_TUNE_MAX_CANDIDATES 12
 typedef struct vx_tune_result {
     int32_t mode;  /* chosen VX_BATCH_FUSED / _STAGED / _PIPELINED / _SPLIT */

@@ -185,8 +185,8 @@ inline int words_per_row(int edge) { return (edge + 31) / 32; }
 // parts (512 chunks at 1 / 3 / 5 / 8 parts 127 / 95 / 94 / 101 us a pass), three up
 // to kEmitThree, but for chunks of many faces (emit_shares; 1,640 chunks of
 // instances at 1 / 3 parts 171 / 170 us density, 184 / 174 reference rule, 139 / 133
-// heightmap), one beyond (1,980 alike ones 353 / 374 / 353, 2,450 424 / 463 / 429 at
-// 1 / 2 / 3).  Slabs of 64^3 chunks hold more faces: kEmitGrid64 (1,292 slabs at 1 / 3 /
+// heightmap), one beyond (with vertices 1 / 3 parts tie at 1,740 to 1,815 chunks, then
+// three lose: 2,048 of the reference rule 232 / 244, density 225 / 232).  Slabs of 64^3 chunks hold more faces: kEmitGrid64 (1,292 slabs at 1 / 3 /
 // 5 / 8 parts 430 / 386 / 364 / 416); without vertices seven at most from 256 slabs
 // on (600 slabs at 3 / 7 / 11 parts 156 / 146 / 159 us density, 490 / 496 / 523 with
 // 22,000 faces each; with vertices the latter prefer 11, 582 / 552); one at
@@ -251,6 +251,10 @@ hipError_t launch_emit(const MeshWork *work, const int32_t *order, int32_t n, in
                        int32_t max_edge, uint64_t *bases, const uint32_t *counts,
                        const uint32_t *slabs, MeshOut out, const MeshTables *tables,
                        uint32_t *overflow, int32_t parts_hint, uint64_t *total, hipStream_t s);
+// 4 us of launch and scan against sums that grow with n and the scan's
+// largest-first order: 32^3 batches gain 3 to 5 us a pass up to 128 chunks, 1 to 4
+// at 200 to 450, 0.5 to 4 at 512 (density to heightmap); 64^3 ones gain up to 9,
+// but 256 of them lose 3 to 8.  At 600 to 1,000 some gain and some lose 3, 1,640 lose 6.
 constexpr int kSelfScan = 512;
 // Emit items of a batch: its chunks, or for batches that hold 64^3 chunks
 // kSlabs per 64^3 chunk and one per other chunk.

@@ -10,10 +10,13 @@
 //           src/shaders/vertex.vert:24)
 //   frustum AABB-vs-6-planes cull mask (src/frustum_culling.rs:16-40)
 //
-// Exactness: every floating-point expression is the oracle's expression in
-// the same order, compiled with -ffp-contract=off.  The only explicit FMAs
-// are fma(a, b, c) where a*b is exact (b in {+-1, +-0}), which round to
-// exactly the oracle's separate multiply and add.
+// Exactness: every output bit is the oracle's.  Where a float is an output, its
+// expression is the oracle's in the same order, compiled with
+// -ffp-contract=off; the only FMAs there are fma(a, b, c) where a*b is exact (b
+// in {+-1, +-0}), which round to exactly the oracle's separate multiply and
+// add.  The fast density fill, whose output is a sign, sums with ordinary FMAs
+// and decides by a bound on the difference; what the bound leaves open is
+// evaluated in the oracle's order ("density with a decided sign").
 #include "vx_internal.h"
 
 #include <mutex>
@@ -1520,7 +1523,7 @@ __device__ __forceinline__ void fast_item(const FillWork &w, const TerrainDev *t
     }
 }
 
-// `parts` workgroups per chunk (1, 2, 4 or 8), each on a band of rows.
+// `parts` workgroups per chunk (1, 2, 4, 8 or 16), each on a tile of it (fast_part).
 template <int MAXN>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
 fill_fast_kernel(const FillWork *__restrict__ work, const int32_t *__restrict__ order, int32_t n,
