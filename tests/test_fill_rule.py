@@ -207,7 +207,8 @@ def test_batches_that_gain(tmp_path):
         # 16^3 chunks, alone and beside larger ones
         (3, 1 / 64, 2.0, 0, 16, 16, 383, 0), (3, 1 / 64, 2.0, 0, 16, 16, 384, 1), (3, 1 / 64, 2.0, 0, 16, 32, 64, 1),
         (1, 1 / 64, 2.0, 0, 16, 16, 4000, 0), (3, 1 / 64, 2.0, 1, 16, 16, 4000, 0), (3, 0.013, 1.9, 1, 16, 16, 512, 1),
-        (4, 1 / 64, 2.0, 1, 16, 16, 1023, 0), (4, 1 / 64, 2.0, 1, 16, 16, 1024, 1),
+        (4, 1 / 64, 2.0, 0, 16, 16, 8, 1), (4, 1 / 64, 2.0, 0, 16, 16, 9, 0), (4, 1 / 64, 2.0, 1, 16, 16, 1, 0),
+        (3, 1 / 64, 2.0, 0, 16, 16, 1, 0), (4, 1 / 64, 2.0, 1, 16, 16, 1023, 0), (4, 1 / 64, 2.0, 1, 16, 16, 1024, 1),
     ]
     text = "\n".join(" ".join(repr(float(v)) if isinstance(v, float) else str(v) for v in c[:-1]) for c in cases)
     out = subprocess.run([str(tmp_path / "p")], input=text, capture_output=True, text=True, check=True)

@@ -110,8 +110,9 @@ inline bool on_lattice(float f) {
 //     terrains.  Where all cells are larger than 50,000 voxels it is zero nearly
 //     everywhere: 0.85.
 //   - 16^3 chunks pay for a chunk's tables over a quarter of the lines: 0.6 to
-//     1.05 below 384 chunks (one octave 0.8 to 1.0 at any number), then 0.95 to 1.3,
-//     on a lattice at threshold zero 0.5 to 1.0 below 1,024.
+//     1.05 below 384 chunks (one octave 0.8 to 1.0 at any number; four octaves of
+//     1 to 8 chunks 1.05 to 1.2), then 0.95 to 1.3, on a lattice at threshold zero
+//     0.5 to 1.0 below 1,024.
 inline bool fast_pays(int32_t octaves, float frequency, float lacunarity, bool zero, int32_t edge,
                       int32_t max_edge, int32_t n) {
     float f = frequency, fine = 0.0f;
@@ -125,6 +126,7 @@ inline bool fast_pays(int32_t octaves, float frequency, float lacunarity, bool z
     if (octaves > 4) return true;
     if (max_edge <= 16) {
         if (octaves == 1) return false;
+        if (octaves == 4 && !zero && n <= 8) return true;
         return lattice ? octaves == 4 && n >= 1024 : n >= 384;
     }
     if (edge == 64) {
