@@ -137,7 +137,7 @@ def test_batch_rule(ctx, oracle_mod, name, n):
     edges = [16 if name == "16^3" else (16, 32)[i % 2] for i in range(n)]
     coords = [(i % 23 - 11, 0, i // 23) for i in range(n)]
     b = V.Batch(ctx, coords, edges, [ctx.terrain(ts[i % 4]) for i in range(n)])
-    for splits in ((0, 0), (2, 1)):
+    for splits in ((0, 0), (2, 1), (2, 1), (2, 1)):  # launched, captured, replayed twice
         b.set_splits(*splits)
         b.run()
         b.wait()
